@@ -56,10 +56,12 @@ extern "C" {
                                  float arrays, rounded once per step on store
                                  (2-D periodic RK4 only; not in batches)     */
 /* RK4 engines (nls_problem.engine, nls_batch_create) */
-#define NLS_ENGINE_AUTO  -1   /* RESIDENT if the instance (every member of a
-                                 batch) fits, else FUSED for 2-D and STAGE
-                                 for 1-D; a batch of which only some members
-                                 fit: HYBRID                                 */
+#define NLS_ENGINE_AUTO  -1   /* a plain 1-D solve: pieces of the line held in
+                                 registers, many steps per launch; 2-D:
+                                 RESIDENT if the instance fits, else FUSED.
+                                 Batches: RESIDENT if every member fits, else
+                                 FUSED for 2-D and STAGE for 1-D, HYBRID if
+                                 only some members fit                       */
 #define NLS_ENGINE_STAGE  0   /* one launch per RK4 stage                    */
 #define NLS_ENGINE_FUSED  1   /* one launch per RK4 step, halo recomputed on
                                  chip (2-D only)                             */

@@ -839,30 +839,24 @@ template <typename T, int ORDER, int BC, int DIM>
 __device__ __forceinline__ cplx_t<T> resident_lap(const cplx_t<T> *Y, int idx, int n, const T *w,
                                                   const T *wrow) {
     constexpr int R = (ORDER - 1) / 2;
-    const cplx_t<T> c = Y[idx];
-    if (DIM == 1) {
-        T lr = 0, li = 0;
-        if (BC == BC_PERIODIC) {
-            lr = lap_centre<T>(w[0], c.x); li = lap_centre<T>(w[0], c.y);
+    if constexpr (DIM == 1) {
+        // the points around it; outside the reference's grid zero
+        T ex[2 * R + 1], ey[2 * R + 1];
 #pragma unroll
-            for (int d = 1; d <= R; ++d) {
-                int im = idx - d, ip = idx + d;
-                if (im < 0) im += n;
-                if (ip >= n) ip -= n;
-                lr += lap_pair<T>(w[d], c.x, Y[im].x, Y[ip].x, d);
-                li += lap_pair<T>(w[d], c.y, Y[im].y, Y[ip].y, d);
+        for (int d = -R; d <= R; ++d) {
+            int j = idx + d;
+            if (BC == BC_PERIODIC) {
+                if (j < 0) j += n;
+                if (j >= n) j -= n;
             }
-        } else {
-#pragma unroll
-            for (int d = -R; d <= R; ++d) {
-                const int j = idx + d;
-                if (j < 0 || j >= n) continue;
-                lr += wrow[d + R] * Y[j].x;
-                li += wrow[d + R] * Y[j].y;
-            }
+            const cplx_t<T> v = j >= 0 && j < n ? Y[j] : mk<T>(0, 0);
+            ex[R + d] = v.x;
+            ey[R + d] = v.y;
         }
-        return mk<T>(lr, li);
-    }
+        if (BC == BC_PERIODIC) return mk<T>(line_lap<T, R>(w, ex + R), line_lap<T, R>(w, ey + R));
+        return mk<T>(line_lap_row<T, R>(wrow, ex + R), line_lap_row<T, R>(wrow, ey + R));
+    } else {
+    const cplx_t<T> c = Y[idx];
     const int row = idx / n, col = idx - row * n;
     T lr = lap_centre<T>((T)2 * w[0], c.x), li = lap_centre<T>((T)2 * w[0], c.y);
 #pragma unroll
@@ -885,6 +879,14 @@ __device__ __forceinline__ cplx_t<T> resident_lap(const cplx_t<T> *Y, int idx, i
         li += lap_quad<T>(w[d], c.y, a0.y, a1.y, b0.y, b1.y, d);
     }
     return mk<T>(lr, li);
+    }
+}
+
+template <typename T, bool DYN, int DIM>
+__device__ __forceinline__ void resident_rhs(const Coeffs<T> &c, T P, cplx_t<T> y, T yn, cplx_t<T> lap, cplx_t<T> &k,
+                                             T &kn) {
+    if constexpr (DIM == 1) line_rhs<T, DYN>(c, pump_term<T, DYN>(c, P), y, yn, lap.x, lap.y, k, kn);
+    else rhs_point<T, DYN>(c, P, y, yn, lap, k, kn);
 }
 
 template <typename T, int ORDER, int BC, bool DYN, int DIM>
@@ -936,14 +938,22 @@ __global__ void __launch_bounds__(ResShape<T>::THREADS) k_resident(const Residen
     }
     __syncthreads();
     int b = 0;
-    for (int it = 0; it < steps; ++it) {
-#pragma unroll
-        for (int s = 1; s <= 4; ++s) {
+    const LineStep<T> h = line_step(dt);          // 1-D lines
+    auto run_stage = [&](auto s_) {
+            constexpr int s = decltype(s_)::value;
             const T wacc = (s == 1 || s == 4) ? (T)1 : (T)2;
             const T anext = (s == 3) ? (T)1 : (T)0.5;
             // acc += wacc k; the next stage input u + k dt anext, or at stage
             // 4 the new state u + acc dt / 6
             auto advance_point = [&](int q, int idx, const C &kk, T kn, const C &u, C *Yout) {
+                if constexpr (DIM == 1) {
+                    const C v = mk<T>(line_combine<T, s>(acc[q].x, kk.x, u.x, h),
+                                      line_combine<T, s>(acc[q].y, kk.y, u.y, h));
+                    Yout[idx] = v;
+                    if (DYN) yn[q] = line_combine<T, s>(accn[q], kn, un[q], h);
+                    if (s == 4 && DYN) un[q] = yn[q];
+                    return s == 4 ? v : u;
+                }
                 if (s == 1) { acc[q] = kk; accn[q] = kn; }
                 else {
                     acc[q] = mk<T>(acc[q].x + wacc * kk.x, acc[q].y + wacc * kk.y);
@@ -969,7 +979,7 @@ __global__ void __launch_bounds__(ResShape<T>::THREADS) k_resident(const Residen
                     C kk;
                     T kn = 0;
                     const C lap = resident_lap<T, ORDER, BC, DIM>(Yin, idx, n, w, wtab ? wtab + (size_t)idx * ORDER : nullptr);
-                    rhs_point<T, DYN>(m.c, pp[q], Yin[idx], yn[q], lap, kk, kn);
+                    resident_rhs<T, DYN, DIM>(m.c, pp[q], Yin[idx], yn[q], lap, kk, kn);
                     uu[PINGPONG ? q : 0] = advance_point(q, idx, kk, kn, uu[PINGPONG ? q : 0], Yout);
                 }
                 __syncthreads();
@@ -983,7 +993,7 @@ __global__ void __launch_bounds__(ResShape<T>::THREADS) k_resident(const Residen
                     kk[q] = mk<T>(0, 0); kn[q] = 0;
                     if (idx < N) {
                         const C lap = resident_lap<T, ORDER, BC, DIM>(Y[0], idx, n, w, wtab ? wtab + (size_t)idx * ORDER : nullptr);
-                        rhs_point<T, DYN>(m.c, pp[q], Y[0][idx], yn[q], lap, kk[q], kn[q]);
+                        resident_rhs<T, DYN, DIM>(m.c, pp[q], Y[0][idx], yn[q], lap, kk[q], kn[q]);
                     }
                 }
                 __syncthreads();                     // every read of Y[0] for this stage is done
@@ -994,7 +1004,12 @@ __global__ void __launch_bounds__(ResShape<T>::THREADS) k_resident(const Residen
                 }
                 __syncthreads();
             }
-        }
+    };
+    for (int it = 0; it < steps; ++it) {
+        run_stage(std::integral_constant<int, 1>{});
+        run_stage(std::integral_constant<int, 2>{});
+        run_stage(std::integral_constant<int, 3>{});
+        run_stage(std::integral_constant<int, 4>{});
     }
 #pragma unroll
     for (int q = 0; q < RES_PPT; ++q) {
@@ -1084,7 +1099,7 @@ static void launch_fused(int order, int bc, bool dyn, int form, const FusedArgs<
 }
 
 // Compute units of the current device, read once per device.
-static int device_cus() {
+int device_cus() {
     static std::atomic<int> cache[64];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;

@@ -48,17 +48,19 @@ int check_problem(const nls_problem *p) {
     return NLS_OK;
 }
 
-// RK4 engine of a plain solve.  AUTO: the resident kernel when the instance
-// fits on chip (one launch runs a block of steps) -- every 1-D line up to
-// 4096 points, 2-D grids up to 64 x 64 in single precision (in double
-// precision one workgroup computing the whole grid is slower than the fused
-// kernel's tiles) -- else the fused one-launch-per-step kernel for 2-D grids
-// and the per-stage kernels for 1-D lines.
+// RK4 engine of a plain solve.  AUTO: the line kernel for 1-D (us per step
+// against the engines it replaced: n = 256 FP32 0.56 / 0.88 resident, n = 1000
+// radial FP32 0.59 / 3.6, n = 4096 FP64 0.67 / 6.3; longer lines took 8 to 15
+// on the per-stage kernels, 20,000 points take 0.67); in 2-D the resident
+// kernel when the grid fits one workgroup -- up to 64 x 64 in single precision
+// (in double precision one workgroup computing the whole grid is slower than
+// the fused kernel's tiles) -- else the fused one-launch-per-step kernel.
 int plain_engine(const nls_problem *p) {
     if (p->flags & NLS_FLAG_F64_ARITH) return NLS_ENGINE_FUSED;
     if (p->engine != NLS_ENGINE_AUTO) return p->engine;
-    if (resident_fits(p) && (p->dim == 1 || p->dtype == NLS_F32)) return NLS_ENGINE_RESIDENT;
-    return p->dim == 2 && fused_holds((long long)p->n * p->n, p->dtype) ? NLS_ENGINE_FUSED : NLS_ENGINE_STAGE;
+    if (p->dim == 1) return ENGINE_LINE;
+    if (resident_fits(p) && p->dtype == NLS_F32) return NLS_ENGINE_RESIDENT;
+    return fused_holds((long long)p->n * p->n, p->dtype) ? NLS_ENGINE_FUSED : NLS_ENGINE_STAGE;
 }
 
 static size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -202,6 +204,7 @@ size_t nls_workspace_bytes(const nls_problem *p) {
     switch (plain_engine(p)) {
     case NLS_ENGINE_FUSED: return fused_grid_workspace_bytes(p);
     case NLS_ENGINE_RESIDENT: return resident_workspace_bytes(p);
+    case ENGINE_LINE: return line_workspace_bytes(p);
     default: return rk4_workspace(p, nullptr);
     }
 }
@@ -213,6 +216,7 @@ static int advance_direct(const nls_problem *p, int iters, const void *pumping, 
     const int engine = plain_engine(p);
     if (engine == NLS_ENGINE_FUSED) return fused_grid_advance(p, iters, pumping, psi, nres, ws, s);
     if (engine == NLS_ENGINE_RESIDENT) return resident_advance(p, iters, pumping, psi, nres, ws, s);
+    if (engine == ENGINE_LINE) return line_advance(p, iters, pumping, psi, nres, ws, s);
     if (p->dtype == NLS_F64)
         return rk4_advance<double>(p, iters, (const double *)pumping, (double2 *)psi, (double *)nres, (char *)ws, s);
     return rk4_advance<float>(p, iters, (const float *)pumping, (float2 *)psi, (float *)nres, (char *)ws, s);

@@ -34,6 +34,15 @@ size_t resident_workspace_bytes(const nls_problem *p);
 int resident_advance(const nls_problem *p, int iters, const void *pumping, void *psi, void *nres, void *ws,
                      hipStream_t s);
 
+// plain RK4 solve of one line of any length: the engine AUTO takes for 1-D
+// problems (nls_line.hip; plain_engine returns ENGINE_LINE, which callers
+// cannot ask for by number)
+constexpr int ENGINE_LINE = 100;
+size_t line_workspace_bytes(const nls_problem *p);
+int line_advance(const nls_problem *p, int iters, const void *pumping, void *psi, void *nres, void *ws,
+                 hipStream_t s);
+int device_cus();                                  // compute units of the current device, 0 if unknown
+
 // split-step Fourier scheme (nls_ssf.hip)
 size_t ssf_workspace_bytes(const nls_problem *p);
 int ssf_check(const nls_problem *p);               // size limits of the scheme

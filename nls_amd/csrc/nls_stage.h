@@ -92,42 +92,6 @@ __device__ __forceinline__ void stage_epilogue(const StageArgs<T> &a, size_t gi,
     }
 }
 
-// Stage input at a point: y = u + (k_prev*dt)*a.
-template <typename T>
-__device__ __forceinline__ cplx_t<T> stage_input(const StageArgs<T> &a, size_t gi) {
-    cplx_t<T> u = a.u[gi];
-    if (a.stage != 1) {
-        const cplx_t<T> k = a.kin[gi];
-        u.x = u.x + (k.x * a.dt) * a.scale;
-        u.y = u.y + (k.y * a.dt) * a.scale;
-    }
-    return u;
-}
-
-// Pointwise part of a stage at one point, given y and its Laplacian.
-template <typename T, bool DYN>
-__device__ __forceinline__ void stage_point(const StageArgs<T> &a, size_t gi, cplx_t<T> y, T lr, T li) {
-    const cplx_t<T> u = a.u[gi];
-    cplx_t<T> kin = mk<T>(0, 0);
-    T kin_n = 0, un = 0, yn = 0;
-    if (a.stage != 1) kin = a.kin[gi];
-    if (DYN) {
-        un = a.un[gi];
-        yn = un;
-        if (a.stage != 1) { kin_n = a.kin_n[gi]; yn = un + (kin_n * a.dt) * a.scale; }
-    }
-    cplx_t<T> acc = mk<T>(0, 0);
-    T accn = 0;
-    if (a.stage >= 3) {
-        acc = a.acc[gi];
-        if (DYN) accn = a.acc_n[gi];
-    }
-    cplx_t<T> k;
-    T kn = 0;
-    rhs_point<T, DYN>(a.c, a.P[gi], y, yn, mk<T>(lr, li), k, kn);
-    stage_epilogue<T, DYN>(a, gi, u, kin, kin_n, acc, accn, k, kn, un);
-}
-
 // One 64 x TY tile of a 2-D stage with origin (x0, y0); called by all 256
 // threads of the workgroup.  Thread (tx, ty) = (tid % 64, tid / 64) owns the
 // TY/4 points (x0 + tx, y0 + ty + 4j).  Every global load of a thread's own
@@ -196,7 +160,7 @@ __device__ __forceinline__ void stage_tile_2d(const StageArgs<T> &a, int x0, int
         else ok = ok && hx >= 0 && hx < n && hy >= 0 && hy < n;
         // unconditional loads (index 0 when the point is not used) keep every
         // halo load of the thread in one group; the stage input is formed at
-        // the store, as stage_input does
+        // the store
         const size_t hi = ok ? (size_t)hy * n + hx : (size_t)0;
         const C v = a.u[hi];
         const C k = first ? mk<T>(0, 0) : a.kin[hi];
@@ -244,20 +208,27 @@ __device__ __forceinline__ void stage_tile_2d(const StageArgs<T> &a, int x0, int
     }
 }
 
-// One 256-point tile of a 1-D stage starting at x0.
+// One 256-point tile of a 1-D stage starting at x0, in the arithmetic that
+// the 1-D engines share (line_lap .. line_combine).
 template <typename T, int ORDER, int BC, bool DYN>
 __device__ __forceinline__ void stage_tile_1d(const StageArgs<T> &a, int x0, cplx_t<T> *tile) {
     constexpr int R = (ORDER - 1) / 2;
     constexpr int LW = TILE1 + 2 * R;
-    const int n = a.n;
+    const int n = a.n, st = a.stage;
+    const LineStep<T> h = line_step(a.dt);
+    // stage input u + k_prev (dt/2, dt/2, dt)
+    auto input = [&](T u, T k) {
+        T unused = 0;
+        return st == 1 ? u : st == 4 ? line_combine<T, 3>(unused, k, u, h)
+                                     : line_combine<T, 1>(unused, k, u, h);
+    };
     for (int idx = threadIdx.x; idx < LW; idx += TILE1) {
         int gx = x0 + idx - R;
+        if (BC == BC_PERIODIC) gx = wrap_index(gx, n);
         cplx_t<T> y = mk<T>(0, 0);
-        if (BC == BC_PERIODIC) {
-            gx = wrap_index(gx, n);
-            y = stage_input(a, (size_t)gx);
-        } else if (gx >= 0 && gx < n) {
-            y = stage_input(a, (size_t)gx);
+        if (gx >= 0 && gx < n) {
+            const cplx_t<T> u = a.u[gx], k = st == 1 ? mk<T>(0, 0) : a.kin[gx];
+            y = mk<T>(input(u.x, k.x), input(u.y, k.y));
         }
         tile[idx] = y;
     }
@@ -265,29 +236,60 @@ __device__ __forceinline__ void stage_tile_1d(const StageArgs<T> &a, int x0, cpl
     const int gx = x0 + threadIdx.x;
     if (gx >= n) return;
     const int l = threadIdx.x + R;
-    const cplx_t<T> c = tile[l];
-    T lr = 0, li = 0;
+    T ex[2 * R + 1], ey[2 * R + 1];
+#pragma unroll
+    for (int d = 0; d <= 2 * R; ++d) {
+        const cplx_t<T> v = tile[l - R + d];
+        ex[d] = v.x;
+        ey[d] = v.y;
+    }
+    T lr, li;
     if (BC == BC_PERIODIC) {
         const T w[4] = {a.w0, a.w1, a.w2, a.w3};
-        lr = lap_centre<T>(w[0], c.x);
-        li = lap_centre<T>(w[0], c.y);
-#pragma unroll
-        for (int d = 1; d <= R; ++d) {
-            const cplx_t<T> a0 = tile[l - d], a1 = tile[l + d];
-            lr += lap_pair<T>(w[d], c.x, a0.x, a1.x, d);
-            li += lap_pair<T>(w[d], c.y, a0.y, a1.y, d);
-        }
+        lr = line_lap<T, R>(w, ex + R);
+        li = line_lap<T, R>(w, ey + R);
     } else {
-        const T *wr = a.wtab + (size_t)gx * ORDER;
+        T w[ORDER];
 #pragma unroll
-        for (int d = -R; d <= R; ++d) {
-            const T wd = wr[d + R];
-            const cplx_t<T> v = tile[l + d];
-            lr += wd * v.x;
-            li += wd * v.y;
-        }
+        for (int k = 0; k < ORDER; ++k) w[k] = a.wtab[(size_t)gx * ORDER + k];
+        lr = line_lap_row<T, R>(w, ex + R);
+        li = line_lap_row<T, R>(w, ey + R);
     }
-    stage_point<T, DYN>(a, (size_t)gx, c, lr, li);
+    const size_t gi = (size_t)gx;
+    const cplx_t<T> u = a.u[gi];
+    cplx_t<T> acc = st == 1 ? mk<T>(0, 0) : st == 2 ? a.kin[gi] : a.acc[gi];
+    T un = 0, kin_n = 0, accn = 0;
+    if (DYN) {
+        un = a.un[gi];
+        kin_n = st == 1 ? (T)0 : a.kin_n[gi];
+        accn = st == 1 ? (T)0 : st == 2 ? kin_n : a.acc_n[gi];
+    }
+    cplx_t<T> k;
+    T kn = 0;
+    line_rhs<T, DYN>(a.c, pump_term<T, DYN>(a.c, a.P[gi]), mk<T>(ex[R], ey[R]), input(un, kin_n), lr, li, k, kn);
+    // the accumulator after stages 2 and 3, the new state after stage 4
+    cplx_t<T> av;
+    T avn = 0;
+    if (st == 4) {
+        av.x = line_combine<T, 4>(acc.x, k.x, u.x, h);
+        av.y = line_combine<T, 4>(acc.y, k.y, u.y, h);
+        avn = line_combine<T, 4>(accn, kn, un, h);
+    } else {
+        (void)line_combine<T, 2>(acc.x, k.x, u.x, h);
+        (void)line_combine<T, 2>(acc.y, k.y, u.y, h);
+        (void)line_combine<T, 2>(accn, kn, un, h);
+        av = acc;
+        avn = accn;
+    }
+    // two store sites with fixed base pointers (stage_epilogue)
+    if (st != 4) {
+        a.kout[gi] = k;
+        if (DYN) a.kout_n[gi] = kn;
+    }
+    if (st != 1) {
+        a.acc[gi] = av;
+        if (DYN) a.acc_n[gi] = avn;
+    }
 }
 
 }  // namespace nls
