@@ -45,6 +45,7 @@ template <typename T> struct MemberDev {
     T dt;
     T w0, w1, w2, w3;       // Cartesian second-derivative weights
     Coeffs<T> c;
+    GridCoeffs<T> g;        // of the fused 2-D step
 };
 
 struct TileDesc {
@@ -285,6 +286,7 @@ k_fused_step_2d(const FusedArgs<T> f) {
     constexpr int J = (NP + NT - 1) / NT;
     constexpr int JOUT = TX * TY / NT;    // list entries t + NT j, j < JOUT, are the output tile
     static_assert(TX * TY % NT == 0 && W < 256 && HH < 256, "fused tile shape");
+    static_assert(DB || BC != BC_REF, "points outside the grid are written once per buffer");
     // psi stage input, point (x, y) of the region at ys_mem[b][PAD + y WS + x]:
     // the front pad makes every stencil read a non-negative constant offset
     // from the point's own index, so each read is one LDS instruction with an
@@ -335,29 +337,26 @@ k_fused_step_2d(const FusedArgs<T> f) {
         return;
     }
 
-    const T dt = m.dt;
-    const T dt2 = dt * (T)0.5;
-    const T dt6 = dt / (T)6;
+    const T dt = m.dt, dt2 = dt * (T)0.5, dt6 = dt / (T)6;                   // of the reservoir
+    const T dtw = m.g.dtw, dtw2 = dtw * (T)0.5, dtw6 = dtw / (T)6;           // of psi
     Coeffs<T> c = m.c;
+    GridCoeffs<T> g = m.g;
     if constexpr (sizeof(T) == 4) {
         // coefficients that meet another coefficient in one fused
-        // multiply-add of the right-hand side (c3 r - c4, d13 + d14 s,
-        // c13 + c14 s): a VALU instruction reads one scalar register, so
-        // held in scalar registers each would be copied to a vector register
-        // per point and stage; kept in vector registers for the whole kernel
-        asm volatile("" : "+v"(c.c4), "+v"(c.d13), "+v"(c.c13));
+        // multiply-add of the right-hand side (c3 r - c4, c6 r - wc,
+        // d13 + d14 s, c13 + c14 s): a VALU instruction reads one scalar
+        // register, so held in scalar registers each would be copied to a
+        // vector register per point and stage; kept in vector registers for
+        // the whole kernel
+        asm volatile("" : "+v"(g.c4), "+v"(g.wc), "+v"(c.d13), "+v"(c.c13));
     }
-    const T w0 = (T)2 * m.w0;          // centre weight of the 2-D Laplacian
-    const T w[4] = {m.w0, m.w1, m.w2, m.w3};
-    T wc = w0;                         // meets c6 in one fused multiply-add: held in a vector register
-    if constexpr (sizeof(T) == 4) asm volatile("" : "+v"(wc));
     const unsigned *map = ring_map<W, HH, R, WS>.v;
 
     C uu[J], acc[J], ynext[DB ? 1 : J];
     T cp[J], nn[J], yn[J], accn[J];
     int li[J];                         // LDS index of the point
-    unsigned long long inside = 0;     // bit j: point j lies on the grid
-    static_assert(J <= 64, "inside mask");
+    unsigned inside = 0;               // BC_REF, bit j: point j lies on the grid
+    static_assert(J <= 32, "inside mask");
 
     const bool near = n >= TX + H;     // region offsets stay within one period of the grid
 
@@ -417,7 +416,7 @@ k_fused_step_2d(const FusedArgs<T> f) {
             }
             if (ok) {
                 const unsigned gi = grid_index(gy, n, gx);
-                inside |= 1ull << j;
+                if (BC == BC_REF) inside |= 1u << j;
                 if constexpr (sizeof(T) == 4) {
                     uu[j] = buffer_load_c<T>(ru, gi * (unsigned)sizeof(C));
                     cp[j] = buffer_load_r<T>(rp, gi * (unsigned)sizeof(T));   // the pump term is formed at the store
@@ -431,7 +430,10 @@ k_fused_step_2d(const FusedArgs<T> f) {
                     if (DYN) nn[j] = (T)un[gi];
                 }
             }
-            if (!GROUPED) ya[li[j]] = uu[j];
+            if (!GROUPED) {
+                ya[li[j]] = uu[j];
+                if (BC == BC_REF && !ok) yb[li[j]] = uu[j];
+            }
         }
         if (!GROUPED) {
             cp[j] = pump_term<T, DYN>(c, cp[j]);
@@ -441,7 +443,10 @@ k_fused_step_2d(const FusedArgs<T> f) {
     if (GROUPED) {
 #pragma unroll
         for (int j = 0; j < J; ++j) {
-            if (NP % NT == 0 || j < J - 1 || tid + NT * j < NP) ya[li[j]] = uu[j];
+            if (NP % NT == 0 || j < J - 1 || tid + NT * j < NP) {
+                ya[li[j]] = uu[j];
+                if (BC == BC_REF && !((inside >> j) & 1u)) yb[li[j]] = uu[j];
+            }
             cp[j] = pump_term<T, DYN>(c, cp[j]);
             yn[j] = nn[j];
         }
@@ -463,34 +468,29 @@ k_fused_step_2d(const FusedArgs<T> f) {
         auto rd = [&](int i) { const V2 v = ys[i]; return mk<T>(v.x, v.y); };
         const int idx = R * WS;
         const C y = rd(idx);
-        // the stencil sum as written (neighbour sums weighted; the
-        // difference form of lap_quad costs 8 more operations per point and
-        // stage, and this kernel is bound by its arithmetic).  In single
-        // precision the centre term joins the point's own factor in the
-        // right-hand side (rhs_point_centre: two products fewer); double
-        // precision adds it here.
-        T lr, lm;
-        if constexpr (sizeof(T) == 8) { lr = w0 * y.x; lm = w0 * y.y; }
+        // the neighbour sum (the difference form of lap_quad
+        // costs 8 more operations per point and stage, and this kernel is
+        // bound by its arithmetic)
+        T sr, sm;
 #pragma unroll
         for (int d = 1; d <= R; ++d) {
             const C a0 = rd(idx - d), a1 = rd(idx + d);
             const C b0 = rd(idx - d * WS), b1 = rd(idx + d * WS);
-            const T sr = (a0.x + a1.x) + (b0.x + b1.x), sm = (a0.y + a1.y) + (b0.y + b1.y);
-            if (sizeof(T) == 4 && d == 1) {
-                lr = w[1] * sr;
-                lm = w[1] * sm;
+            if (d == 1) {
+                sr = grid_ring1(g, a0.x, a1.x, b0.x, b1.x);
+                sm = grid_ring1(g, a0.y, a1.y, b0.y, b1.y);
             } else {
-                lr += w[d] * sr;
-                lm += w[d] * sm;
+                sr = grid_ring(sr, d == 2 ? g.r2 : g.r3, a0.x, a1.x, b0.x, b1.x);
+                sm = grid_ring(sm, d == 2 ? g.r2 : g.r3, a0.y, a1.y, b0.y, b1.y);
             }
         }
-        kn = 0;
-        if constexpr (sizeof(T) == 4) rhs_point_centre<T, DYN>(c, cp[j], wc, y, yn[j], mk<T>(lr, lm), k, kn);
-        else rhs_point_cp<T, DYN>(c, cp[j], y, yn[j], mk<T>(lr, lm), k, kn);
+        grid_rhs<T, DYN>(g, c, cp[j], y, yn[j], mk<T>(sr, sm), k, kn);
     };
 
     // stages 1..3 on the shrinking rectangles.  Stage s computes the points
     // with at least sR halo rings around them: the first cnt list entries.
+    // Points outside the reference's grid hold zero in both buffers from the
+    // start and are skipped.
     // The test against cnt is made opaque to the compiler so that each
     // point's body stays a block of its own; resolved at compile time, the
     // stage's bodies would merge and all their LDS reads be hoisted together.
@@ -499,29 +499,25 @@ k_fused_step_2d(const FusedArgs<T> f) {
         const int cnt = (W - 2 * s * R) * (HH - 2 * s * R);
         int lim = cnt;
         asm volatile("" : "+s"(lim));
-        const T dta = (s == 3) ? dt : dt2;           // y_{s+1} = u + k_s * dt * (1/2, 1/2, 1)
+        // y_{s+1} = u + k_s dt (1/2, 1/2, 1)
+        const T dta = (s == 3) ? dt : dt2, dtwa = (s == 3) ? dtw : dtw2;
         const C *yin = (s == 2) ? yb : ya;
         C *yout = (s == 2) ? ya : yb;
 #pragma unroll
         for (int j = 0; j < J; ++j) {
             if (NT * j >= cnt) break;
             if (tid + NT * j >= lim) continue;
+            if (BC == BC_REF && !((inside >> j) & 1u)) continue;
             C k;
             T kn;
             stage_rhs(yin, j, k, kn);
-            if (s == 1) {
-                acc[j] = k;
-                if (DYN) accn[j] = kn;
-            } else {
-                acc[j].x = acc[j].x + (T)2 * k.x;
-                acc[j].y = acc[j].y + (T)2 * k.y;
-                if (DYN) accn[j] = accn[j] + (T)2 * kn;
-            }
-            C yv = mk<T>(uu[j].x + k.x * dta, uu[j].y + k.y * dta);
-            if (BC != BC_PERIODIC && !((inside >> j) & 1ull)) yv = mk<T>(0, 0);
+            grid_acc(acc[j].x, k.x, s == 1);
+            grid_acc(acc[j].y, k.y, s == 1);
+            if (DYN) grid_acc(accn[j], kn, s == 1);
+            const C yv = mk<T>(grid_input(uu[j].x, k.x, dtwa), grid_input(uu[j].y, k.y, dtwa));
             if (DB) yout[li[j]] = yv;
             else ynext[j] = yv;
-            if (DYN) yn[j] = nn[j] + kn * dta;
+            if (DYN) yn[j] = grid_input(nn[j], kn, dta);
         }
         __syncthreads();
         if (!DB) {
@@ -547,9 +543,8 @@ k_fused_step_2d(const FusedArgs<T> f) {
         T kn;
         stage_rhs(yb, j, k, kn);
         const size_t gi = (size_t)gy * n + gx;
-        const C v = mk<T>(uu[j].x + (acc[j].x + k.x) * dt6, uu[j].y + (acc[j].y + k.y) * dt6);
-        uo[gi] = SC{(SR)v.x, (SR)v.y};
-        if (DYN) uno[gi] = (SR)(nn[j] + (accn[j] + kn) * dt6);
+        uo[gi] = SC{(SR)grid_new(uu[j].x, acc[j].x, k.x, dtw6), (SR)grid_new(uu[j].y, acc[j].y, k.y, dtw6)};
+        if (DYN) uno[gi] = (SR)grid_new(nn[j], accn[j], kn, dt6);
     }
 }
 
@@ -648,21 +643,18 @@ k_fused_pairs_2d(const FusedArgs<float> f) {
         return;
     }
 
-    const T dt = m.dt;
-    const T dt2 = dt * (T)0.5;
-    const T dt6 = dt / (T)6;
+    const T dt = m.dt, dt2 = dt * (T)0.5, dt6 = dt / (T)6;
+    const T dtw = m.g.dtw, dtw2 = dtw * (T)0.5, dtw6 = dtw / (T)6;
     Coeffs<T> c = m.c;
-    asm volatile("" : "+v"(c.c4), "+v"(c.d13), "+v"(c.c13));
-    T wc = (T)2 * m.w0;                // centre weight of the 2-D Laplacian, joins the point's factor
-    asm volatile("" : "+v"(wc));
-    const T w1 = m.w1, w2 = m.w2;
+    GridCoeffs<T> g = m.g;
+    asm volatile("" : "+v"(g.c4), "+v"(g.wc), "+v"(c.d13), "+v"(c.c13));
     const unsigned *map = pair_map<W, HH, WS>.v;
 
     C uu[J][2], acc[J][2];
     T cp[J][2], nn[J][2], yn[J][2], accn[J][2];
     int li[J];                         // LDS index of the pair's upper point
-    unsigned long long inside = 0;     // bit 2 j + q: point q of pair j lies on the grid
-    static_assert(2 * J <= 64, "inside mask");
+    unsigned inside = 0;               // BC_REF, bit 2 j + q: point q of pair j lies on the grid
+    static_assert(2 * J <= 32, "inside mask");
     const bool near = n >= TX + H;
 
     unsigned ent[J];
@@ -702,7 +694,7 @@ k_fused_pairs_2d(const FusedArgs<float> f) {
                 else ok = gx >= 0 && gx < n && gy >= 0 && gy < n;
                 if (ok) {
                     const unsigned gi = grid_index(gy, n, gx);
-                    inside |= 1ull << (2 * j + q);
+                    if (BC == BC_REF) inside |= 1u << (2 * j + q);
                     uu[j][q] = buffer_load_c<T>(ru, gi * (unsigned)sizeof(C));
                     cp[j][q] = buffer_load_r<T>(rp, gi * (unsigned)sizeof(T));
                     if (DYN) nn[j][q] = buffer_load_r<T>(rn, gi * (unsigned)sizeof(T));
@@ -715,6 +707,9 @@ k_fused_pairs_2d(const FusedArgs<float> f) {
         if (NPP % NT == 0 || j < J - 1 || tid + NT * j < NPP) {
             ya[li[j]] = uu[j][0];
             ya[li[j] + WS] = uu[j][1];
+            // outside the reference's grid both buffers hold zero throughout
+            if (BC == BC_REF && !((inside >> (2 * j)) & 1u)) yb[li[j]] = mk<T>(0, 0);
+            if (BC == BC_REF && !((inside >> (2 * j + 1)) & 1u)) yb[li[j] + WS] = mk<T>(0, 0);
         }
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
@@ -736,23 +731,19 @@ k_fused_pairs_2d(const FusedArgs<float> f) {
         auto rd = [&](int i) { const V2 v = ys[i]; return mk<T>(v.x, v.y); };
         const C c0 = rd(0), c1 = rd(WS), yA = rd(2 * WS), yB = rd(3 * WS), c4 = rd(4 * WS), c5 = rd(5 * WS);
         const C a1m = rd(2 * WS - 1), a1p = rd(2 * WS + 1), a2m = rd(2 * WS - 2), a2p = rd(2 * WS + 2);
-        // the stencil sum as in k_fused_step_2d: (horizontal pair + vertical pair) per distance
-        T lr = w1 * ((a1m.x + a1p.x) + (c1.x + yB.x));
-        T lm = w1 * ((a1m.y + a1p.y) + (c1.y + yB.y));
-        lr += w2 * ((a2m.x + a2p.x) + (c0.x + c4.x));
-        lm += w2 * ((a2m.y + a2p.y) + (c0.y + c4.y));
-        kn[0] = 0;
-        rhs_point_centre<T, DYN>(c, cp[j][0], wc, yA, yn[j][0], mk<T>(lr, lm), k[0], kn[0]);
+        T sr = grid_ring1(g, a1m.x, a1p.x, c1.x, yB.x), sm = grid_ring1(g, a1m.y, a1p.y, c1.y, yB.y);
+        sr = grid_ring(sr, g.r2, a2m.x, a2p.x, c0.x, c4.x);
+        sm = grid_ring(sm, g.r2, a2m.y, a2p.y, c0.y, c4.y);
+        grid_rhs<T, DYN>(g, c, cp[j][0], yA, yn[j][0], mk<T>(sr, sm), k[0], kn[0]);
         // the lower point's row after the upper point is done, so that its
         // reads do not all live in registers at once
         __builtin_amdgcn_sched_barrier(0);
         const C b1m = rd(3 * WS - 1), b1p = rd(3 * WS + 1), b2m = rd(3 * WS - 2), b2p = rd(3 * WS + 2);
-        lr = w1 * ((b1m.x + b1p.x) + (yA.x + c4.x));
-        lm = w1 * ((b1m.y + b1p.y) + (yA.y + c4.y));
-        lr += w2 * ((b2m.x + b2p.x) + (c1.x + c5.x));
-        lm += w2 * ((b2m.y + b2p.y) + (c1.y + c5.y));
-        kn[1] = 0;
-        rhs_point_centre<T, DYN>(c, cp[j][1], wc, yB, yn[j][1], mk<T>(lr, lm), k[1], kn[1]);
+        sr = grid_ring1(g, b1m.x, b1p.x, yA.x, c4.x);
+        sm = grid_ring1(g, b1m.y, b1p.y, yA.y, c4.y);
+        sr = grid_ring(sr, g.r2, b2m.x, b2p.x, c1.x, c5.x);
+        sm = grid_ring(sm, g.r2, b2m.y, b2p.y, c1.y, c5.y);
+        grid_rhs<T, DYN>(g, c, cp[j][1], yB, yn[j][1], mk<T>(sr, sm), k[1], kn[1]);
     };
 
 #pragma unroll
@@ -760,7 +751,7 @@ k_fused_pairs_2d(const FusedArgs<float> f) {
         const int cnt = (W - 2 * s * R) * (HH - 2 * s * R) / 2;
         int lim = cnt;
         asm volatile("" : "+s"(lim));
-        const T dta = (s == 3) ? dt : dt2;
+        const T dta = (s == 3) ? dt : dt2, dtwa = (s == 3) ? dtw : dtw2;
         const C *yin = (s == 2) ? yb : ya;
         C *yout = (s == 2) ? ya : yb;
 #pragma unroll
@@ -772,18 +763,12 @@ k_fused_pairs_2d(const FusedArgs<float> f) {
             pair_rhs(yin, j, k, kn);
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
-                if (s == 1) {
-                    acc[j][q] = k[q];
-                    if (DYN) accn[j][q] = kn[q];
-                } else {
-                    acc[j][q].x = acc[j][q].x + (T)2 * k[q].x;
-                    acc[j][q].y = acc[j][q].y + (T)2 * k[q].y;
-                    if (DYN) accn[j][q] = accn[j][q] + (T)2 * kn[q];
-                }
-                C yv = mk<T>(uu[j][q].x + k[q].x * dta, uu[j][q].y + k[q].y * dta);
-                if (BC != BC_PERIODIC && !((inside >> (2 * j + q)) & 1ull)) yv = mk<T>(0, 0);
-                yout[li[j] + q * WS] = yv;
-                if (DYN) yn[j][q] = nn[j][q] + kn[q] * dta;
+                grid_acc(acc[j][q].x, k[q].x, s == 1);
+                grid_acc(acc[j][q].y, k[q].y, s == 1);
+                if (DYN) grid_acc(accn[j][q], kn[q], s == 1);
+                const C yv = mk<T>(grid_input(uu[j][q].x, k[q].x, dtwa), grid_input(uu[j][q].y, k[q].y, dtwa));
+                if (BC != BC_REF || ((inside >> (2 * j + q)) & 1u)) yout[li[j] + q * WS] = yv;
+                if (DYN) yn[j][q] = grid_input(nn[j][q], kn[q], dta);
             }
         }
         __syncthreads();
@@ -803,8 +788,9 @@ k_fused_pairs_2d(const FusedArgs<float> f) {
         for (int q = 0; q < 2; ++q) {
             if (gy + q >= ylim) break;
             const size_t gi = (size_t)(gy + q) * n + gx;
-            uo[gi] = mk<T>(uu[j][q].x + (acc[j][q].x + k[q].x) * dt6, uu[j][q].y + (acc[j][q].y + k[q].y) * dt6);
-            if (DYN) uno[gi] = nn[j][q] + (accn[j][q] + kn[q]) * dt6;
+            uo[gi] = mk<T>(grid_new(uu[j][q].x, acc[j][q].x, k[q].x, dtw6),
+                           grid_new(uu[j][q].y, acc[j][q].y, k[q].y, dtw6));
+            if (DYN) uno[gi] = grid_new(nn[j][q], accn[j][q], kn[q], dt6);
         }
     }
 }
@@ -1049,15 +1035,16 @@ static void launch_batch_stage(int dim, int order, int bc, bool dyn, const Batch
 template <typename T, int O, int B, bool D, bool S32 = false>
 static void launch_fused_form(int form, const FusedArgs<T> &f, hipStream_t s) {
     const dim3 grid(8 * f.chunk);
-    // periodic grids (the variants with reflecting boundaries or row slabs
-    // would spill registers in pairs and keep one point per entry)
-    if constexpr (sizeof(T) == 4 && O == 5 && B == BC_PERIODIC && NLS_FUSED_PAIRS) {
+    if constexpr (sizeof(T) == 4 && O == 5 && NLS_FUSED_PAIRS) {
+        // zero-outside grids with a reservoir field would spill at 1024
+        // threads (64 registers) and run the tall tile on 512
+        constexpr int TALL = B == BC_REF && D ? FORM_TALL512 : FORM_TALL;
         if (form == FORM_SHORT)
             hipLaunchKernelGGL((k_fused_pairs_2d<B, D, FORM_SHORT>), grid, dim3(1024), 0, s, f);
-        else if (form == FORM_TALL512)
+        else if (form == FORM_TALL512 && B == BC_PERIODIC)
             hipLaunchKernelGGL((k_fused_pairs_2d<B, D, FORM_TALL512>), grid, dim3(512), 0, s, f);
         else
-            hipLaunchKernelGGL((k_fused_pairs_2d<B, D, FORM_TALL>), grid, dim3(1024), 0, s, f);
+            hipLaunchKernelGGL((k_fused_pairs_2d<B, D, TALL>), grid, dim3(FusedTile<T, O, TALL>::NT), 0, s, f);
         return;
     }
     if constexpr (O != 7) {
@@ -1207,6 +1194,7 @@ template <typename T> static MemberDev<T> plain_member(const nls_problem *p) {
     d.tab = -1;
     d.dt = (T)p->dt;
     d.c = make_coeffs<T>(p->coeffs);
+    d.g = make_grid_coeffs<T>(p->coeffs, p->order, p->dt, p->dx);
     T w[4] = {0, 0, 0, 0};
     for (int q = 0; q <= (p->order - 1) / 2; ++q) w[q] = (T)stencil_s2(p->order, q, p->dx);
     d.w0 = w[0]; d.w1 = w[1]; d.w2 = w[2]; d.w3 = w[3];
@@ -1470,6 +1458,7 @@ static void fill_members(nls_batch *b, const nls_member *ms, const int *ids) {
         d.dV = radial ? 2.0 * M_PI * m.dx * m.dx : (b->dim == 1 ? m.dx : m.dx * m.dx);
         d.dt = (T)m.dt;
         d.c = make_coeffs<T>(m.coeffs);
+        d.g = make_grid_coeffs<T>(m.coeffs, b->order, m.dt, m.dx);
         const int R = (b->order - 1) / 2;
         T w[4] = {0, 0, 0, 0};
         for (int q = 0; q <= R; ++q) w[q] = (T)stencil_s2(b->order, q, m.dx);

@@ -71,24 +71,6 @@ __device__ __forceinline__ void rhs_point_cp(const Coeffs<T> &c, T cP, cplx_t<T>
     if (DYN) kn = fma(-fma(c.d14, s, c.d13), yn, cP);
 }
 
-// The same right-hand side with the Laplacian given as its neighbour part S
-// (lap = wc y + S, wc the centre weight): the centre term joins the
-// point's own factor, q' = c5 |y|^2 + c6 r - wc, so
-//   k.re = (c3 r - c4) y.re + q' y.im - S.im,  k.im = (c3 r - c4) y.im - q' y.re + S.re,
-// which saves the two products wc y.re, wc y.im.  Equal to rhs_point_cp up to
-// rounding (q' rounds at the scale of wc, as wc y does in the sum).
-template <typename T, bool DYN>
-__device__ __forceinline__ void rhs_point_centre(const Coeffs<T> &c, T cP, T wc, cplx_t<T> y, T yn, cplx_t<T> S,
-                                                 cplx_t<T> &k, T &kn) {
-    const T s = y.x * y.x + y.y * y.y;
-    const T r = DYN ? yn : cP / (c.c13 + c.c14 * s);
-    const T g = c.c3 * r - c.c4;
-    const T q = fma(c.c5, s, fma(c.c6, r, -wc));
-    k.x = fma(g, y.x, fma(q, y.y, -S.y));
-    k.y = fma(g, y.y, fma(-q, y.x, S.x));
-    if (DYN) kn = fma(-fma(c.d14, s, c.d13), yn, cP);
-}
-
 template <typename T, bool DYN>
 __device__ __forceinline__ void rhs_point(const Coeffs<T> &c, T P, cplx_t<T> y, T yn, cplx_t<T> lap,
                                           cplx_t<T> &k, T &kn) {
@@ -121,6 +103,86 @@ template <typename T> __device__ __forceinline__ T lap_quad(T w, T c, T a0, T a1
     if (sizeof(T) == 8) return w * ((a0 + a1) + (b0 + b1));
     if (d == 1) return w * (((a0 - c) + (a1 - c)) + ((b0 - c) + (b1 - c)));
     return w * (((a0 + a1) + (b0 + b1)) - (T)4 * c);
+}
+
+// Coefficients of the fused 2-D step.  Single precision keeps the slopes of
+// psi in units of the first neighbour weight w_1: with K = k / w_1 the
+// neighbour sum enters with weights 1, w_2/w_1, w_3/w_1 (order 5: -1/16,
+// exact), the centre weight becomes 2 w_0/w_1 (-3.75, exact) and joins the
+// point's own factor, and the step sizes take the factor w_1 back (dt w_1).
+// Two products a point and stage fewer; and what is large in the Laplacian,
+// its weights, is no longer rounded: against 64 bits the 2048^2 grid ends 300
+// steps 5.8e-7 off instead of 3.3e-6, the 512-grid sweep 500 steps 5.9e-7
+// instead of 2.1e-6.  Double precision takes the weights as they are (the
+// unit of its slopes is 1).  The reservoir's slope keeps its own units.
+template <typename T> struct GridCoeffs {
+    T c3, c4, c5, c6, wc;    // c_k / unit, 2 w_0 / unit
+    T r1, r2, r3;            // w_d / unit
+    T dtw;                   // dt unit
+};
+template <typename T> inline GridCoeffs<T> make_grid_coeffs(const double *c, int order, double dt, double dx) {
+    // where the Laplacian's weights vanish beside the coefficients (a spacing
+    // beyond 1e14 or so), the unit is held at 2^-100 of the largest
+    // coefficient, so that the quotients stay in range; the Laplacian then
+    // stays far below rounding
+    double cmax = 0.0;
+    for (int k = 2; k < 6; ++k) cmax = c[k] > cmax ? c[k] : -c[k] > cmax ? -c[k] : cmax;
+    const double w = stencil_s2(order, 1, dx), least = cmax * 0x1p-100;
+    const double unit = sizeof(T) == 8 ? 1.0 : w > least ? w : least;
+    // in units of w_1 the ratios do not depend on the spacing
+    const double h = sizeof(T) == 8 ? dx : 1.0, per = sizeof(T) == 8 ? 1.0 : stencil_s2(order, 1, 1.0);
+    GridCoeffs<T> g;
+    g.c3 = (T)(c[2] / unit); g.c4 = (T)(c[3] / unit); g.c5 = (T)(c[4] / unit); g.c6 = (T)(c[5] / unit);
+    g.wc = (T)(2.0 * stencil_s2(order, 0, h) / per);
+    g.r1 = (T)(stencil_s2(order, 1, h) / per);
+    g.r2 = order > 3 ? (T)(stencil_s2(order, 2, h) / per) : (T)0;
+    g.r3 = order > 5 ? (T)(stencil_s2(order, 3, h) / per) : (T)0;
+    g.dtw = (T)(dt * unit);
+    return g;
+}
+
+// Arithmetic of one point of the fused 2-D step, shared by its kernels, with
+// every fused multiply-add written out and contraction off: a grid's result
+// has the same bits in every form, tile shape and row slab.
+// The neighbour sum, ring by ring: sum of r_d ((left + right) + (up + down)),
+// r_1 = 1 in single precision.
+template <typename T> __device__ __forceinline__ T grid_ring1(const GridCoeffs<T> &g, T l, T r, T u, T d) {
+#pragma clang fp contract(off)
+    const T s = (l + r) + (u + d);
+    return sizeof(T) == 4 ? s : g.r1 * s;
+}
+template <typename T> __device__ __forceinline__ T grid_ring(T S, T ratio, T l, T r, T u, T d) {
+#pragma clang fp contract(off)
+    return fma(ratio, (l + r) + (u + d), S);
+}
+// Slopes at a point (y, yn) from its neighbour sum S.
+template <typename T, bool DYN>
+__device__ __forceinline__ void grid_rhs(const GridCoeffs<T> &g, const Coeffs<T> &c, T cP, cplx_t<T> y, T yn,
+                                         cplx_t<T> S, cplx_t<T> &k, T &kn) {
+#pragma clang fp contract(off)
+    const T s = fma(y.x, y.x, y.y * y.y);
+    const T r = DYN ? yn : cP / fma(c.c14, s, c.c13);
+    const T a = fma(g.c3, r, -g.c4);
+    T q;
+    if constexpr (sizeof(T) == 4) {
+        q = fma(g.c5, s, fma(g.c6, r, -g.wc));
+    } else {
+        q = fma(g.c5, s, g.c6 * r);
+        S.x = fma(g.wc, y.x, S.x);
+        S.y = fma(g.wc, y.y, S.y);
+    }
+    k.x = fma(a, y.x, fma(q, y.y, -S.y));
+    k.y = fma(a, y.y, fma(-q, y.x, S.x));
+    kn = DYN ? fma(-fma(c.d14, s, c.d13), yn, cP) : (T)0;
+}
+// Accumulator after stage s = 1..3, the next stage's input u + k step, and
+// the new state u + (acc + k4) dt/6.
+template <typename T> __device__ __forceinline__ void grid_acc(T &acc, T k, bool first) {
+    acc = first ? k : fma((T)2, k, acc);
+}
+template <typename T> __device__ __forceinline__ T grid_input(T u, T k, T step) { return fma(k, step, u); }
+template <typename T> __device__ __forceinline__ T grid_new(T u, T acc, T k, T step6) {
+    return fma(acc + k, step6, u);
 }
 
 // Arithmetic of one point of a 1-D line, shared by the resident and the line
