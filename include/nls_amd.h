@@ -247,8 +247,9 @@ int nls_rhs(const nls_problem *p, const void *pumping, const void *psi, const vo
  * counterpart in the reference. */
 int nls_tune_stage_tile(int dtype, int rows);
 
-/* Tile form of the fused RK4 kernel for dtype: 0 chooses it per launch from
- * the tile counts against the compute units (the default), 1 = 64 x 32 tiles
+/* Tile form of the fused RK4 kernel for dtype: 0 chooses per launch (the
+ * default: order-5 periodic launches that fill the device march down strips of
+ * columns, others take the tile form that suits their tile counts), 1 = 64 x 32 tiles
  * of 1024 threads (64 x 16 at order 7), 2 = 64 x 16 tiles of 1024 threads,
  * 3 = 64 x 16 tiles of 512 threads with one stage buffer (double precision
  * on periodic grids; elsewhere it runs as 1), 4 = 64 x 32 tiles of 512

@@ -30,27 +30,12 @@
 
 #include "nls_amd.h"
 #include "nls_internal.h"
+#include "nls_march.h"
 #include "nls_rk4.h"
 
 namespace nls {
 
 constexpr int BATCH_STAGE_TY = 16;    // tile height of the STAGE engine's 2-D tiles
-
-template <typename T> struct MemberDev {
-    int n, steps;
-    long long off;          // first point of the member in the packed arrays
-    long long tab;          // first entry of its radial table (1-D ref), else -1
-    int id, pad;            // the member's index in the caller's batch (observables go to out[4 id ..])
-    double dV;              // volume element of its observables
-    T dt;
-    T w0, w1, w2, w3;       // Cartesian second-derivative weights
-    Coeffs<T> c;
-    GridCoeffs<T> g;        // of the fused 2-D step
-};
-
-struct TileDesc {
-    int m, x0, y0, pad;
-};
 
 template <typename T> struct BatchArgs {
     const MemberDev<T> *mem;
@@ -1142,6 +1127,130 @@ static int fused_form(int dtype, int order, int bc, long long tiles16, long long
 }
 static long long tiles_of(int n, int rows, int ty) { return (long long)((n + 63) / 64) * ((rows + ty - 1) / ty); }
 
+// ---- marching strips or tiles ------------------------------------------------
+// The marching kernel (nls_march.hip: order 5, periodic) runs the step of
+// launches that fill the device; its strips are cut for that.  Times in us on
+// MI355X, as measured:
+//  - a piece costs its rows and MARCH_PIECE more (its halo's stages and first
+//    loads), and a CU's workgroups add up: 0.37 a row for one on the CU (one
+//    wave a SIMD does not hide its latency), 0.23 for each of several; double
+//    precision 0.55 and 0.45;
+//  - a round of tiles (512 of the pair kernel's 64 x 32, 512 of double
+//    precision's 64 x 16) costs 7.4 and 7.7.
+// us per step, tiles -> strips: 2048^2 FP32 32.5 -> 26.5, FP64 58.6 -> 49; 154
+// grids of 128^2 and 102 of 256^2 FP32 73 -> 52, FP64 175 -> 117; 64 of 200^2
+// FP32 28.1 -> 21.9, FP64 52.4 -> 40.8; one 1024^2 grid stays on tiles (11.7; FP64
+// 19.8 as strips and tiles).
+constexpr double MARCH_LAUNCH = 3.0;
+constexpr int MARCH_PIECE = 16;
+static double march_us(int dtype, int percu, int rows) {
+    return percu * rows * (dtype == NLS_F64 ? (percu > 1 ? 0.45 : 0.55) : (percu > 1 ? 0.23 : 0.37));
+}
+static double tiles_us(int dtype, long long tiles16, long long tiles32) {
+    return MARCH_LAUNCH + (dtype == NLS_F64 ? 7.7 * ((tiles16 + 511) / 512) : 7.4 * ((tiles32 + 511) / 512));
+}
+// Members the kernel takes: rows of at least one wave, and byte offsets that
+// stay below 2^32 when they run past the grid's end by up to its size.
+static bool march_holds(int n, int dtype) {
+    return n >= 64 && (long long)n * n * (dtype == NLS_F64 ? 16 : 8) < (1ll << 31);
+}
+static bool march_applies(int dtype, int order, int bc) {
+    return order == 5 && bc == NLS_BC_PERIODIC && get_fused_form(dtype) < 0;   // a form asked for is a tile form
+}
+// Columns of a strip, strips across and pieces side by side for an n x n grid.
+struct StripShape {
+    int wd, nx, subs;
+};
+static StripShape strip_shape(int n) {
+    if (n <= 256) return StripShape{n, 1, 256 / n};
+    const int nx = (n + 239) / 240;
+    return StripShape{(n + nx - 1) / nx, nx, 1};
+}
+// Workgroups a CU holds at once: registers (three waves a SIMD in single
+// precision, two in double), or LDS.
+static int march_slots(int dtype) { return dtype == NLS_F64 ? 2 : 3; }
+
+// A plain n x n grid: each of its strips cut into equal pieces, one for each of
+// at most `percu` workgroups a CU; no groups where tiles are faster.
+struct MarchGrid {
+    int groups, percu, nx, wd, rows;
+};
+static MarchGrid march_grid(const nls_problem *p) {
+    MarchGrid best = {0, 0, 0, 0, 0};
+    const int n = p->n, cus = device_cus();
+    if (n <= 256 || !march_applies(p->dtype, p->order, p->bc) || !march_holds(n, p->dtype) || cus <= 0) return best;
+    double least = tiles_us(p->dtype, tiles_of(n, n, 16), tiles_of(n, n, 32));
+    const StripShape sh = strip_shape(n);
+    for (int per = 1; per <= march_slots(p->dtype); ++per) {
+        const int pieces = std::max(1, per * cus / sh.nx);
+        const int L = (n + pieces - 1) / pieces, groups = sh.nx * ((n + L - 1) / L);
+        const double t = MARCH_LAUNCH + march_us(p->dtype, per, L + MARCH_PIECE) * ((groups + per * cus - 1) / (per * cus));
+        if (t < least) { least = t; best = MarchGrid{groups, per, sh.nx, sh.wd, L}; }
+    }
+    return best;
+}
+
+// The pieces of a batch's members of up to 256 points a side (full) or of the
+// others: the members' strips laid end to end and cut into pieces of equal
+// cost, one run of pieces for each of `percu` workgroups a CU.
+struct MarchCut {
+    std::vector<StripDesc> strips;
+    std::vector<int> first;              // of each workgroup, and the end
+    int percu = 0;
+    double us = 0;
+};
+static MarchCut march_cut(int dtype, const nls_member *members, int count, bool full, int cus) {
+    MarchCut best;
+    // cuts for workgroups of at most `cost` rows, MARCH_PIECE of them a piece's;
+    // returns the number of workgroups
+    auto cut = [&](int cost, MarchCut *out) {
+        int groups = 1, left = cost;
+        if (out) { out->strips.clear(); out->first.assign(1, 0); }
+        for (int i = 0; i < count; ++i) {
+            const int n = members[i].n;
+            if ((n <= 256) != full) continue;
+            const StripShape sh = strip_shape(n);
+            const int E = (n + sh.subs - 1) / sh.subs;
+            for (int k = 0; k < sh.nx; ++k)
+                for (int y = 0; y < E;) {
+                    if (left < MARCH_PIECE + 12 && left < cost) {     // not for a few rows
+                        ++groups;
+                        left = cost;
+                        if (out) out->first.push_back((int)out->strips.size());
+                    }
+                    const int L = std::min(E - y, left - MARCH_PIECE);
+                    if (out) out->strips.push_back(StripDesc{i, k * sh.wd, sh.wd, y, L, E, sh.subs});
+                    y += L;
+                    left -= L + MARCH_PIECE;
+                }
+        }
+        if (out) out->first.push_back((int)out->strips.size());
+        return groups;
+    };
+    long long rows = 0;
+    for (int i = 0; i < count; ++i) {
+        const StripShape sh = strip_shape(members[i].n);
+        if ((members[i].n <= 256) == full) rows += (long long)sh.nx * ((members[i].n + sh.subs - 1) / sh.subs);
+    }
+    if (rows == 0) return best;
+    for (int per = 1; per <= march_slots(dtype); ++per) {
+        const int groups = per * cus;
+        int lo = std::max(MARCH_PIECE + 11, (int)(rows / groups)), hi = lo + 64;
+        while (cut(hi, nullptr) > groups) { lo = hi; hi += hi / 2; }
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) / 2;
+            if (cut(mid, nullptr) > groups) lo = mid;
+            else hi = mid;
+        }
+        const double us = MARCH_LAUNCH + march_us(dtype, per, hi);
+        if (best.percu && us >= best.us) continue;
+        cut(hi, &best);
+        best.percu = per;
+        best.us = us;
+    }
+    return best;
+}
+
 // The double-precision 2-D order-7 variant would spill registers to scratch;
 // it is not built and such batches use the fused or stage engine.
 template <typename T> constexpr bool resident_2d_ok(int order) { return !(sizeof(T) == 8 && order == 7); }
@@ -1216,12 +1325,26 @@ static int fused_grid_run(const nls_problem *p, int iters, const T *P, cplx_t<T>
     f.chunk = (f.ntiles + 7) / 8;
     f.grid = plain_member<T>(p);
     f.P = P;
+    const MarchGrid mg = march_grid(p);
+    MarchArgs<T> a;
+    memset(&a, 0, sizeof a);
+    a.groups = mg.groups;
+    a.chunk = (mg.groups + 7) / 8;
+    a.grid_nx = mg.nx; a.grid_wd = mg.wd; a.grid_L = mg.rows;
+    a.grid = f.grid;
+    a.P = P;
     C *cur = psi, *alt = (C *)ws;
     T *curn = nres, *altn = dyn ? (T *)(ws + align256b(N * sizeof(C))) : nullptr;
     for (int it = 0; it < iters; ++it) {
-        f.it = it;
-        f.u = cur; f.un = curn; f.uo = alt; f.uno = altn;
-        launch_fused<T>(p->order, p->bc, dyn, form, f, s);
+        if (mg.groups) {
+            a.it = it;
+            a.u = cur; a.un = curn; a.uo = alt; a.uno = altn;
+            launch_march<T>(dyn, false, mg.percu, a, s);
+        } else {
+            f.it = it;
+            f.u = cur; f.un = curn; f.uo = alt; f.uno = altn;
+            launch_fused<T>(p->order, p->bc, dyn, form, f, s);
+        }
         std::swap(cur, alt);
         std::swap(curn, altn);
     }
@@ -1408,6 +1531,13 @@ struct nls_batch {
     long long tab_total = 0;            // radial table entries (1-D reference grids)
     int min_steps = 0x7fffffff;         // smallest member step budget
     int fform = FORM_TALL;              // fused engine: tile form (fused_form)
+    // fused engine, marching: the pieces of the members of up to 256 points a
+    // side and of the others, on the device one behind the other (strips,
+    // then the workgroups' first pieces, for each)
+    MarchCut cuts[2];
+    bool march = false;
+    void *d_strips = nullptr;
+    size_t cap_strips = 0;
     int flags = 0;                      // NLS_FLAG_EAGER: no step-block graphs
     // the captured step block and the buffers it was captured on
     hipGraphExec_t graph = nullptr;
@@ -1519,10 +1649,30 @@ static int batch_steps(nls_batch *b, int it0, int iters, const T *P, cplx_t<T> *
         f.ntiles = b->ntiles;
         f.chunk = b->chunk;
         f.P = P;
+        MarchArgs<T> a[2];
+        const char *at = (const char *)b->d_strips;
+        for (int w = 0; w < 2; ++w) {
+            const MarchCut &cut = b->cuts[w];
+            memset(&a[w], 0, sizeof a[w]);
+            a[w].mem = f.mem;
+            a[w].strips = (const StripDesc *)at;
+            at += cut.strips.size() * sizeof(StripDesc);
+            a[w].first = (const int *)at;
+            at += cut.first.size() * sizeof(int);
+            a[w].groups = cut.first.empty() ? 0 : (int)cut.first.size() - 1;
+            a[w].chunk = (a[w].groups + 7) / 8;
+            a[w].P = P;
+        }
         for (int it = 0; it < iters; ++it) {
             f.it = it0 + it;
             f.u = cur; f.un = curn; f.uo = alt; f.uno = altn;
-            launch_fused<T>(b->order, b->bc, dyn, b->fform, f, s);
+            if (!b->march) launch_fused<T>(b->order, b->bc, dyn, b->fform, f, s);
+            else
+                for (int w = 0; w < 2; ++w) {
+                    a[w].it = it0 + it;
+                    a[w].u = cur; a[w].un = curn; a[w].uo = alt; a[w].uno = altn;
+                    if (a[w].groups) launch_march<T>(dyn, w == 0, b->cuts[w].percu, a[w], s);
+                }
             std::swap(cur, alt);
             std::swap(curn, altn);
         }
@@ -1805,6 +1955,18 @@ static void plan(nls_batch *b, const nls_member *members, int count, const int *
         }
         b->fform = fused_form(b->dtype, b->order, b->bc, tiles16, tiles32);
         ty = fused_ty(b->order, b->fform);
+        const int cus = device_cus();
+        b->march = cus > 0 && count > 0 && march_applies(b->dtype, b->order, b->bc);
+        for (int i = 0; i < count; ++i) b->march = b->march && march_holds(members[i].n, b->dtype);
+        b->cuts[0] = b->cuts[1] = MarchCut();
+        if (b->march) {
+            const double tiles = tiles_us(b->dtype, tiles16, tiles32);
+            // (nothing marches faster than a few rows of every CU)
+            b->march = tiles > MARCH_LAUNCH + march_us(b->dtype, 1, 12 + MARCH_PIECE);
+            if (b->march)
+                for (int w = 0; w < 2; ++w) b->cuts[w] = march_cut(b->dtype, members, count, w == 0, cus);
+            b->march = b->march && b->cuts[0].us + b->cuts[1].us < tiles;
+        }
     }
     if (b->dim == 1) { tx = TILE1; ty = 1; }
     b->h_tiles.clear();
@@ -1845,10 +2007,14 @@ static int upload(nls_batch *b, hipStream_t s, bool tables) {
     if (nm == 0) return NLS_OK;
     const size_t nt = tables ? b->h_tiles.size() * sizeof(TileDesc) : 0;
     const size_t nd = tables ? b->h_dx.size() * sizeof(double) : 0;
+    size_t ns = 0;
+    if (tables && b->march)
+        for (const MarchCut &c : b->cuts) ns += c.strips.size() * sizeof(StripDesc) + c.first.size() * sizeof(int);
     const size_t rs = b->dtype == NLS_F64 ? 8 : 4;
     int rc = grow(&b->d_mem, &b->cap_mem, nm, s, "batch members");
     if (!rc && nt) rc = grow(&b->d_tiles, &b->cap_tiles, nt, s, "batch tiles");
     if (!rc && nd) rc = grow(&b->d_dx, &b->cap_dx, nd, s, "batch spacings");
+    if (!rc && ns) rc = grow(&b->d_strips, &b->cap_strips, ns, s, "batch strips");
     if (!rc && tables && b->tab_total > 0) rc = grow(&b->d_wtab, &b->cap_wtab, b->tab_total * rs, s, "radial tables");
     if (rc) return rc;
     nls_batch::Stage &st = b->stage[b->stage_next];
@@ -1856,7 +2022,7 @@ static int upload(nls_batch *b, hipStream_t s, bool tables) {
     if (!st.done) rc = hip_check(hipEventCreateWithFlags(&st.done, hipEventDisableTiming), "staging event");
     else rc = hip_check(hipEventSynchronize(st.done), "staging slot");
     if (rc) return rc;
-    const size_t om = 0, ot = align256b(nm), od = ot + align256b(nt), need = od + nd;
+    const size_t om = 0, ot = align256b(nm), od = ot + align256b(nt), os = od + align256b(nd), need = os + ns;
     if (need > st.cap) {
         if (st.host) (void)hipHostFree(st.host);
         st.host = nullptr;
@@ -1869,9 +2035,20 @@ static int upload(nls_batch *b, hipStream_t s, bool tables) {
     memcpy(h + om, b->h_mem.data(), nm);
     if (nt) memcpy(h + ot, b->h_tiles.data(), nt);
     if (nd) memcpy(h + od, b->h_dx.data(), nd);
+    if (ns) {
+        char *to = h + os;
+        for (const MarchCut &c : b->cuts) {
+            memcpy(to, c.strips.data(), c.strips.size() * sizeof(StripDesc));
+            to += c.strips.size() * sizeof(StripDesc);
+            memcpy(to, c.first.data(), c.first.size() * sizeof(int));
+            to += c.first.size() * sizeof(int);
+        }
+    }
     rc = hip_check(hipMemcpyAsync(b->d_mem, h + om, nm, hipMemcpyHostToDevice, s), "upload members");
     if (!rc && nt) rc = hip_check(hipMemcpyAsync(b->d_tiles, h + ot, nt, hipMemcpyHostToDevice, s), "upload tiles");
     if (!rc && nd) rc = hip_check(hipMemcpyAsync(b->d_dx, h + od, nd, hipMemcpyHostToDevice, s), "upload spacings");
+    if (!rc && ns)
+        rc = hip_check(hipMemcpyAsync(b->d_strips, h + os, ns, hipMemcpyHostToDevice, s), "upload strips");
     if (!rc) rc = hip_check(hipEventRecord(st.done, s), "staging event");
     if (!rc && tables && b->tab_total > 0) {
         if (b->dtype == NLS_F64)
@@ -2047,7 +2224,7 @@ int nls_batch_destroy(nls_batch *b) {
         }
         if (st.host) (void)hipHostFree(st.host);
     }
-    for (void *p : {b->d_mem, b->d_tiles, b->d_dx, b->d_wtab, b->d_obs})
+    for (void *p : {b->d_mem, b->d_tiles, b->d_dx, b->d_wtab, b->d_obs, b->d_strips})
         if (p) (void)hipFree(p);
     delete b;
     return NLS_OK;

@@ -1,0 +1,51 @@
+// nls_march.h -- members of a launch (batches and plain grids) and the launch
+// interface of the marching kernel (nls_march.hip).
+#pragma once
+#include "nls_core.h"
+
+namespace nls {
+
+template <typename T> struct MemberDev {
+    int n, steps;
+    long long off;          // first point of the member in the packed arrays
+    long long tab;          // first entry of its radial table (1-D ref), else -1
+    int id, pad;            // the member's index in the caller's batch (observables go to out[4 id ..])
+    double dV;              // volume element of its observables
+    T dt;
+    T w0, w1, w2, w3;       // Cartesian second-derivative weights
+    Coeffs<T> c;
+    GridCoeffs<T> g;        // of the fused 2-D step
+};
+
+struct TileDesc {
+    int m, x0, y0, pad;
+};
+
+// A piece of a member: columns x0 .. x0 + wd - 1, rows y0 .. y0 + L - 1 of each
+// of `subs` row ranges of E rows side by side in the workgroup (range s starts
+// at row s E; rows past the grid's end are dropped).
+struct StripDesc {
+    int m, x0, wd, y0, L, E, subs;
+};
+
+template <typename T> struct MarchArgs {
+    const MemberDev<T> *mem;
+    const StripDesc *strips;
+    const int *first;                    // the workgroups' pieces
+    int groups, chunk;                   // workgroups; an eighth of them, rounded up
+    int it;
+    const cplx_t<T> *u; const T *un;     // state at the start of the step
+    cplx_t<T> *uo; T *uno;               // state at its end
+    const T *P;
+    // one grid (n > 256) instead of a member table: grid_nx > 0 strips of
+    // grid_wd columns across, pieces of grid_L rows
+    int grid_nx, grid_wd, grid_L;
+    MemberDev<T> grid;
+};
+
+// full: every strip spans its member's whole rows (64 <= n <= 256 columns,
+// up to 256 / n pieces side by side); else strips of at most 240 columns of
+// members of n > 256.  percu: workgroups a CU is to hold at once, at most.
+template <typename T> void launch_march(bool dyn, bool full, int percu, const MarchArgs<T> &a, hipStream_t s);
+
+}  // namespace nls
