@@ -322,8 +322,8 @@ k_fused_step_2d(const FusedArgs<T> f) {
         return;
     }
 
-    const T dt = m.dt, dt2 = dt * (T)0.5, dt6 = dt / (T)6;                   // of the reservoir
-    const T dtw = m.g.dtw, dtw2 = dtw * (T)0.5, dtw6 = dtw / (T)6;           // of psi
+    const T dt = m.dt, dt2 = dt * (T)0.5, dt6 = m.g.dt6;                   // of the reservoir
+    const T dtw = m.g.dtw, dtw2 = dtw * (T)0.5, dtw6 = m.g.dtw6;           // of psi
     Coeffs<T> c = m.c;
     GridCoeffs<T> g = m.g;
     if constexpr (sizeof(T) == 4) {
@@ -628,8 +628,8 @@ k_fused_pairs_2d(const FusedArgs<float> f) {
         return;
     }
 
-    const T dt = m.dt, dt2 = dt * (T)0.5, dt6 = dt / (T)6;
-    const T dtw = m.g.dtw, dtw2 = dtw * (T)0.5, dtw6 = dtw / (T)6;
+    const T dt = m.dt, dt2 = dt * (T)0.5, dt6 = m.g.dt6;
+    const T dtw = m.g.dtw, dtw2 = dtw * (T)0.5, dtw6 = m.g.dtw6;
     Coeffs<T> c = m.c;
     GridCoeffs<T> g = m.g;
     asm volatile("" : "+v"(g.c4), "+v"(g.wc), "+v"(c.d13), "+v"(c.c13));
@@ -781,13 +781,11 @@ k_fused_pairs_2d(const FusedArgs<float> f) {
 }
 
 // ---------------------------------------------------------------------------
-// Engine RESIDENT: one workgroup per member holds the member's
-// whole grid on chip (1-D n <= 4096, 2-D n <= 64) and runs all of the call's
-// steps in one launch -- a persistent kernel per step block.  LDS holds the
-// psi state at the start of the step (U) and the psi stage input (Y);
-// registers hold each thread's pumping, reservoir, reservoir stage input and
-// accumulators.  HBM is touched only to load the state
-// at the start and store it at the end.
+// Engine RESIDENT: one workgroup per member holds the member's whole grid on
+// chip and runs all of the call's steps in one launch -- a persistent kernel
+// per step block.  HBM is touched only to load the state at the start and
+// store it at the end.  1-D lines (n <= 4096) here; 2-D grids (n <= 64) in
+// nls_small.hip.
 // ---------------------------------------------------------------------------
 
 constexpr int RES_MAXP = 4096;
@@ -796,15 +794,6 @@ constexpr int RES_MAXP = 4096;
 template <typename T> struct ResShape;
 template <> struct ResShape<float> { static constexpr int THREADS = 1024; };
 template <> struct ResShape<double> { static constexpr int THREADS = 512; };
-
-template <typename T> struct ResidentArgs {
-    const MemberDev<T> *mem;
-    int iters;
-    const T *wtab;
-    cplx_t<T> *psi;
-    T *nres;
-    const T *P;
-};
 
 template <typename T, int ORDER, int BC, int DIM>
 __device__ __forceinline__ cplx_t<T> resident_lap(const cplx_t<T> *Y, int idx, int n, const T *w,
@@ -853,39 +842,29 @@ __device__ __forceinline__ cplx_t<T> resident_lap(const cplx_t<T> *Y, int idx, i
     }
 }
 
-template <typename T, bool DYN, int DIM>
-__device__ __forceinline__ void resident_rhs(const Coeffs<T> &c, T P, cplx_t<T> y, T yn, cplx_t<T> lap, cplx_t<T> &k,
-                                             T &kn) {
-    if constexpr (DIM == 1) line_rhs<T, DYN>(c, pump_term<T, DYN>(c, P), y, yn, lap.x, lap.y, k, kn);
-    else rhs_point<T, DYN>(c, P, y, yn, lap, k, kn);
-}
-
-template <typename T, int ORDER, int BC, bool DYN, int DIM>
+template <typename T, int ORDER, int BC, bool DYN>
 __global__ void __launch_bounds__(ResShape<T>::THREADS) k_resident(const ResidentArgs<T> r) {
     using C = cplx_t<T>;
     constexpr int RES_THREADS = ResShape<T>::THREADS, RES_PPT = RES_MAXP / RES_THREADS;
-    // Single precision: Y[b] is the psi stage input, double-buffered -- stage
-    // s reads Y[b] and writes the next stage's input into Y[b ^ 1], so one
-    // barrier per stage suffices (a thread writes Y[b] again only after the
-    // next barrier, which every thread reaches after its reads of Y[b]); the
-    // state at the start of the step is read at the thread's own points only
-    // and stays in registers.  Double precision does the same on 1-D lines of
-    // order 3 and 5; elsewhere it has no registers to spare for that state (it
+    // Y[b] is the psi stage input, double-buffered -- stage s reads Y[b] and
+    // writes the next stage's input into Y[b ^ 1], so one barrier per stage
+    // suffices (a thread writes Y[b] again only after the next barrier, which
+    // every thread reaches after its reads of Y[b]); the state at the start of
+    // the step is read at the thread's own points only and stays in registers.
+    // Double precision of order 7 has no registers to spare for that state (it
     // would spill): Y[0] is the stage input, Y[1] the state, and each stage
     // waits for all reads of Y[0] before writing it.
-    constexpr bool PINGPONG = sizeof(T) == 4 || (DIM == 1 && ORDER < 7);
+    constexpr bool PINGPONG = sizeof(T) == 4 || ORDER < 7;
     __shared__ C Y[2][RES_MAXP];
     const MemberDev<T> m = r.mem[blockIdx.x];
-    const int n = m.n;
-    const int N = DIM == 1 ? n : n * n;
+    const int n = m.n, N = n;
     const int steps = r.iters < m.steps ? r.iters : m.steps;
     if (N > RES_MAXP || steps <= 0) return;        // the host never plans such members
     C *psi = r.psi + m.off;
     T *nres = DYN ? r.nres + m.off : nullptr;
     const T *P = r.P + m.off;
-    const T *wtab = (DIM == 1 && BC == BC_REF) ? r.wtab + m.tab : nullptr;
+    const T *wtab = BC == BC_REF ? r.wtab + m.tab : nullptr;
     const T w[4] = {m.w0, m.w1, m.w2, m.w3};
-    const T dt = m.dt;
     const int tid = threadIdx.x;
     T pp[RES_PPT], un[RES_PPT], yn[RES_PPT], accn[RES_PPT];
     C acc[RES_PPT], uu[PINGPONG ? RES_PPT : 1];
@@ -909,72 +888,52 @@ __global__ void __launch_bounds__(ResShape<T>::THREADS) k_resident(const Residen
     }
     __syncthreads();
     int b = 0;
-    const LineStep<T> h = line_step(dt);          // 1-D lines
+    const LineStep<T> h = line_step(m.dt);
     auto run_stage = [&](auto s_) {
-            constexpr int s = decltype(s_)::value;
-            const T wacc = (s == 1 || s == 4) ? (T)1 : (T)2;
-            const T anext = (s == 3) ? (T)1 : (T)0.5;
-            // acc += wacc k; the next stage input u + k dt anext, or at stage
-            // 4 the new state u + acc dt / 6
-            auto advance_point = [&](int q, int idx, const C &kk, T kn, const C &u, C *Yout) {
-                if constexpr (DIM == 1) {
-                    const C v = mk<T>(line_combine<T, s>(acc[q].x, kk.x, u.x, h),
-                                      line_combine<T, s>(acc[q].y, kk.y, u.y, h));
-                    Yout[idx] = v;
-                    if (DYN) yn[q] = line_combine<T, s>(accn[q], kn, un[q], h);
-                    if (s == 4 && DYN) un[q] = yn[q];
-                    return s == 4 ? v : u;
-                }
-                if (s == 1) { acc[q] = kk; accn[q] = kn; }
-                else {
-                    acc[q] = mk<T>(acc[q].x + wacc * kk.x, acc[q].y + wacc * kk.y);
-                    accn[q] = accn[q] + wacc * kn;
-                }
-                if (s < 4) {
-                    Yout[idx] = mk<T>(u.x + (kk.x * dt) * anext, u.y + (kk.y * dt) * anext);
-                    if (DYN) yn[q] = un[q] + (kn * dt) * anext;
-                    return u;
-                }
-                const C v = mk<T>(u.x + (acc[q].x * dt) / (T)6, u.y + (acc[q].y * dt) / (T)6);
-                Yout[idx] = v;
-                if (DYN) { un[q] = un[q] + (accn[q] * dt) / (T)6; yn[q] = un[q]; }
-                return v;
-            };
-            if constexpr (PINGPONG) {
-                const C *Yin = Y[b];
-                C *Yout = Y[b ^ 1];
+        constexpr int s = decltype(s_)::value;
+        // the next stage input, or at stage 4 the new state; returns the state
+        auto advance_point = [&](int q, int idx, const C &kk, T kn, const C &u, C *Yout) {
+            const C v = mk<T>(line_combine<T, s>(acc[q].x, kk.x, u.x, h), line_combine<T, s>(acc[q].y, kk.y, u.y, h));
+            Yout[idx] = v;
+            if (DYN) yn[q] = line_combine<T, s>(accn[q], kn, un[q], h);
+            if (s == 4 && DYN) un[q] = yn[q];
+            return s == 4 ? v : u;
+        };
+        auto slopes = [&](const C *Yin, int q, int idx, C &kk, T &kn) {
+            const C lap = resident_lap<T, ORDER, BC, 1>(Yin, idx, n, w, wtab ? wtab + (size_t)idx * ORDER : nullptr);
+            line_rhs<T, DYN>(m.c, pump_term<T, DYN>(m.c, pp[q]), Yin[idx], yn[q], lap.x, lap.y, kk, kn);
+        };
+        if constexpr (PINGPONG) {
+            const C *Yin = Y[b];
+            C *Yout = Y[b ^ 1];
 #pragma unroll
-                for (int q = 0; q < RES_PPT; ++q) {
-                    const int idx = tid + RES_THREADS * q;
-                    if (idx >= N) continue;
-                    C kk;
-                    T kn = 0;
-                    const C lap = resident_lap<T, ORDER, BC, DIM>(Yin, idx, n, w, wtab ? wtab + (size_t)idx * ORDER : nullptr);
-                    resident_rhs<T, DYN, DIM>(m.c, pp[q], Yin[idx], yn[q], lap, kk, kn);
-                    uu[PINGPONG ? q : 0] = advance_point(q, idx, kk, kn, uu[PINGPONG ? q : 0], Yout);
-                }
-                __syncthreads();
-                b ^= 1;
-            } else {
-                C kk[RES_PPT];
-                T kn[RES_PPT];
-#pragma unroll
-                for (int q = 0; q < RES_PPT; ++q) {
-                    const int idx = tid + RES_THREADS * q;
-                    kk[q] = mk<T>(0, 0); kn[q] = 0;
-                    if (idx < N) {
-                        const C lap = resident_lap<T, ORDER, BC, DIM>(Y[0], idx, n, w, wtab ? wtab + (size_t)idx * ORDER : nullptr);
-                        resident_rhs<T, DYN, DIM>(m.c, pp[q], Y[0][idx], yn[q], lap, kk[q], kn[q]);
-                    }
-                }
-                __syncthreads();                     // every read of Y[0] for this stage is done
-#pragma unroll
-                for (int q = 0; q < RES_PPT; ++q) {
-                    const int idx = tid + RES_THREADS * q;
-                    if (idx < N) Y[1][idx] = advance_point(q, idx, kk[q], kn[q], Y[1][idx], Y[0]);
-                }
-                __syncthreads();
+            for (int q = 0; q < RES_PPT; ++q) {
+                const int idx = tid + RES_THREADS * q;
+                if (idx >= N) continue;
+                C kk;
+                T kn = 0;
+                slopes(Yin, q, idx, kk, kn);
+                uu[PINGPONG ? q : 0] = advance_point(q, idx, kk, kn, uu[PINGPONG ? q : 0], Yout);
             }
+            __syncthreads();
+            b ^= 1;
+        } else {
+            C kk[RES_PPT];
+            T kn[RES_PPT];
+#pragma unroll
+            for (int q = 0; q < RES_PPT; ++q) {
+                const int idx = tid + RES_THREADS * q;
+                kk[q] = mk<T>(0, 0); kn[q] = 0;
+                if (idx < N) slopes(Y[0], q, idx, kk[q], kn[q]);
+            }
+            __syncthreads();                     // every read of Y[0] for this stage is done
+#pragma unroll
+            for (int q = 0; q < RES_PPT; ++q) {
+                const int idx = tid + RES_THREADS * q;
+                if (idx < N) Y[1][idx] = advance_point(q, idx, kk[q], kn[q], Y[1][idx], Y[0]);
+            }
+            __syncthreads();
+        }
     };
     for (int it = 0; it < steps; ++it) {
         run_stage(std::integral_constant<int, 1>{});
@@ -1136,7 +1095,8 @@ static long long tiles_of(int n, int rows, int ty) { return (long long)((n + 63)
 //    wave a SIMD does not hide its latency), 0.23 for each of several; double
 //    precision 0.55 and 0.45;
 //  - a round of tiles (512 of the pair kernel's 64 x 32, 512 of double
-//    precision's 64 x 16) costs 7.4 and 7.7.
+//    precision's 64 x 16) costs 7.4 and 7.7; short tiles that fit one per CU
+//    5.4 and 6.7 in all.
 // us per step, tiles -> strips: 2048^2 FP32 32.5 -> 26.5, FP64 58.6 -> 49; 154
 // grids of 128^2 and 102 of 256^2 FP32 73 -> 52, FP64 175 -> 117; 64 of 200^2
 // FP32 28.1 -> 21.9, FP64 52.4 -> 40.8; one 1024^2 grid stays on tiles (11.7; FP64
@@ -1146,7 +1106,8 @@ constexpr int MARCH_PIECE = 16;
 static double march_us(int dtype, int percu, int rows) {
     return percu * rows * (dtype == NLS_F64 ? (percu > 1 ? 0.45 : 0.55) : (percu > 1 ? 0.23 : 0.37));
 }
-static double tiles_us(int dtype, long long tiles16, long long tiles32) {
+static double tiles_us(int dtype, long long tiles16, long long tiles32, int cus) {
+    if (tiles16 <= cus) return dtype == NLS_F64 ? 6.7 : 5.4;
     return MARCH_LAUNCH + (dtype == NLS_F64 ? 7.7 * ((tiles16 + 511) / 512) : 7.4 * ((tiles32 + 511) / 512));
 }
 // Members the kernel takes: rows of at least one wave, and byte offsets that
@@ -1179,7 +1140,7 @@ static MarchGrid march_grid(const nls_problem *p) {
     MarchGrid best = {0, 0, 0, 0, 0};
     const int n = p->n, cus = device_cus();
     if (n <= 256 || !march_applies(p->dtype, p->order, p->bc) || !march_holds(n, p->dtype) || cus <= 0) return best;
-    double least = tiles_us(p->dtype, tiles_of(n, n, 16), tiles_of(n, n, 32));
+    double least = tiles_us(p->dtype, tiles_of(n, n, 16), tiles_of(n, n, 32), cus);
     const StripShape sh = strip_shape(n);
     for (int per = 1; per <= march_slots(p->dtype); ++per) {
         const int pieces = std::max(1, per * cus / sh.nx);
@@ -1251,19 +1212,12 @@ static MarchCut march_cut(int dtype, const nls_member *members, int count, bool 
     return best;
 }
 
-// The double-precision 2-D order-7 variant would spill registers to scratch;
-// it is not built and such batches use the fused or stage engine.
-template <typename T> constexpr bool resident_2d_ok(int order) { return !(sizeof(T) == 8 && order == 7); }
-
 template <typename T>
 static void launch_resident(int dim, int order, int bc, bool dyn, int count, const ResidentArgs<T> &r, hipStream_t s) {
+    if (dim == 2) return launch_resident_2d<T>(order, bc, dyn, count, r, s);
 #define NLS_CASE(O, B, D)                                                                                     \
     if (order == O && bc == B && dyn == D) {                                                                 \
-        if (dim == 1)                                                                                        \
-            hipLaunchKernelGGL((k_resident<T, O, B, D, 1>), dim3(count), dim3(ResShape<T>::THREADS), 0, s, r); \
-        else if (resident_2d_ok<T>(O))                                                                       \
-            hipLaunchKernelGGL((k_resident<T, O, B, D, (resident_2d_ok<T>(O) ? 2 : 1)>), dim3(count),         \
-                               dim3(ResShape<T>::THREADS), 0, s, r);                                         \
+        hipLaunchKernelGGL((k_resident<T, O, B, D>), dim3(count), dim3(ResShape<T>::THREADS), 0, s, r);       \
         return;                                                                                               \
     }
     NLS_CASE(3, 0, false) NLS_CASE(3, 0, true) NLS_CASE(3, 1, false) NLS_CASE(3, 1, true)
@@ -1310,6 +1264,14 @@ template <typename T> static MemberDev<T> plain_member(const nls_problem *p) {
     return d;
 }
 
+// Steps a launch of a plain fused solve makes: several on a small grid, unless
+// a tile form is asked for (tiles step once) or the arithmetic is
+// NLS_FLAG_F64_ARITH's.
+int fused_steps_per_launch(const nls_problem *p) {
+    if (get_fused_form(p->dtype) >= 0 || (p->flags & NLS_FLAG_F64_ARITH)) return 1;
+    return std::max(1, multi_steps(p->n, p->order, device_cus()));
+}
+
 template <typename T>
 static int fused_grid_run(const nls_problem *p, int iters, const T *P, cplx_t<T> *psi, T *nres, char *ws,
                           hipStream_t s) {
@@ -1333,10 +1295,21 @@ static int fused_grid_run(const nls_problem *p, int iters, const T *P, cplx_t<T>
     a.grid_nx = mg.nx; a.grid_wd = mg.wd; a.grid_L = mg.rows;
     a.grid = f.grid;
     a.P = P;
+    // a small grid: its own tiles, several steps a launch
+    const int many = get_fused_form(p->dtype) >= 0 ? 0 : multi_steps(p->n, p->order, device_cus());
+    MultiArgs<T> b;
+    memset(&b, 0, sizeof b);
+    b.grid = f.grid;
+    b.P = P;
     C *cur = psi, *alt = (C *)ws;
     T *curn = nres, *altn = dyn ? (T *)(ws + align256b(N * sizeof(C))) : nullptr;
-    for (int it = 0; it < iters; ++it) {
-        if (mg.groups) {
+    for (int it = 0, done; it < iters; it += done) {
+        done = 1;
+        if (many && iters - it >= many) {
+            b.u = cur; b.un = curn; b.uo = alt; b.uno = altn;
+            launch_multi<T>(p->order, p->bc, dyn, b, device_cus(), s);
+            done = many;
+        } else if (mg.groups) {
             a.it = it;
             a.u = cur; a.un = curn; a.uo = alt; a.uno = altn;
             launch_march<T>(dyn, false, mg.percu, a, s);
@@ -1960,7 +1933,7 @@ static void plan(nls_batch *b, const nls_member *members, int count, const int *
         for (int i = 0; i < count; ++i) b->march = b->march && march_holds(members[i].n, b->dtype);
         b->cuts[0] = b->cuts[1] = MarchCut();
         if (b->march) {
-            const double tiles = tiles_us(b->dtype, tiles16, tiles32);
+            const double tiles = tiles_us(b->dtype, tiles16, tiles32, cus);
             // (nothing marches faster than a few rows of every CU)
             b->march = tiles > MARCH_LAUNCH + march_us(b->dtype, 1, 12 + MARCH_PIECE);
             if (b->march)

@@ -51,15 +51,17 @@ int check_problem(const nls_problem *p) {
 // RK4 engine of a plain solve.  AUTO: the line kernel for 1-D (us per step
 // against the engines it replaced: n = 256 FP32 0.56 / 0.88 resident, n = 1000
 // radial FP32 0.59 / 3.6, n = 4096 FP64 0.67 / 6.3; longer lines took 8 to 15
-// on the per-stage kernels, 20,000 points take 0.67); in 2-D the resident
-// kernel when the grid fits one workgroup -- up to 64 x 64 in single precision
-// (in double precision one workgroup computing the whole grid is slower than
-// the fused kernel's tiles) -- else the fused one-launch-per-step kernel.
+// on the per-stage kernels, 20,000 points take 0.67); in 2-D the fused engine,
+// whose small grids step several times a launch: 40^2 order 3 FP32 1.76 us per
+// step against 2.12 of one workgroup holding the grid (resident), 64^2 order 5
+// 3.0 against 5.0, 16^2 the same.  At order 7, one step a launch, the resident
+// kernel is faster up to 48^2 in single precision (4.0 against 4.7; 64^2 6.3
+// against 4.7).
 int plain_engine(const nls_problem *p) {
     if (p->flags & NLS_FLAG_F64_ARITH) return NLS_ENGINE_FUSED;
     if (p->engine != NLS_ENGINE_AUTO) return p->engine;
     if (p->dim == 1) return ENGINE_LINE;
-    if (resident_fits(p) && p->dtype == NLS_F32) return NLS_ENGINE_RESIDENT;
+    if (p->order == 7 && p->n <= 48 && p->dtype == NLS_F32) return NLS_ENGINE_RESIDENT;
     return fused_holds((long long)p->n * p->n, p->dtype) ? NLS_ENGINE_FUSED : NLS_ENGINE_STAGE;
 }
 
@@ -256,7 +258,11 @@ static thread_local GraphCache *g_graphs = nullptr;
 static bool graphs_apply(const nls_problem *p, int iters) {
     if ((p->flags & NLS_FLAG_EAGER) || iters < 2 * GRAPH_BLOCK || p->scheme != NLS_SCHEME_RK4) return false;
     const int engine = plain_engine(p);
-    return engine == NLS_ENGINE_FUSED || engine == NLS_ENGINE_STAGE;
+    // launches of several steps outlast their issue: replaying them as a graph
+    // gains nothing (256^2: 3.70 us per step replayed, 3.68 issued) and the
+    // capture costs a first call a tenth of a millisecond or more
+    if (engine == NLS_ENGINE_FUSED) return fused_steps_per_launch(p) == 1;
+    return engine == NLS_ENGINE_STAGE;
 }
 
 static int block_graph(const nls_problem *p, const void *P, void *psi, void *nres, void *ws, hipGraphExec_t *out) {

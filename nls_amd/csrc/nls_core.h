@@ -118,7 +118,7 @@ template <typename T> __device__ __forceinline__ T lap_quad(T w, T c, T a0, T a1
 template <typename T> struct GridCoeffs {
     T c3, c4, c5, c6, wc;    // c_k / unit, 2 w_0 / unit
     T r1, r2, r3;            // w_d / unit
-    T dtw;                   // dt unit
+    T dtw, dtw6, dt6;        // dt unit, dt unit / 6, dt / 6, each rounded once
 };
 template <typename T> inline GridCoeffs<T> make_grid_coeffs(const double *c, int order, double dt, double dx) {
     // where the Laplacian's weights vanish beside the coefficients (a spacing
@@ -138,6 +138,8 @@ template <typename T> inline GridCoeffs<T> make_grid_coeffs(const double *c, int
     g.r2 = order > 3 ? (T)(stencil_s2(order, 2, h) / per) : (T)0;
     g.r3 = order > 5 ? (T)(stencil_s2(order, 3, h) / per) : (T)0;
     g.dtw = (T)(dt * unit);
+    g.dtw6 = (T)(dt * unit / 6.0);
+    g.dt6 = (T)(dt / 6.0);
     return g;
 }
 

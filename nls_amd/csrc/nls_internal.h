@@ -25,6 +25,7 @@ int get_fused_form(int dtype);
 size_t fused_grid_workspace_bytes(const nls_problem *p);
 int fused_grid_advance(const nls_problem *p, int iters, const void *pumping, void *psi, void *nres, void *ws,
                        hipStream_t s);
+int fused_steps_per_launch(const nls_problem *p);
 // one RK4 step of a row slab with 4R ghost rows on each side (fused kernel, BC_SLAB)
 int fused_slab_step(const nls_problem *p, int rows, const void *P, const void *psi_in, const void *nres_in,
                     void *psi_out, void *nres_out, hipStream_t s);

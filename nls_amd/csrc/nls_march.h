@@ -1,5 +1,6 @@
 // nls_march.h -- members of a launch (batches and plain grids) and the launch
-// interface of the marching kernel (nls_march.hip).
+// interfaces of the marching kernel (nls_march.hip) and of the small grids'
+// kernels (nls_small.hip).
 #pragma once
 #include "nls_core.h"
 
@@ -47,5 +48,32 @@ template <typename T> struct MarchArgs {
 // up to 256 / n pieces side by side); else strips of at most 240 columns of
 // members of n > 256.  percu: workgroups a CU is to hold at once, at most.
 template <typename T> void launch_march(bool dyn, bool full, int percu, const MarchArgs<T> &a, hipStream_t s);
+
+template <typename T> struct ResidentArgs {
+    const MemberDev<T> *mem;
+    int iters;
+    const T *wtab;
+    cplx_t<T> *psi;
+    T *nres;
+    const T *P;
+};
+
+// One workgroup per member of a batch of 2-D grids of up to 64 x 64, all steps
+// of a call in one launch (nls_small.hip; not double precision of order 7).
+template <typename T>
+void launch_resident_2d(int order, int bc, bool dyn, int count, const ResidentArgs<T> &r, hipStream_t s);
+
+// Several steps of one small grid per launch (nls_small.hip).
+template <typename T> struct MultiArgs {
+    int ntx;                             // tiles across
+    const cplx_t<T> *u; const T *un;
+    cplx_t<T> *uo; T *uno;
+    const T *P;
+    MemberDev<T> grid;
+};
+// Steps a launch makes on an n x n grid (0: not such a grid).
+int multi_steps(int n, int order, int cus);
+template <typename T>
+void launch_multi(int order, int bc, bool dyn, MultiArgs<T> a, int cus, hipStream_t s);
 
 }  // namespace nls

@@ -107,8 +107,8 @@ __device__ __forceinline__ void march_piece(const MarchArgs<T> &f, const StripDe
     const __amdgpu_buffer_rsrc_t ru = rsrc(u, cbytes), rp = rsrc(P, cbytes / 2), rn = rsrc(DYN ? un : P, cbytes / 2),
                                  wu = rsrc(uo, cbytes), wn = rsrc(DYN ? uno : nullptr, DYN ? cbytes / 2 : 0);
 
-    const T dt = m.dt, dt2 = dt * (T)0.5, dt6 = dt / (T)6;
-    const T dtw = m.g.dtw, dtw2 = dtw * (T)0.5, dtw6 = dtw / (T)6;
+    const T dt = m.dt, dt2 = dt * (T)0.5, dt6 = m.g.dt6;
+    const T dtw = m.g.dtw, dtw2 = dtw * (T)0.5, dtw6 = m.g.dtw6;
     Coeffs<T> c = m.c;
     GridCoeffs<T> g = m.g;
     if constexpr (sizeof(T) == 4) asm volatile("" : "+v"(g.c4), "+v"(g.wc), "+v"(c.d13), "+v"(c.c13));
