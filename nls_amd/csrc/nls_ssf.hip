@@ -15,8 +15,8 @@
 //               inverse y-FFT                          (reads/writes psi)
 // so a step moves 4 c + 3 r bytes per point (c complex, r real).  The first
 // row pass has no inverse transform and the last one no forward transform.
-// 1-D: a workgroup holds a whole line (n <= 4096) in LDS and runs all steps
-// on chip.
+// 1-D: a workgroup holds a whole line (n <= 4096) in registers and runs all
+// steps on chip.
 //
 // Precision: the fields sit in HBM in the problem's dtype; every kernel
 // computes in double precision (FFT stages, pointwise RK4, twiddle and phase
@@ -26,39 +26,23 @@
 // HBM bytes; rounding the state once per pass instead of at every FFT stage
 // keeps its error far below that of single-precision transforms.
 //
-// FFTs: in-place Stockham stages, radix-8 while at least three factors of two
-// remain, then radix-4 and a last radix-2 as needed, on the complex values a
-// workgroup holds in LDS (2048 in the 2-D passes, 4096 for a 1-D line); each
+// FFTs: Stockham stages with a line's values in the registers of its threads,
+// the stage-to-stage exchanges through LDS (fft_regs).  The middle row pass of
+// 2048-point rows and the kinetic energy keep them in LDS and work in place: a
 // stage stages its butterfly inputs and twiddles in registers, synchronises,
-// then writes the outputs in place.  Twiddles exp(-2 pi i m / n) and the
-// phase table are generated in double precision.
+// then writes the outputs.  Twiddles exp(-2 pi i m / n) and the phase table are
+// generated in double precision.
 #include <cstring>
+#include <type_traits>
 
 #include "nls_core.h"
 #include "nls_internal.h"
 
 namespace nls {
 
-// Points and threads per workgroup.  Row and column passes hold one
-// 2048-point line (or several shorter lines) per workgroup: 32 KB of LDS in
-// double precision, so up to five workgroups share a CU.  The 1-D kernel
-// holds a whole line of up to 4096 points in one workgroup (1024 threads in
-// single precision; 512 in double precision, within 256 registers).
+// Row kernels with their values in LDS: one 2048-point line (or several
+// shorter lines) per workgroup, 32 KB, so four workgroups share a CU.
 constexpr int ROW_PTS = 2048, ROW_LOG_PTS = 11, ROW_NTH = 256;
-constexpr int LINE_PTS = 4096;
-template <typename T> struct LineShape { static constexpr int NTH = sizeof(T) == 8 ? 512 : 1024; };
-// Column pass: 2^LOG_L adjacent columns per workgroup (fewer when n is
-// smaller), so each row segment it reads and writes is 32 bytes: two FP64
-// or four FP32 columns.  More columns per workgroup would only leave fewer
-// workgroups for small grids.  WIDE: the 2048-point column pass (stages in
-// registers), four columns per workgroup of 1024 threads, 136 KB of LDS, one
-// workgroup per CU: 64-byte row segments (2048^2 per step, same box, two
-// rounds: FP64 99.6 -> 96.6 us, FP32 storage 89.9 -> 88.1 us; one column
-// per workgroup, 16-byte segments: 123 / 108 us).
-template <typename T, bool WIDE = false> struct ColShape;
-template <> struct ColShape<double, false> { static constexpr int LOG_L = 1, PTS = 4096, NTH = 512; };
-template <> struct ColShape<double, true> { static constexpr int LOG_L = 2, PTS = 8192, NTH = 1024; };
-
 // LDS layout of the transforms: element i at i + (i >> SHIFT), one complex of
 // padding per 2^SHIFT, so that the strided writes of the first radix-8
 // stages (stride 8, then groups of 8 at stride 64) spread over the LDS banks
@@ -70,13 +54,6 @@ template <> struct ColShape<double, true> { static constexpr int LOG_L = 2, PTS 
 #endif
 #ifndef NLS_SSF_COL_PAD
 #define NLS_SSF_COL_PAD 4
-#endif
-// The 2048-point column pass (four columns, stages in registers) is the
-// faster unpadded: 2048^2 per step, same box, two rounds each, FP64 95.2 /
-// 94.8 -> 93.8 / 93.7 us, FP32 storage 87.8 / 87.6 -> 87.0 / 87.1 us (one pad
-// per 8 or per 32 complex: in between).
-#ifndef NLS_SSF_COL2048_PAD
-#define NLS_SSF_COL2048_PAD 31
 #endif
 #ifndef NLS_SSF_LINE_PAD
 #define NLS_SSF_LINE_PAD 4
@@ -546,264 +523,60 @@ __host__ __device__ constexpr int lines_per_wg(int logN, int logP) {
     return logP - logN < logN ? logP - logN : logN;
 }
 
-// Row pass: 2^(11-logN) rows per workgroup (at most n).
-// ROW2048: the middle row pass of a grid of 2048-point rows, a kernel of its
-// own, held to 128 registers (four waves per SIMD; in one kernel with the
-// general path, or left to the compiler with double-precision storage, it
-// took 131-136 and three).
-template <typename S, typename T, bool DYN, int MODE, bool ROW2048 = false>
-__global__ void __launch_bounds__(ROW_NTH, ROW2048 ? 4 : 1) k_ssf_rows(const SsfArgs<S, T> a) {
+// Middle row pass of a grid of 2048-point rows (8 x 8 x 8 x 4), one row a
+// workgroup: the first inverse stage reads HBM; the last inverse stage, the two
+// pointwise half steps and the first forward stage run in registers
+// (fft_2048_turn: a thread's points are the elements tid + 256 s, its slots s of
+// ps and ns); the last forward stage writes HBM.  Held to 128 registers, so four
+// workgroups share a CU.  On a grid of 2048^2 points it takes 60 us (reservoir, double
+// precision; 56 us single), against 66 (60) in registers throughout
+// (k_ssf_row_regs, two workgroups a CU for its registers).  VALU issue is 26 us of it, HBM at the
+// rate of a large copy 45: the FFT stages, the pointwise part and the memory
+// phases overlap only across those four workgroups.
+template <typename S, typename T, bool DYN>
+__global__ void __launch_bounds__(ROW_NTH, 4) k_ssf_rows2048(const SsfArgs<S, T> a) {
     using C = cplx_t<T>;
-    constexpr int PPT = ROW_PTS / ROW_NTH;
+    static_assert(sizeof(T) == 8, "double-precision transforms");
+    constexpr int PPT = ROW_PTS / ROW_NTH, LN = ROW_LOG_PTS, NN = 1 << LN;
+    static_assert(PPT == 8, "a thread holds eight points of the row");
     __shared__ C buf_mem[lds_padded(ROW_PTS, NLS_SSF_ROW_PAD)];
     const Lds<T, NLS_SSF_ROW_PAD> buf{buf_mem};
-    const int logN = a.logN, N = 1 << logN;
-    const int logL = lines_per_wg(logN, ROW_LOG_PTS);
-    const int pts = 1 << (logL + logN);
-    const size_t base = (size_t)blockIdx.x << (logL + logN);    // rows are contiguous
-    T pp[PPT], nn[PPT];
-    if constexpr (ROW2048) {
-        static_assert(MODE == ROWS_MIDDLE && sizeof(T) == 8, "the 2048-point middle pass");
-        // one 2048-point row (8 x 8 x 8 x 4, compile-time sizes): the first
-        // inverse stage reads HBM; the last inverse stage, the two pointwise
-        // half steps and the first forward stage run in registers
-        // (fft_2048_turn: a thread's points are the elements tid + 256 s, its
-        // slots s of pp and nn); the last forward stage writes HBM -- six
-        // passes through LDS fewer and about half the barriers
-        constexpr int LN = ROW_LOG_PTS, NN = 1 << LN;
-        static_assert(PPT == 8, "a thread holds eight points of the row");
-        // the fields stay in the storage precision until used (exact
-        // conversion; single-precision storage then holds them in half the
-        // registers)
-        S ps[PPT], ns[PPT];
-#pragma unroll
-        for (int q = 0; q < PPT; ++q) {
-            const int idx = threadIdx.x + ROW_NTH * q;
-            ps[q] = a.P[base + idx];
-            ns[q] = DYN ? a.nres[base + idx] : (S)0;
-        }
-        auto lds_ld = [&](int, int e) { return buf[e]; };
-        auto lds_st = [&](int, int e, C v, int, int) { buf[e] = v; };
-        const C w8 = a.tw[NN >> 3];
-        fft_radix8_io<T, true, false, ROW_PTS, ROW_NTH, false, false>(
-            LN, 0, 0, a.tw, w8, [&](int, int e) { return widen<T, S>(a.psi[base + e]); }, lds_st);
-        __syncthreads();
-        fft_radix8_stage<T, true, false, ROW_PTS, ROW_NTH>(buf, LN, 0, NN, 1, 3, a.tw, w8);
-        fft_radix8_stage<T, true, false, ROW_PTS, ROW_NTH>(buf, LN, 0, NN, 1, 6, a.tw, w8);
-        fft_2048_turn<T, true, false, false, ROW_PTS, ROW_NTH>(
-            0, a.tw, w8, lds_ld,
-            [&](int, int e, int slot, C v) {
-                T nv = (T)ns[slot];
-                const T pv = (T)ps[slot];
-                pointwise_rk4<T, DYN>(a.c, a.inv_c11, pv, a.half_dt, v, nv);
-                pointwise_rk4<T, DYN>(a.c, a.inv_c11, pv, a.half_dt, v, nv);
-                // the reservoir is final here (the transforms act on psi only)
-                if (DYN) a.nres[base + e] = (S)nv;
-                return v;
-            },
-            lds_st);
-        __syncthreads();
-        fft_radix8_stage<T, false, false, ROW_PTS, ROW_NTH>(buf, LN, 0, NN, 1, 3, a.tw, w8);
-        fft_radix8_stage<T, false, false, ROW_PTS, ROW_NTH>(buf, LN, 0, NN, 1, 6, a.tw, w8);
-        fft_radix4_io<T, false, false, ROW_PTS, ROW_NTH, false>(
-            LN, 0, 9, a.tw, lds_ld, [&](int, int e, C v, int, int) { a.psi[base + e] = narrow<S, T>(v); });
-        return;
-    }
+    const size_t base = (size_t)blockIdx.x << LN;               // rows are contiguous
+    // the fields stay in the storage precision until used (exact
+    // conversion; single-precision storage then holds them in half the
+    // registers)
+    S ps[PPT], ns[PPT];
 #pragma unroll
     for (int q = 0; q < PPT; ++q) {
         const int idx = threadIdx.x + ROW_NTH * q;
-        pp[q] = 0; nn[q] = 0;
-        if (idx < pts) {
-            buf[idx] = widen<T, S>(a.psi[base + idx]);
-            pp[q] = (T)a.P[base + idx];
-            if (DYN) nn[q] = (T)a.nres[base + idx];
-        }
+        ps[q] = a.P[base + idx];
+        ns[q] = DYN ? a.nres[base + idx] : (S)0;
     }
+    auto lds_ld = [&](int, int e) { return buf[e]; };
+    auto lds_st = [&](int, int e, C v, int, int) { buf[e] = v; };
+    const C w8 = a.tw[NN >> 3];
+    fft_radix8_io<T, true, false, ROW_PTS, ROW_NTH, false, false>(
+        LN, 0, 0, a.tw, w8, [&](int, int e) { return widen<T, S>(a.psi[base + e]); }, lds_st);
     __syncthreads();
-    // a grid of 2048-point rows (one a workgroup) takes a copy of the
-    // transform with its sizes known at compile time: every stage's index
-    // arithmetic folds to constants (6% of the step at 2048^2)
-    if (MODE != ROWS_FIRST) {
-        if (logN == ROW_LOG_PTS) lds_fft<T, true, false, ROW_PTS, ROW_NTH>(buf, ROW_LOG_PTS, 0, ROW_PTS, 1, a.tw);
-        else lds_fft<T, true, false, ROW_PTS, ROW_NTH>(buf, logN, logL, N, 1, a.tw);
-    }
-#pragma unroll
-    for (int q = 0; q < PPT; ++q) {
-        const int idx = threadIdx.x + ROW_NTH * q;
-        if (idx < pts) {
-            C v = buf[idx];
-            T nv = nn[q];
-            pointwise_rk4<T, DYN>(a.c, a.inv_c11, pp[q], a.half_dt, v, nv);
-            if (MODE == ROWS_MIDDLE) pointwise_rk4<T, DYN>(a.c, a.inv_c11, pp[q], a.half_dt, v, nv);
-            buf[idx] = v;
-            nn[q] = nv;
-        }
-    }
+    fft_radix8_stage<T, true, false, ROW_PTS, ROW_NTH>(buf, LN, 0, NN, 1, 3, a.tw, w8);
+    fft_radix8_stage<T, true, false, ROW_PTS, ROW_NTH>(buf, LN, 0, NN, 1, 6, a.tw, w8);
+    fft_2048_turn<T, true, false, false, ROW_PTS, ROW_NTH>(
+        0, a.tw, w8, lds_ld,
+        [&](int, int e, int slot, C v) {
+            T nv = (T)ns[slot];
+            const T pv = (T)ps[slot];
+            pointwise_rk4<T, DYN>(a.c, a.inv_c11, pv, a.half_dt, v, nv);
+            pointwise_rk4<T, DYN>(a.c, a.inv_c11, pv, a.half_dt, v, nv);
+            // the reservoir is final here (the transforms act on psi only)
+            if (DYN) a.nres[base + e] = (S)nv;
+            return v;
+        },
+        lds_st);
     __syncthreads();
-    if (MODE != ROWS_LAST) {
-        if (logN == ROW_LOG_PTS) lds_fft<T, false, false, ROW_PTS, ROW_NTH>(buf, ROW_LOG_PTS, 0, ROW_PTS, 1, a.tw);
-        else lds_fft<T, false, false, ROW_PTS, ROW_NTH>(buf, logN, logL, N, 1, a.tw);
-    }
-#pragma unroll
-    for (int q = 0; q < PPT; ++q) {
-        const int idx = threadIdx.x + ROW_NTH * q;
-        if (idx < pts) {
-            a.psi[base + idx] = narrow<S, T>(buf[idx]);
-            if (DYN) a.nres[base + idx] = (S)nn[q];
-        }
-    }
-}
-
-// Column pass: min(2^LOG_L, n) adjacent columns per workgroup, LDS
-// [row][col].  Workgroups of one XCD take adjacent column blocks
-// (round-robin dispatch).
-template <typename S, typename T, bool COL2048 = false>
-__global__ void __launch_bounds__((ColShape<T, COL2048>::NTH)) k_ssf_cols(const SsfArgs<S, T> a, int nblocks,
-                                                                           int chunk) {
-    using C = cplx_t<T>;
-    using CS = ColShape<T, COL2048>;
-    constexpr int COL_PTS = CS::PTS, COL_NTH = CS::NTH;
-    constexpr int PPT = COL_PTS / COL_NTH;
-    static_assert(COL_PTS == 2048 << CS::LOG_L, "column block of 2048-point columns");
-    constexpr int PAD = COL2048 ? NLS_SSF_COL2048_PAD : NLS_SSF_COL_PAD;
-    __shared__ C buf_mem[lds_padded(COL_PTS, PAD)];
-    const Lds<T, PAD> buf{buf_mem};
-    const int b = blockIdx.x;
-    const int blk = (b & 7) * chunk + (b >> 3);
-    if (blk >= nblocks) return;
-    const int logN = a.logN, N = 1 << logN;
-    const int logL = CS::LOG_L < logN ? CS::LOG_L : logN;
-    const int L = 1 << logL, pts = L << logN;
-    const int col0 = blk << logL;
-    constexpr int LL = CS::LOG_L;
-    if constexpr (COL2048) {
-        static_assert(sizeof(T) == 8, "the 2048-point column pass");
-        // 2048-point columns (8 x 8 x 8 x 4, compile-time sizes): the first
-        // forward stage reads HBM, the last forward stage, the phase and the
-        // first inverse stage run in registers (fft_2048_turn), and the last
-        // inverse stage writes HBM -- six passes through LDS (reads and
-        // writes) fewer and half the barriers of load / transform / phase /
-        // transform / store
-        constexpr int LN = ROW_LOG_PTS, NN = 1 << LN, LW = 1 << LL;
-        auto lds_ld = [&](int l, int e) { return buf[l + e * LW]; };
-        auto lds_st = [&](int l, int e, C v, int, int) { buf[l + e * LW] = v; };
-        const C w8 = a.tw[NN >> 3];
-        fft_radix8_io<T, false, true, COL_PTS, COL_NTH, false, false>(
-            LN, LL, 0, a.tw, w8, [&](int l, int e) { return widen<T, S>(a.psi[(size_t)e * NN + col0 + l]); }, lds_st);
-        __syncthreads();
-        fft_radix8_stage<T, false, true, COL_PTS, COL_NTH>(buf, LN, LL, 1, LW, 3, a.tw, w8);
-        fft_radix8_stage<T, false, true, COL_PTS, COL_NTH>(buf, LN, LL, 1, LW, 6, a.tw, w8);
-        fft_2048_turn<T, false, true, true, COL_PTS, COL_NTH>(
-            LL, a.tw, w8, lds_ld, [&](int l, int e, int, C v) { return cmul<T>(v, cmul<T>(a.ph[e], a.ph[col0 + l])); },
-            lds_st);
-        __syncthreads();
-        fft_radix8_stage<T, true, true, COL_PTS, COL_NTH>(buf, LN, LL, 1, LW, 3, a.tw, w8);
-        fft_radix8_stage<T, true, true, COL_PTS, COL_NTH>(buf, LN, LL, 1, LW, 6, a.tw, w8);
-        fft_radix4_io<T, true, true, COL_PTS, COL_NTH, false>(
-            LN, LL, 9, a.tw, lds_ld,
-            [&](int l, int e, C v, int, int) { a.psi[(size_t)e * NN + col0 + l] = narrow<S, T>(v); });
-        return;
-    }
-#pragma unroll
-    for (int q = 0; q < PPT; ++q) {
-        const int idx = threadIdx.x + COL_NTH * q;
-        if (idx < pts) {
-            const int m = idx >> logL, cc = idx & (L - 1);
-            buf[idx] = widen<T, S>(a.psi[(size_t)m * N + col0 + cc]);
-        }
-    }
-    __syncthreads();
-    // 2048-point columns: the transform with compile-time sizes, as in the row pass
-    if (logN == ROW_LOG_PTS) lds_fft<T, false, true, COL_PTS, COL_NTH>(buf, ROW_LOG_PTS, LL, 1, 1 << LL, a.tw);
-    else lds_fft<T, false, true, COL_PTS, COL_NTH>(buf, logN, logL, 1, L, a.tw);
-#pragma unroll
-    for (int q = 0; q < PPT; ++q) {
-        const int idx = threadIdx.x + COL_NTH * q;
-        if (idx < pts) {
-            const int m = idx >> logL, cc = idx & (L - 1);
-            buf[idx] = cmul<T>(buf[idx], cmul<T>(a.ph[m], a.ph[col0 + cc]));
-        }
-    }
-    __syncthreads();
-    if (logN == ROW_LOG_PTS) lds_fft<T, true, true, COL_PTS, COL_NTH>(buf, ROW_LOG_PTS, LL, 1, 1 << LL, a.tw);
-    else lds_fft<T, true, true, COL_PTS, COL_NTH>(buf, logN, logL, 1, L, a.tw);
-#pragma unroll
-    for (int q = 0; q < PPT; ++q) {
-        const int idx = threadIdx.x + COL_NTH * q;
-        if (idx < pts) {
-            const int m = idx >> logL, cc = idx & (L - 1);
-            a.psi[(size_t)m * N + col0 + cc] = narrow<S, T>(buf[idx]);
-        }
-    }
-}
-
-// 1-D: one workgroup holds the whole line in LDS and runs every step; the
-// pumping and reservoir of the thread's points stay in registers.
-template <typename S, typename T, bool DYN>
-__global__ void __launch_bounds__(LineShape<T>::NTH) k_ssf_line(const SsfArgs<S, T> a) {
-    using C = cplx_t<T>;
-    constexpr int LINE_NTH = LineShape<T>::NTH;
-    constexpr int PPT = LINE_PTS / LINE_NTH;
-    __shared__ C buf_mem[lds_padded(LINE_PTS, NLS_SSF_LINE_PAD)];
-    const Lds<T, NLS_SSF_LINE_PAD> buf{buf_mem};
-    const int logN = a.logN, N = 1 << logN;
-    T pp[PPT], nn[PPT];
-    C ph[PPT];                                       // the phase of each point, for every step
-#pragma unroll
-    for (int q = 0; q < PPT; ++q) {
-        const int idx = threadIdx.x + LINE_NTH * q;
-        pp[q] = 0; nn[q] = 0; ph[q] = mk<T>(0, 0);
-        if (idx < N) {
-            ph[q] = a.ph[idx];
-            pp[q] = (T)a.P[idx];
-            if (DYN) nn[q] = (T)a.nres[idx];
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < PPT; ++q) {
-        const int idx = threadIdx.x + LINE_NTH * q;
-        if (idx < N) buf[idx] = widen<T, S>(a.psi[idx]);
-    }
-    for (int it = 0; it < a.iters; ++it) {
-        // each thread only touches its own points here, so no barrier is
-        // needed before the first FFT stage (which starts with one)
-#pragma unroll
-        for (int q = 0; q < PPT; ++q) {
-            const int idx = threadIdx.x + LINE_NTH * q;
-            if (idx < N) {
-                C v = buf[idx];
-                pointwise_rk4<T, DYN>(a.c, a.inv_c11, pp[q], a.half_dt, v, nn[q]);
-                buf[idx] = v;
-            }
-        }
-        __syncthreads();
-        lds_fft<T, false, false, LINE_PTS, LINE_NTH>(buf, logN, 0, N, 1, a.tw);
-#pragma unroll
-        for (int q = 0; q < PPT; ++q) {
-            const int idx = threadIdx.x + LINE_NTH * q;
-            if (idx < N) buf[idx] = cmul<T>(buf[idx], ph[q]);
-        }
-        __syncthreads();
-        lds_fft<T, true, false, LINE_PTS, LINE_NTH>(buf, logN, 0, N, 1, a.tw);
-#pragma unroll
-        for (int q = 0; q < PPT; ++q) {
-            const int idx = threadIdx.x + LINE_NTH * q;
-            if (idx < N) {
-                C v = buf[idx];
-                pointwise_rk4<T, DYN>(a.c, a.inv_c11, pp[q], a.half_dt, v, nn[q]);
-                buf[idx] = v;
-            }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int q = 0; q < PPT; ++q) {
-        const int idx = threadIdx.x + LINE_NTH * q;
-        if (idx < N) {
-            a.psi[idx] = narrow<S, T>(buf[idx]);
-            if (DYN) a.nres[idx] = (S)nn[q];
-        }
-    }
+    fft_radix8_stage<T, false, false, ROW_PTS, ROW_NTH>(buf, LN, 0, NN, 1, 3, a.tw, w8);
+    fft_radix8_stage<T, false, false, ROW_PTS, ROW_NTH>(buf, LN, 0, NN, 1, 6, a.tw, w8);
+    fft_radix4_io<T, false, false, ROW_PTS, ROW_NTH, false>(
+        LN, 0, 9, a.tw, lds_ld, [&](int, int e, C v, int, int) { a.psi[base + e] = narrow<S, T>(v); });
 }
 
 // Radix-8 butterfly of Stockham stage logNs of a 2^LN-point transform on
@@ -842,72 +615,292 @@ __device__ __forceinline__ void bfly8(cplx_t<T> x[8], int j, int logNs, int LN, 
     x[7] = mk<T>(e3.x - o3.x, e3.y - o3.y);
 }
 
-// 1-D, n = 4096 = 8^4 (the longest line): the line's values stay in
-// registers.  Every radix-8 stage of this transform reads the elements
-// j + 512 r of thread j's butterfly, and the last stage writes them back to
-// the same elements, so a thread's eight points (j + 512 s) are its inputs of
-// the first stage and its outputs of the last: the pointwise half steps and
-// the phase run in registers, and only the three stage-to-stage exchanges of
-// a transform go through LDS, alternating between two buffers (one barrier
-// each instead of two).  Six barriers a step instead of about nineteen.
-template <typename S, typename T, bool DYN>
-__global__ void __launch_bounds__(512) k_ssf_line4096(const SsfArgs<S, T> a) {
+// Radix-4 butterfly of Stockham stage logNs on the inputs x[0..3] (elements
+// j + r 2^(LN-2)), in place, as bfly8: x[r] becomes the output element d + r Ns,
+// d = ((j >> logNs) << (logNs + 2)) + (j & (Ns - 1)).
+template <typename T, bool INV, bool TW>
+__device__ __forceinline__ void bfly4(cplx_t<T> &x0, cplx_t<T> &x1, cplx_t<T> &x2, cplx_t<T> &x3, int j, int logNs,
+                                      int LN, const cplx_t<T> *tw) {
     using C = cplx_t<T>;
-    constexpr int LN = 12, NN = 1 << LN, NTH = NN / 8;
-    static_assert(sizeof(T) == 8, "double-precision transforms");
-    __shared__ C mem[2][lds_padded(NN, NLS_SSF_LINE_PAD)];
-    const Lds<T, NLS_SSF_LINE_PAD> A{mem[0]}, B{mem[1]};
-    const int j = threadIdx.x;
-    C x[8], ph[8];
-    T pp[8], nn[8];
+    if (TW) {
+        const int k = j & ((1 << logNs) - 1), sh = LN - logNs - 2;
+        C w1 = tw[k << sh], w2 = tw[(2 * k) << sh], w3 = tw[(3 * k) << sh];
+        if (INV) { w1.y = -w1.y; w2.y = -w2.y; w3.y = -w3.y; }
+        x1 = cmul<T>(x1, w1);
+        x2 = cmul<T>(x2, w2);
+        x3 = cmul<T>(x3, w3);
+    }
+    dft4<T, INV>(x0, x1, x2, x3);
+}
+
+// Radix-16 butterfly, as bfly8 (elements j + r 2^(LN-4), outputs d + r Ns, d =
+// ((j >> logNs) << (logNs + 4)) + (j & (Ns - 1))): four 4-point DFTs over the
+// inputs of equal remainder mod 4, the sixteenth roots of unity, four more.
+template <typename T, bool INV, bool TW>
+__device__ __forceinline__ void bfly16(cplx_t<T> x[16], int j, int logNs, int LN, const cplx_t<T> *tw) {
+    using C = cplx_t<T>;
+    if (TW) {
+        const int k = j & ((1 << logNs) - 1), sh = LN - logNs - 4;
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-        const int e = j + NTH * r;
+        for (int r = 1; r < 16; ++r) {
+            C wr = tw[(r * k) << sh];
+            if (INV) wr.y = -wr.y;
+            x[r] = cmul<T>(x[r], wr);
+        }
+    }
+    const T c1 = (T)0.92387953251128675613, s1 = (T)0.38268343236508977173, h = (T)0.70710678118654752440;
+    const T wc[4] = {1, c1, h, s1}, ws[4] = {0, s1, h, c1};
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        dft4<T, INV>(x[m], x[4 + m], x[8 + m], x[12 + m]);
+        // slot 4 k + m times exp(-+ 2 pi i k m / 16)
+#pragma unroll
+        for (int k = 1; k < 4; ++k) {
+            const int e = k * m, f = e < 4 ? e : e == 4 ? 0 : e == 6 ? 2 : 1;      // quarter turns taken out below
+            C v = x[4 * k + m];
+            if (e != 0 && e != 4) v = cmul<T>(v, mk<T>(wc[f], INV ? ws[f] : -ws[f]));
+            if (e == 4 || e == 6) v = INV ? mk<T>(-v.y, v.x) : mk<T>(v.y, -v.x);    // w16^4 = -i
+            if (e == 9) v = mk<T>(-v.x, -v.y);                                      // w16^9 = -w16
+            x[4 * k + m] = v;
+        }
+    }
+    C y[16];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        dft4<T, INV>(x[4 * k], x[4 * k + 1], x[4 * k + 2], x[4 * k + 3]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) y[k + 4 * q] = x[4 * k + q];
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) x[r] = y[r];
+}
+
+// Transform of a 2^LN-point line (LN = 4 .. 12) whose values stay in
+// registers: thread j of the line's 2^LN / PT holds the PT (4, 8 or 16)
+// elements j + (2^LN / PT) s in x[s].  Those are the inputs of its radix-PT
+// butterfly of every stage, and the inputs and outputs of its butterflies of
+// the last one, whether that is radix 8, 4 (PT / 4 butterflies) or 2 (PT / 2).
+// So a transform starts and ends in the thread's own elements, and only the
+// exchanges between stages go through LDS: ex(logNs) writes the outputs of
+// stage logNs (element d + r Ns from x[r]) and reads the thread's elements
+// back.  Stages: radix PT, and one of a smaller radix for the bits left over.
+__host__ __device__ constexpr int log2_pt(int PT) { return PT == 16 ? 4 : PT == 8 ? 3 : 2; }
+template <typename T, bool INV, int LN, int PT, typename EX>
+__device__ __forceinline__ void fft_regs(cplx_t<T> x[PT], int j, const cplx_t<T> *tw, EX ex) {
+    using C = cplx_t<T>;
+    static_assert(LN >= 4 && LN <= 12 && (PT == 4 || PT == 8 || PT == 16), "line length and points per thread");
+    constexpr int LP = log2_pt(PT), Q = 1 << (LN - LP), REM = LN % LP, SP = LN / LP;
+    C w8;
+    if constexpr (PT >= 8) w8 = tw[(1 << LN) >> 3];
+    auto stage = [&](auto first, int logNs) {
+        if constexpr (PT == 16) bfly16<T, INV, !decltype(first)::value>(x, j, logNs, LN, tw);
+        else if constexpr (PT == 8) bfly8<T, INV, !decltype(first)::value>(x, j, logNs, LN, tw, w8);
+        else bfly4<T, INV, !decltype(first)::value>(x[0], x[1], x[2], x[3], j, logNs, LN, tw);
+    };
+    stage(std::true_type(), 0);
+#pragma unroll
+    for (int s = 1; s < SP; ++s) {
+        ex(LP * (s - 1));
+        stage(std::false_type(), LP * s);
+    }
+    if constexpr (REM > 0) ex(LP * (SP - 1));
+    if constexpr (REM == 3) {
+#pragma unroll
+        for (int q = 0; q < PT / 8; ++q) {
+            C y[8];
+#pragma unroll
+            for (int r = 0; r < 8; ++r) y[r] = x[q + PT / 8 * r];
+            bfly8<T, INV, true>(y, j + Q * q, LN - 3, LN, tw, w8);
+#pragma unroll
+            for (int r = 0; r < 8; ++r) x[q + PT / 8 * r] = y[r];
+        }
+    } else if constexpr (REM == 2) {
+        constexpr int M = PT / 4;
+#pragma unroll
+        for (int q = 0; q < M; ++q)
+            bfly4<T, INV, true>(x[q], x[q + M], x[q + 2 * M], x[q + 3 * M], j + Q * q, LN - 2, LN, tw);
+    } else if constexpr (REM == 1) {
+        constexpr int M = PT / 2;
+#pragma unroll
+        for (int q = 0; q < M; ++q) {
+            C w = tw[j + Q * q];
+            if (INV) w.y = -w.y;
+            const C v = cmul<T>(x[q + M], w), u = x[q];
+            x[q] = mk<T>(u.x + v.x, u.y + v.y);
+            x[q + M] = mk<T>(u.x - v.x, u.y - v.y);
+        }
+    }
+}
+
+// Order the wave's LDS accesses around this point for the compiler (the
+// hardware runs one wave's LDS operations in order; no instruction).
+__device__ __forceinline__ void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Lines in registers, L of them in a workgroup of at least one wave: LDS for
+// the exchanges of fft_regs.  One wave: its LDS operations run in order, one
+// buffer and no barrier.  Several: two buffers in turn and one barrier each (a
+// buffer is written again only after the next exchange's barrier, which every
+// thread reaches after its reads); NBUF = 1: one buffer, two barriers, for half
+// the LDS.  COLS: the lines interleaved (element e of line l at e L + l), else
+// one behind the other.
+template <typename T, int LN, int PT, int L, int PAD, bool COLS, int NBUF = 2> struct LineLds {
+    static constexpr int LP = log2_pt(PT), Q = 1 << (LN - LP), NTH = L * Q;
+    static constexpr bool WAVE = NTH <= 64;
+    static constexpr int EX = (LN + LP - 1) / LP - 1;      // exchanges of a transform
+    static constexpr int PTS = lds_padded(L << LN, PAD);
+    static constexpr int MEM = WAVE ? PTS : NBUF * PTS;
+    // the mth exchange since the start is at buffer (first + m) & 1
+    static __device__ __forceinline__ auto exchange(cplx_t<T> *mem, cplx_t<T> x[PT], int j, int l, int first) {
+        return [=](int logNs) {
+            const int Ns = 1 << logNs, d = ((j >> logNs) << (logNs + LP)) + (j & (Ns - 1));
+            const int es = COLS ? L : 1, l0 = COLS ? l : l << LN;
+            const Lds<T, PAD> B{mem + (WAVE || NBUF == 1 ? 0 : ((first + logNs / LP) & 1) * PTS)};
+            if (WAVE) wave_order();
+            else if (NBUF == 1) __syncthreads();
+#pragma unroll
+            for (int r = 0; r < PT; ++r) B[l0 + (d + r * Ns) * es] = x[r];
+            if (WAVE) wave_order();
+            else __syncthreads();
+#pragma unroll
+            for (int r = 0; r < PT; ++r) x[r] = B[l0 + (j + Q * r) * es];
+        };
+    }
+};
+
+// Points per thread, lines per workgroup and LDS buffers of the passes in
+// registers, by the line's length; double precision (f32: single-precision
+// storage), us a step or a pass.  Few points a thread spread the pointwise part,
+// which a small grid or a single line leaves to few waves, but cost more
+// exchanges and narrower butterflies.
+// - 1-D lines, 4 points against 8: n = 256 2.2 / 3.4 a step, 1024 4.3 / 6.2,
+//   2048 8.3 / 7.5, 4096 18.0 / 14.6.
+// - Rows, 4 against 8: a step of 64^2 6.9 / 9.2, 256^2 9.0 / 10.1; the pass at
+//   512^2 7.2 / 6.6, without a reservoir (the stationary density divides) 8.4 /
+//   9.6; at 1024^2 19.8 / 19.0.  2048-point rows take k_ssf_rows2048 between the
+//   first and the last pass, which are in registers with one buffer, four
+//   workgroups a CU.
+// - Columns: a pass moves 32 bytes a point; the short ones are latency, one
+//   column of 4 points a thread (a step of 64^2: 7.9, two columns 8.5, two of 8
+//   points 8.7), 512^2 two of 8 points (5.3; of 4 points 5.8, of 16 6.5).
+//   From 1024 on 16 points a thread, an exchange fewer a transform: the pass at 1024^2
+//   four columns 17.6 against 19.1 of 8 points (f32 13.8 / 15.5), at 2048^2 two
+//   columns 43.6, four 45.6 (f32, the same 32 bytes a row with four: 41.1 / 38.6),
+//   four of 8 points in LDS 48.2 (43.9).
+constexpr int line_pt(int LN) { return LN <= 10 ? 4 : 8; }
+constexpr int row_pt(int LN, bool dyn) { return LN <= (dyn ? 8 : 9) ? 4 : 8; }
+constexpr int row_bufs(int LN) { return LN <= 10 ? 2 : 1; }
+constexpr int col_pt(int LN) { return LN <= 8 ? 4 : LN == 9 ? 8 : 16; }
+constexpr int col_lines(int LN, bool f64) { return LN <= 8 ? 1 : LN == 9 || (LN == 11 && f64) ? 2 : 4; }
+constexpr int col_bufs(int LN) { return LN <= 9 ? 2 : 1; }
+
+// 1-D: one workgroup runs every step of a line in registers (fft_regs): the
+// pointwise half steps and the phase act on the thread's own points.  The
+// threads of a line shorter than a wave's points hold it several times over.
+// Against the line in LDS, us a step: n = 16 2.3 -> 1.4, 256 3.6 -> 2.2, 1024
+// 6.3 -> 4.2, 2048 10.0 -> 7.5 (4096 was in registers: 14.6).  One CU's VALU issue
+// bounds the longest lines (8 us of 14.6), barriers and latency the rest.
+template <int LN, int PT> constexpr int line_threads = (1 << LN) / PT < 64 ? 64 : (1 << LN) / PT;
+template <typename S, typename T, bool DYN, int LN, int PT>
+__global__ void __launch_bounds__((line_threads<LN, PT>)) k_ssf_line(const SsfArgs<S, T> a) {
+    using C = cplx_t<T>;
+    using LL = LineLds<T, LN, PT, 1, NLS_SSF_LINE_PAD, false>;
+    constexpr int Q = LL::Q;
+    __shared__ C mem[LL::MEM];
+    const int j = threadIdx.x & (Q - 1);
+    C x[PT], ph[PT];
+    T pp[PT], nn[PT];
+#pragma unroll
+    for (int r = 0; r < PT; ++r) {
+        const int e = j + Q * r;
         x[r] = widen<T, S>(a.psi[e]);
         ph[r] = a.ph[e];
         pp[r] = (T)a.P[e];
         nn[r] = DYN ? (T)a.nres[e] : (T)0;
     }
-    const C w8 = a.tw[NN >> 3];
-    // outputs of stage logNs to buffer L (elements d + r Ns), then the
-    // thread's inputs of the next stage (elements j + 512 r)
-    auto exchange = [&](const Lds<T, NLS_SSF_LINE_PAD> &L, int logNs) {
-        const int Ns = 1 << logNs;
-        const int d = ((j >> logNs) << (logNs + 3)) + (j & (Ns - 1));
-#pragma unroll
-        for (int r = 0; r < 8; ++r) L[d + r * Ns] = x[r];
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < 8; ++r) x[r] = L[j + NTH * r];
-    };
     for (int it = 0; it < a.iters; ++it) {
 #pragma unroll
-        for (int r = 0; r < 8; ++r) pointwise_rk4<T, DYN>(a.c, a.inv_c11, pp[r], a.half_dt, x[r], nn[r]);
-        bfly8<T, false, false>(x, j, 0, LN, a.tw, w8);
-        exchange(A, 0);
-        bfly8<T, false, true>(x, j, 3, LN, a.tw, w8);
-        exchange(B, 3);
-        bfly8<T, false, true>(x, j, 6, LN, a.tw, w8);
-        exchange(A, 6);
-        bfly8<T, false, true>(x, j, 9, LN, a.tw, w8);     // outputs j + 512 r: the thread's own points
+        for (int r = 0; r < PT; ++r) pointwise_rk4<T, DYN>(a.c, a.inv_c11, pp[r], a.half_dt, x[r], nn[r]);
+        fft_regs<T, false, LN, PT>(x, j, a.tw, LL::exchange(mem, x, j, 0, 0));
 #pragma unroll
-        for (int r = 0; r < 8; ++r) x[r] = cmul<T>(x[r], ph[r]);
-        bfly8<T, true, false>(x, j, 0, LN, a.tw, w8);
-        exchange(B, 0);
-        bfly8<T, true, true>(x, j, 3, LN, a.tw, w8);
-        exchange(A, 3);
-        bfly8<T, true, true>(x, j, 6, LN, a.tw, w8);
-        exchange(B, 6);
-        bfly8<T, true, true>(x, j, 9, LN, a.tw, w8);
+        for (int r = 0; r < PT; ++r) x[r] = cmul<T>(x[r], ph[r]);
+        fft_regs<T, true, LN, PT>(x, j, a.tw, LL::exchange(mem, x, j, 0, LL::EX));
 #pragma unroll
-        for (int r = 0; r < 8; ++r) pointwise_rk4<T, DYN>(a.c, a.inv_c11, pp[r], a.half_dt, x[r], nn[r]);
+        for (int r = 0; r < PT; ++r) pointwise_rk4<T, DYN>(a.c, a.inv_c11, pp[r], a.half_dt, x[r], nn[r]);
     }
+    if (threadIdx.x >= Q) return;                    // a copy of a short line
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-        const int e = j + NTH * r;
+    for (int r = 0; r < PT; ++r) {
+        const int e = j + Q * r;
         a.psi[e] = narrow<S, T>(x[r]);
         if (DYN) a.nres[e] = (S)nn[r];
     }
+}
+
+// Row pass: rows in registers (fft_regs), as many as fill a wave or one of
+// several waves a workgroup; the points' pumping and reservoir are the thread's
+// own.  Against whole rows in LDS, 2048 points a workgroup: a step of 64^2 16.6
+// -> 6.6 us, 512^2 22.9 -> 13.2, 1024^2 42.0 -> 29.1 (single-precision storage,
+// both passes), since 512 rows were 128 workgroups, half the CUs, and every
+// stage cost two barriers.  Up to 512^2 a pass is latency: a wave or two a
+// SIMD run six stages and 24 to 64 evaluations of the pointwise part.
+template <typename S, typename T, bool DYN, int MODE, int LN, int PT>
+__global__ void __launch_bounds__((line_threads<LN, PT>)) k_ssf_row_regs(const SsfArgs<S, T> a) {
+    using C = cplx_t<T>;
+    constexpr int Q = (1 << LN) / PT, L = line_threads<LN, PT> / Q;
+    using LL = LineLds<T, LN, PT, L, NLS_SSF_ROW_PAD, false, row_bufs(LN)>;
+    __shared__ C mem[LL::MEM];
+    const int j = threadIdx.x & (Q - 1), l = threadIdx.x / Q;
+    const size_t base = ((size_t)blockIdx.x * L + l) << LN;
+    C x[PT];
+    T pp[PT], nn[PT];
+#pragma unroll
+    for (int r = 0; r < PT; ++r) {
+        const size_t e = base + j + Q * r;
+        x[r] = widen<T, S>(a.psi[e]);
+        pp[r] = (T)a.P[e];
+        nn[r] = DYN ? (T)a.nres[e] : (T)0;
+    }
+    if (MODE != ROWS_FIRST) fft_regs<T, true, LN, PT>(x, j, a.tw, LL::exchange(mem, x, j, l, 0));
+#pragma unroll
+    for (int r = 0; r < PT; ++r) {
+        pointwise_rk4<T, DYN>(a.c, a.inv_c11, pp[r], a.half_dt, x[r], nn[r]);
+        if (MODE == ROWS_MIDDLE) pointwise_rk4<T, DYN>(a.c, a.inv_c11, pp[r], a.half_dt, x[r], nn[r]);
+        if (DYN) a.nres[base + j + Q * r] = (S)nn[r];
+    }
+    if (MODE != ROWS_LAST) fft_regs<T, false, LN, PT>(x, j, a.tw, LL::exchange(mem, x, j, l, LL::EX));
+#pragma unroll
+    for (int r = 0; r < PT; ++r) a.psi[base + j + Q * r] = narrow<S, T>(x[r]);
+}
+
+// Column pass: L adjacent columns per workgroup, in registers.  Workgroups of
+// one XCD take adjacent column blocks (round-robin dispatch), so the lines of
+// memory that blocks share are in its L2.  At 2048^2 VALU issue is 10 us of the
+// 44 and HBM at the rate of a large copy 26.
+template <typename S, typename T, int LN, int PT, int L>
+__global__ void __launch_bounds__(((L << LN) / PT)) k_ssf_col_regs(const SsfArgs<S, T> a, int chunk) {
+    using C = cplx_t<T>;
+    using LL = LineLds<T, LN, PT, L, NLS_SSF_COL_PAD, true, col_bufs(LN)>;
+    constexpr int NN = 1 << LN, Q = LL::Q;
+    __shared__ C mem[LL::MEM];
+    const int blk = (blockIdx.x & 7) * chunk + (blockIdx.x >> 3);
+    if (blk >= NN / L) return;
+    const int l = threadIdx.x % L, j = threadIdx.x / L, col = blk * L + l;
+    C x[PT], ph[PT];
+#pragma unroll
+    for (int r = 0; r < PT; ++r) {
+        x[r] = widen<T, S>(a.psi[(size_t)(j + Q * r) * NN + col]);
+        ph[r] = a.ph[j + Q * r];
+    }
+    const C phc = a.ph[col];
+    fft_regs<T, false, LN, PT>(x, j, a.tw, LL::exchange(mem, x, j, l, 0));
+#pragma unroll
+    for (int r = 0; r < PT; ++r) x[r] = cmul<T>(x[r], cmul<T>(ph[r], phc));
+    fft_regs<T, true, LN, PT>(x, j, a.tw, LL::exchange(mem, x, j, l, LL::EX));
+#pragma unroll
+    for (int r = 0; r < PT; ++r) a.psi[(size_t)(j + Q * r) * NN + col] = narrow<S, T>(x[r]);
 }
 
 // The unit complex number (c, s) in T.  In single precision the rounded
@@ -957,6 +950,25 @@ static int log2_exact(int n) {
     return (1 << l) == n ? l : -1;
 }
 
+// A 2-D grid of 2^LN points a side.
+template <typename S, typename T, bool DYN, int LN>
+static int ssf_run_2d(const SsfArgs<S, T> &a, int iters, hipStream_t s) {
+    constexpr int N = 1 << LN, RP = row_pt(LN, DYN), RT = line_threads<LN, RP>;
+    constexpr int CP = col_pt(LN), L = col_lines(LN, sizeof(S) == 8), chunk = (N / L + 7) / 8;
+    const dim3 rows(N / (RP * RT / N)), rth(RT), cols(8 * chunk), cth(L * N / CP);
+    hipLaunchKernelGGL((k_ssf_row_regs<S, T, DYN, ROWS_FIRST, LN, RP>), rows, rth, 0, s, a);
+    for (int it = 0; it < iters; ++it) {
+        hipLaunchKernelGGL((k_ssf_col_regs<S, T, LN, CP, L>), cols, cth, 0, s, a, chunk);
+        if (it + 1 == iters)
+            hipLaunchKernelGGL((k_ssf_row_regs<S, T, DYN, ROWS_LAST, LN, RP>), rows, rth, 0, s, a);
+        else if constexpr (LN == ROW_LOG_PTS)
+            hipLaunchKernelGGL((k_ssf_rows2048<S, T, DYN>), dim3(N), dim3(ROW_NTH), 0, s, a);
+        else
+            hipLaunchKernelGGL((k_ssf_row_regs<S, T, DYN, ROWS_MIDDLE, LN, RP>), rows, rth, 0, s, a);
+    }
+    return hip_check(hipGetLastError(), "ssf launch");
+}
+
 template <typename S, bool DYN>
 static int ssf_run(const nls_problem *p, int iters, const S *P, cplx_t<S> *psi, S *nres, char *ws, hipStream_t s) {
     using T = double;                 // arithmetic, LDS and tables
@@ -975,33 +987,29 @@ static int ssf_run(const nls_problem *p, int iters, const S *P, cplx_t<S> *psi, 
     a.psi = psi; a.nres = nres; a.P = P; a.tw = tw; a.ph = ph;
     if (p->dim == 1) {
         a.iters = iters;
-        if (logN == 12) hipLaunchKernelGGL((k_ssf_line4096<S, T, DYN>), dim3(1), dim3(512), 0, s, a);
-        else hipLaunchKernelGGL((k_ssf_line<S, T, DYN>), dim3(1), dim3(LineShape<T>::NTH), 0, s, a);
+        switch (logN) {
+#define NLS_CASE(LN)                                                                                       \
+    case LN:                                                                                               \
+        hipLaunchKernelGGL((k_ssf_line<S, T, DYN, LN, line_pt(LN)>), dim3(1),                              \
+                           dim3(line_threads<LN, line_pt(LN)>), 0, s, a);                                  \
         return hip_check(hipGetLastError(), "ssf line launch");
-    }
-    const int rblocks = N >> lines_per_wg(logN, ROW_LOG_PTS);
-    const bool wide = logN == ROW_LOG_PTS;
-    const int clog = wide ? ColShape<T, true>::LOG_L : ColShape<T>::LOG_L;
-    const int cblocks = N >> (clog < logN ? clog : logN);
-    const int chunk = (cblocks + 7) / 8;
-    hipLaunchKernelGGL((k_ssf_rows<S, T, DYN, ROWS_FIRST>), dim3(rblocks), dim3(ROW_NTH), 0, s, a);
-    for (int it = 0; it < iters; ++it) {
-        if (wide)
-            hipLaunchKernelGGL((k_ssf_cols<S, T, true>), dim3(8 * chunk), dim3(ColShape<T, true>::NTH), 0, s, a,
-                               cblocks, chunk);
-        else
-            hipLaunchKernelGGL((k_ssf_cols<S, T>), dim3(8 * chunk), dim3(ColShape<T>::NTH), 0, s, a, cblocks, chunk);
-        if (it + 1 < iters)
-        {
-            if (logN == ROW_LOG_PTS)
-                hipLaunchKernelGGL((k_ssf_rows<S, T, DYN, ROWS_MIDDLE, true>), dim3(rblocks), dim3(ROW_NTH), 0, s, a);
-            else
-                hipLaunchKernelGGL((k_ssf_rows<S, T, DYN, ROWS_MIDDLE>), dim3(rblocks), dim3(ROW_NTH), 0, s, a);
+            NLS_CASE(4) NLS_CASE(5) NLS_CASE(6) NLS_CASE(7) NLS_CASE(8)
+            NLS_CASE(9) NLS_CASE(10) NLS_CASE(11) NLS_CASE(12)
+#undef NLS_CASE
         }
-        else
-            hipLaunchKernelGGL((k_ssf_rows<S, T, DYN, ROWS_LAST>), dim3(rblocks), dim3(ROW_NTH), 0, s, a);
+    } else {
+        switch (logN) {
+        case 4: return ssf_run_2d<S, T, DYN, 4>(a, iters, s);
+        case 5: return ssf_run_2d<S, T, DYN, 5>(a, iters, s);
+        case 6: return ssf_run_2d<S, T, DYN, 6>(a, iters, s);
+        case 7: return ssf_run_2d<S, T, DYN, 7>(a, iters, s);
+        case 8: return ssf_run_2d<S, T, DYN, 8>(a, iters, s);
+        case 9: return ssf_run_2d<S, T, DYN, 9>(a, iters, s);
+        case 10: return ssf_run_2d<S, T, DYN, 10>(a, iters, s);
+        case 11: return ssf_run_2d<S, T, DYN, 11>(a, iters, s);
+        }
     }
-    return hip_check(hipGetLastError(), "ssf launch");
+    return fail(NLS_EUNSUPPORTED, "no split-step kernel for %d points a side", N);
 }
 
 // ---------------------------------------------------------------------------
@@ -1066,17 +1074,17 @@ __global__ void __launch_bounds__(ROW_NTH) k_ssf_kin_rows(const cplx_t<S> *psi, 
     fixed_block_sum<ROW_NTH>((double *)buf_mem, v, part + blockIdx.x);
 }
 
+constexpr int COL_LOG_L = 1, COL_PTS = 4096, COL_NTH = 512;      // two columns per workgroup
 template <typename S>
-__global__ void __launch_bounds__(ColShape<double>::NTH) k_ssf_kin_cols(const cplx_t<S> *psi, int logN,
+__global__ void __launch_bounds__(COL_NTH) k_ssf_kin_cols(const cplx_t<S> *psi, int logN,
                                                                          const cplx_t<double> *tw, double k0,
                                                                          double *part) {
     using C = cplx_t<double>;
-    constexpr int COL_PTS = ColShape<double>::PTS, COL_NTH = ColShape<double>::NTH;
     constexpr int PPT = COL_PTS / COL_NTH;
     __shared__ C buf_mem[lds_padded(COL_PTS, NLS_SSF_COL_PAD)];
     const Lds<double, NLS_SSF_COL_PAD> buf{buf_mem};
     const int N = 1 << logN;
-    const int logL = ColShape<double>::LOG_L < logN ? ColShape<double>::LOG_L : logN;
+    const int logL = COL_LOG_L < logN ? COL_LOG_L : logN;
     const int L = 1 << logL, pts = L << logN;
     const int col0 = blockIdx.x << logL;
 #pragma unroll
@@ -1097,12 +1105,12 @@ __global__ void __launch_bounds__(ColShape<double>::NTH) k_ssf_kin_cols(const cp
 }
 
 // 1-D: one workgroup, the whole line (n <= 4096)
+constexpr int LINE_PTS = 4096, LINE_NTH = 512;
 template <typename S>
-__global__ void __launch_bounds__(LineShape<double>::NTH) k_ssf_kin_line(const cplx_t<S> *psi, int logN,
+__global__ void __launch_bounds__(LINE_NTH) k_ssf_kin_line(const cplx_t<S> *psi, int logN,
                                                                           const cplx_t<double> *tw, double k0,
                                                                           double *part) {
     using C = cplx_t<double>;
-    constexpr int LINE_NTH = LineShape<double>::NTH;
     constexpr int PPT = LINE_PTS / LINE_NTH;
     __shared__ C buf_mem[lds_padded(LINE_PTS, NLS_SSF_LINE_PAD)];
     const Lds<double, NLS_SSF_LINE_PAD> buf{buf_mem};
@@ -1152,23 +1160,23 @@ int ssf_kinetic(const nls_problem *p, const void *psi, void *scratch, double *de
     int nb;
     if (p->dim == 1) {
         nb = 1;
-        if (f64) hipLaunchKernelGGL(k_ssf_kin_line<double>, dim3(1), dim3(LineShape<double>::NTH), 0, s,
+        if (f64) hipLaunchKernelGGL(k_ssf_kin_line<double>, dim3(1), dim3(LINE_NTH), 0, s,
                                     (const double2 *)psi, logN, tw, k0, part);
-        else hipLaunchKernelGGL(k_ssf_kin_line<float>, dim3(1), dim3(LineShape<double>::NTH), 0, s,
+        else hipLaunchKernelGGL(k_ssf_kin_line<float>, dim3(1), dim3(LINE_NTH), 0, s,
                                 (const float2 *)psi, logN, tw, k0, part);
     } else {
         const int rblocks = N >> lines_per_wg(logN, ROW_LOG_PTS);
-        const int cblocks = N >> (ColShape<double>::LOG_L < logN ? ColShape<double>::LOG_L : logN);
+        const int cblocks = N >> (COL_LOG_L < logN ? COL_LOG_L : logN);
         nb = rblocks + cblocks;
         if (f64) {
             hipLaunchKernelGGL(k_ssf_kin_rows<double>, dim3(rblocks), dim3(ROW_NTH), 0, s, (const double2 *)psi,
                                logN, tw, k0, part);
-            hipLaunchKernelGGL(k_ssf_kin_cols<double>, dim3(cblocks), dim3(ColShape<double>::NTH), 0, s,
+            hipLaunchKernelGGL(k_ssf_kin_cols<double>, dim3(cblocks), dim3(COL_NTH), 0, s,
                                (const double2 *)psi, logN, tw, k0, part + rblocks);
         } else {
             hipLaunchKernelGGL(k_ssf_kin_rows<float>, dim3(rblocks), dim3(ROW_NTH), 0, s, (const float2 *)psi,
                                logN, tw, k0, part);
-            hipLaunchKernelGGL(k_ssf_kin_cols<float>, dim3(cblocks), dim3(ColShape<double>::NTH), 0, s,
+            hipLaunchKernelGGL(k_ssf_kin_cols<float>, dim3(cblocks), dim3(COL_NTH), 0, s,
                                (const float2 *)psi, logN, tw, k0, part + rblocks);
         }
     }
