@@ -183,9 +183,11 @@ template <typename T> struct FusedArgs {
 // sized for.
 //
 // FORM, chosen per launch by fused_form():
-//  - FORM_TALL: 64 x 32 tiles of 1024 threads (64 x 16 at order 7), for
-//    launches of several rounds, where the tall tile's smaller halo per
-//    output point pays, or whose tall tiles fit one per compute unit.
+//  - FORM_TALL: 64 x 32 tiles of 1024 threads (order 7: 64 x 24 tiles of 768
+//    threads), for launches of several rounds, where the tall tile's smaller
+//    halo per output point pays, or whose tall tiles fit one per compute unit.
+//    Single precision of order 5 runs the pair kernel, double precision of
+//    order 5 and order 7 the group kernel, order 3 this one.
 //  - FORM_SHORT: 64 x 16 tiles of 1024 threads, for launches with no more
 //    such tiles than the device has compute units (a lone grid, a few small
 //    members): the step is then one workgroup's critical path, which grows
@@ -211,14 +213,14 @@ enum { FORM_TALL = 0, FORM_SHORT = 1, FORM_HALF = 2, FORM_TALL512 = 3 };
 template <typename T, int ORDER, int FORM> struct FusedTile;
 template <int ORDER, int FORM> struct FusedTile<float, ORDER, FORM> {
     static_assert(FORM != FORM_HALF, "single precision has no half-size form");
-    static constexpr int TY = ORDER == 7 || FORM == FORM_SHORT ? 16 : 32;
+    static constexpr int TY = FORM == FORM_SHORT ? 16 : 32;
     static constexpr int NT = FORM == FORM_TALL512 ? 512 : 1024;
     static constexpr bool DB = true;
     static constexpr int WAVES = FORM == FORM_TALL512 ? 4 : 8;
 };
 template <int ORDER, int FORM> struct FusedTile<double, ORDER, FORM> {
     static constexpr bool HALF = FORM == FORM_HALF;
-    static constexpr int TY = ORDER == 7 || FORM != FORM_TALL ? 16 : 32;
+    static constexpr int TY = FORM != FORM_TALL ? 16 : 32;
     static constexpr int NT = HALF ? 512 : 1024;
     static constexpr bool DB = !HALF;
     static constexpr int WAVES = 4;
@@ -228,7 +230,8 @@ template <int ORDER, int FORM> struct FusedTile<double, ORDER, FORM> {
 // distinct banks.
 constexpr int fused_lds_stride(int W, int R) { return W + (R == 1 ? 2 : R == 2 ? 4 : 14); }
 static int fused_ty(int order, int form) {
-    return order == 7 || (form != FORM_TALL && form != FORM_TALL512) ? 16 : 32;
+    if (order == 7) return form == FORM_SHORT ? 16 : 24;
+    return form != FORM_TALL && form != FORM_TALL512 ? 16 : 32;
 }
 
 // Region points in ring order, built at compile time: entry k holds the
@@ -780,6 +783,256 @@ k_fused_pairs_2d(const FusedArgs<float> f) {
     }
 }
 
+// Double precision of order 5, and order 7, on tall tiles: the same step with
+// each thread owning vertical groups of R points (x, y .. y + R - 1).  Every
+// ring of the region is R rows tall, so groups tile all of them; listed in ring
+// order (GroupMap) each stage's rectangle is a prefix, and the outermost ring,
+// which no stage computes, only has its state written to LDS.  The points of a
+// group share a column of 3R values: 9 LDS reads a point at order 7 instead of 13,
+// 7 at order 5 instead of 9, and the groups need one address.  A point's arithmetic is the same
+// expression as in k_fused_step_2d, so results are the same bit for bit.
+//
+// Bound, order 7 in double precision: one workgroup a CU (its two stage buffers fill
+// the LDS), 8.6 us a round of 256 tiles, of which loads and stores are 3 and the
+// stages 5.7, 4.6 of them LDS bandwidth (9816 stage points of 9 reads of 16 bytes); the two
+// do not overlap.  Order 7, us per step, 64 x 16 tiles -> these: 777^2 zero-outside
+// FP64 22.2 -> 20.0, FP32 15.0 -> 12.8; 2048^2 116 -> 104 and 68 -> 58; but 640^2 (two
+// rounds of either) 16.0 -> 19.2, so such launches stay on short tiles (fused_form).
+// Order 5 in double precision, against single points: 640^2 10.5 -> 10.1, 1024^2
+// 24.6 -> 22.8, zero-outside 2048^2 with a reservoir 85.1 -> 80.6.  Measured and left: order 7 on
+// 64 x 18 tiles (one group a thread of 1024: 24.0 at 777^2) and 640 threads (20.8).
+template <int W, int HH, int R, int WS> struct GroupMap {
+    unsigned v[W * HH / R];
+    constexpr GroupMap() : v() {
+        int k = 0;
+        for (int s = 4; s >= 0; --s) {
+            const int a = s * R, b = (s + 1) * R;
+            for (int y = a; y < HH - a; y += R)
+                for (int x = a; x < W - a; ++x) {
+                    const bool inner = s < 4 && y >= b && y < HH - b && x >= b && x < W - b;
+                    if (!inner) v[k++] = (unsigned)(y * WS + x) | (unsigned)x << 16 | (unsigned)y << 24;
+                }
+        }
+    }
+};
+template <int W, int HH, int R, int WS> __device__ const GroupMap<W, HH, R, WS> group_map{};
+
+// Tile rows, threads and waves per SIMD: one workgroup a CU in double precision,
+// two in single.
+template <typename T, int ORDER> struct GroupTile;
+template <> struct GroupTile<double, 5> { static constexpr int TY = 32, NT = 1024, WAVES = 4; };
+template <> struct GroupTile<double, 7> { static constexpr int TY = 24, NT = 768, WAVES = 3; };
+template <> struct GroupTile<float, 7> { static constexpr int TY = 24, NT = 768, WAVES = 6; };
+
+template <typename T, int ORDER, int BC, bool DYN, bool S32 = false>
+__global__ void __launch_bounds__((GroupTile<T, ORDER>::NT), (GroupTile<T, ORDER>::WAVES))
+k_fused_groups_2d(const FusedArgs<T> f) {
+    using C = cplx_t<T>;
+    using GT = GroupTile<T, ORDER>;
+    constexpr int R = (ORDER - 1) / 2, H = 4 * R;
+    constexpr int TX = 64, TY = GT::TY, NT = GT::NT;
+    constexpr int W = TX + 2 * H, HH = TY + 2 * H, WS = W + 2;
+    constexpr int NG = W * HH / R, NA = (W - 2 * R) * (HH - 2 * R) / R;     // groups; those of stage 1
+    constexpr int J = (NA + NT - 1) / NT;          // groups per thread
+    constexpr int NOUT = TX * TY / R;              // output groups: the first entries
+    static_assert(TY % R == 0 && W < 256 && HH < 256 && HH * WS < 65536, "group tile shape");
+    constexpr int PAD = R * WS + R;
+    __shared__ C ys_mem[2][HH * WS + 2 * PAD];
+    C *const ya = ys_mem[0] + PAD;
+    C *const yb = ys_mem[1] + PAD;
+
+    const int t = xcd_tile(f.ntiles, f.chunk);
+    if (t < 0) return;
+    TileDesc td;
+    MemberDev<T> m;
+    if (f.grid_ntx > 0) {
+        td.m = 0; td.x0 = (t % f.grid_ntx) * TX; td.y0 = (t / f.grid_ntx) * TY + (BC == BC_SLAB ? H : 0);
+        m = f.grid;
+    } else {
+        td = f.tiles[t];
+        m = f.mem[td.m];
+    }
+    const int n = m.n;
+    const int ylim = BC == BC_SLAB ? f.slab_end : n;
+    const long long off = m.off;
+    using SC = std::conditional_t<S32, float2, C>;      // storage types
+    using SR = std::conditional_t<S32, float, T>;
+    const SC *u = (const SC *)f.u + off;
+    const SR *un = DYN ? (const SR *)f.un + off : nullptr;
+    const SR *P = (const SR *)f.P + off;
+    SC *uo = (SC *)f.uo + off;
+    SR *uno = DYN ? (SR *)f.uno + off : nullptr;
+    const int tid = threadIdx.x;
+
+    if (f.it >= m.steps) {            // budget used up: pass the state through
+        for (int k = tid; k < TX * TY; k += NT) {
+            const int gx = td.x0 + (k & (TX - 1)), gy = td.y0 + k / TX;
+            if (gx >= n || gy >= ylim) continue;
+            const size_t gi = (size_t)gy * n + gx;
+            uo[gi] = u[gi];
+            if (DYN) uno[gi] = un[gi];
+        }
+        return;
+    }
+
+    const T dt = m.dt, dt2 = dt * (T)0.5, dt6 = m.g.dt6;
+    const T dtw = m.g.dtw, dtw2 = dtw * (T)0.5, dtw6 = m.g.dtw6;
+    Coeffs<T> c = m.c;
+    GridCoeffs<T> g = m.g;
+    // coefficients as in k_fused_step_2d (with a reservoir and reflecting
+    // boundaries there are no registers for them)
+    if constexpr (sizeof(T) == 4 && !(BC == BC_REF && DYN))
+        asm volatile("" : "+v"(g.c4), "+v"(g.wc), "+v"(c.d13), "+v"(c.c13));
+    const unsigned *map = group_map<W, HH, R, WS>.v;
+
+    C uu[J][R], acc[J][R];
+    T cp[J][R], nn[J][R], yn[J][R], accn[J][R];
+    int li[J];                         // LDS index of the group's uppermost point
+    unsigned inside = 0;               // BC_REF, bit R j + q: point q of group j lies on the grid
+    static_assert(R * J <= 32, "inside mask");
+    const bool near = n >= TX + H && n >= TY + H;
+    // grid index of region point (lx, ly); false: outside
+    auto locate = [&](int lx, int ly, unsigned &gi) {
+        int gx = td.x0 - H + lx, gy = td.y0 - H + ly;
+        bool ok = true;
+        if (BC == BC_PERIODIC || BC == BC_SLAB) gx = near ? wrap_near3(gx, n) : wrap_index(gx, n);
+        if (BC == BC_PERIODIC) gy = near ? wrap_near3(gy, n) : wrap_index(gy, n);
+        else if (BC == BC_SLAB) ok = gy < ylim + H;
+        else ok = gx >= 0 && gx < n && gy >= 0 && gy < n;
+        gi = grid_index(gy, n, gx);
+        return ok;
+    };
+
+    // the outermost ring's state
+#pragma unroll
+    for (int j = 0; j < (NG - NA + NT - 1) / NT; ++j) {
+        const int k = NA + tid + NT * j;
+        if (k < NG) {
+            const unsigned e = map[k];
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                unsigned gi;
+                const bool ok = locate((int)((e >> 16) & 255), (int)(e >> 24) + q, gi);
+                ya[(int)(e & 0xffff) + q * WS] = ok ? mk<T>((T)u[gi].x, (T)u[gi].y) : mk<T>(0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        const int k = tid + NT * j;
+        li[j] = 0;
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            uu[j][q] = mk<T>(0, 0); cp[j][q] = 0; nn[j][q] = 0; acc[j][q] = mk<T>(0, 0); accn[j][q] = 0;
+        }
+        if (NA % NT == 0 || j < J - 1 || k < NA) {
+            const unsigned e = map[k];
+            li[j] = e & 0xffff;
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                unsigned gi;
+                if (locate((int)((e >> 16) & 255), (int)(e >> 24) + q, gi)) {
+                    if (BC == BC_REF) inside |= 1u << (R * j + q);
+                    uu[j][q] = mk<T>((T)u[gi].x, (T)u[gi].y);
+                    cp[j][q] = (T)P[gi];
+                    if (DYN) nn[j][q] = (T)un[gi];
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            if (NA % NT == 0 || j < J - 1 || tid + NT * j < NA) {
+                ya[li[j] + q * WS] = uu[j][q];
+                // outside the reference's grid both buffers hold zero throughout
+                if (BC == BC_REF && !((inside >> (R * j + q)) & 1u)) yb[li[j] + q * WS] = mk<T>(0, 0);
+            }
+            cp[j][q] = pump_term<T, DYN>(c, cp[j][q]);
+            yn[j][q] = nn[j][q];
+        }
+    __syncthreads();
+
+    typedef T V2 __attribute__((ext_vector_type(2)));
+    using LV = __attribute__((address_space(3))) const V2;
+    // right-hand sides of the group's points from stage input yin, the points
+    // one after another: done(q, k, kn)
+    auto group_rhs = [&](const C *yin, int j, auto done) {
+        unsigned a = (unsigned)(size_t)((LV *)yin + (li[j] - R * WS));
+        asm volatile("" : "+v"(a));
+        LV *ys = (LV *)(size_t)a;
+        auto rd = [&](int i) { const V2 v = ys[i]; return mk<T>(v.x, v.y); };
+        C col[3 * R];                  // rows y - R .. y + 2R - 1
+#pragma unroll
+        for (int i = 0; i < 2 * R; ++i) col[i] = rd(i * WS);
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            col[2 * R + q] = rd((2 * R + q) * WS);
+            T sr, sm;
+#pragma unroll
+            for (int d = 1; d <= R; ++d) {
+                const C l = rd((R + q) * WS - d), r = rd((R + q) * WS + d), &up = col[R + q - d], &dn = col[R + q + d];
+                if (d == 1) {
+                    sr = grid_ring1(g, l.x, r.x, up.x, dn.x);
+                    sm = grid_ring1(g, l.y, r.y, up.y, dn.y);
+                } else {
+                    sr = grid_ring(sr, d == 2 ? g.r2 : g.r3, l.x, r.x, up.x, dn.x);
+                    sm = grid_ring(sm, d == 2 ? g.r2 : g.r3, l.y, r.y, up.y, dn.y);
+                }
+            }
+            C k;
+            T kn;
+            grid_rhs<T, DYN>(g, c, cp[j][q], col[R + q], yn[j][q], mk<T>(sr, sm), k, kn);
+            done(q, k, kn);
+            // the next row's reads after this point is done, so that they do
+            // not all live in registers at once
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+#pragma unroll
+    for (int s = 1; s <= 3; ++s) {
+        const int cnt = (W - 2 * s * R) * (HH - 2 * s * R) / R;
+        int lim = cnt;
+        asm volatile("" : "+s"(lim));
+        const T dta = (s == 3) ? dt : dt2, dtwa = (s == 3) ? dtw : dtw2;
+        const C *yin = (s == 2) ? yb : ya;
+        C *yout = (s == 2) ? ya : yb;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            if (NT * j >= cnt) break;
+            if (tid + NT * j >= lim) continue;
+            group_rhs(yin, j, [&](int q, const C &k, T kn) {
+                grid_acc(acc[j][q].x, k.x, s == 1);
+                grid_acc(acc[j][q].y, k.y, s == 1);
+                if (DYN) grid_acc(accn[j][q], kn, s == 1);
+                const C yv = mk<T>(grid_input(uu[j][q].x, k.x, dtwa), grid_input(uu[j][q].y, k.y, dtwa));
+                if (BC != BC_REF || ((inside >> (R * j + q)) & 1u)) yout[li[j] + q * WS] = yv;
+                if (DYN) yn[j][q] = grid_input(nn[j][q], kn, dta);
+            });
+        }
+        __syncthreads();
+    }
+
+    // stage 4 on the output tile and u_new = u + (k1 + 2 k2 + 2 k3 + k4) dt/6
+#pragma unroll
+    for (int j = 0; j < (NOUT + NT - 1) / NT; ++j) {
+        const int k0 = tid + NT * j;
+        if (k0 >= NOUT) break;
+        const int gx = td.x0 + (k0 & (TX - 1)), gy = td.y0 + R * (k0 / TX);
+        if (gx >= n || gy >= ylim) continue;
+        group_rhs(yb, j, [&](int q, const C &k, T kn) {
+            if (gy + q < ylim) {
+                const size_t gi = (size_t)(gy + q) * n + gx;
+                uo[gi] = SC{(SR)grid_new(uu[j][q].x, acc[j][q].x, k.x, dtw6),
+                            (SR)grid_new(uu[j][q].y, acc[j][q].y, k.y, dtw6)};
+                if (DYN) uno[gi] = (SR)grid_new(nn[j][q], accn[j][q], kn, dt6);
+            }
+        });
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Engine RESIDENT: one workgroup per member holds the member's whole grid on
 // chip and runs all of the call's steps in one launch -- a persistent kernel
@@ -973,8 +1226,8 @@ static void launch_batch_stage(int dim, int order, int bc, bool dyn, const Batch
 }
 
 // One fused step launch in the given form; forms a configuration does not
-// build (order 7 has one form; FORM_HALF is double precision without
-// reflecting boundaries; FORM_TALL512 is the single-precision pair kernel)
+// build (FORM_HALF is double precision without reflecting boundaries, not of
+// order 7; FORM_TALL512 is the single-precision pair kernel)
 // fall back to FORM_TALL, which fused_form never asks otherwise.
 template <typename T, int O, int B, bool D, bool S32 = false>
 static void launch_fused_form(int form, const FusedArgs<T> &f, hipStream_t s) {
@@ -991,21 +1244,22 @@ static void launch_fused_form(int form, const FusedArgs<T> &f, hipStream_t s) {
             hipLaunchKernelGGL((k_fused_pairs_2d<B, D, TALL>), grid, dim3(FusedTile<T, O, TALL>::NT), 0, s, f);
         return;
     }
-    if constexpr (O != 7) {
-        if (form == FORM_SHORT) {
-            hipLaunchKernelGGL((k_fused_step_2d<T, O, B, D, FORM_SHORT, S32>), grid,
-                               dim3(FusedTile<T, O, FORM_SHORT>::NT), 0, s, f);
+    if (form == FORM_SHORT) {
+        hipLaunchKernelGGL((k_fused_step_2d<T, O, B, D, FORM_SHORT, S32>), grid,
+                           dim3(FusedTile<T, O, FORM_SHORT>::NT), 0, s, f);
+        return;
+    }
+    if constexpr (O != 7 && sizeof(T) == 8 && B != BC_REF)
+        if (form == FORM_HALF) {
+            hipLaunchKernelGGL((k_fused_step_2d<T, O, B, D, FORM_HALF, S32>), grid,
+                               dim3(FusedTile<T, O, FORM_HALF>::NT), 0, s, f);
             return;
         }
-        if constexpr (sizeof(T) == 8 && B != BC_REF)
-            if (form == FORM_HALF) {
-                hipLaunchKernelGGL((k_fused_step_2d<T, O, B, D, FORM_HALF, S32>), grid,
-                                   dim3(FusedTile<T, O, FORM_HALF>::NT), 0, s, f);
-                return;
-            }
-    }
-    hipLaunchKernelGGL((k_fused_step_2d<T, O, B, D, FORM_TALL, S32>), grid, dim3(FusedTile<T, O, FORM_TALL>::NT), 0,
-                       s, f);
+    if constexpr (O == 7 || (O == 5 && sizeof(T) == 8))
+        hipLaunchKernelGGL((k_fused_groups_2d<T, O, B, D, S32>), grid, dim3(GroupTile<T, O>::NT), 0, s, f);
+    else
+        hipLaunchKernelGGL((k_fused_step_2d<T, O, B, D, FORM_TALL, S32>), grid, dim3(FusedTile<T, O, FORM_TALL>::NT),
+                           0, s, f);
 }
 
 // Double-precision arithmetic on single-precision fields (NLS_FLAG_F64_ARITH):
@@ -1042,9 +1296,9 @@ int device_cus() {
 }
 
 // The fused kernel's form for a launch over grids (or row slabs) of the
-// given sizes, from the count of its 64 x 16 tiles (tiles16) and 64 x 32
-// tiles (tiles32) against the compute units.  Measured on MI355X, order 5:
-//  - tiles16 <= CUs, FORM_SHORT: a lone 256^2 grid 7.1 -> 5.2 us per step in
+// given sizes, from the count of its tiles against the compute units.
+// Measured on MI355X, order 5:
+//  - 64 x 16 tiles <= CUs, FORM_SHORT: a lone 256^2 grid 7.1 -> 5.2 us per step in
 //    single precision and 8.8 -> 6.2 us in double; 512^2 (256 tiles)
 //    7.3 -> 5.7 and 9.4 -> 7.1 us.
 //  - otherwise FORM_TALL: where CUs would hold two short tiles the tall
@@ -1056,7 +1310,10 @@ int device_cus() {
 //    on one device): 2048^2 (8 rounds) 89 -> 82 us, the sweep512 batch
 //    196 -> 190 us; at two rounds or fewer the tall tiles are as fast or
 //    faster (1024^2: 41 us tall, 43 us half; a 2048 x 256 slab, one round:
-//    13.1 us tall, 14.9 us half).
+//    13.1 us tall, 14.9 us half);
+//  - order 7: a CU's 64 x 24 tiles cost 1.2 to 1.3 of its 64 x 16 ones (9.0 against 6.9 us
+//    a round in double precision, 5.0 against 4.1 a tile of a CU in single), so the
+//    tall tiles are taken where a CU has fewer than 0.8 as many of them.
 // A process-wide choice of form per dtype (nls_tune_fused_form, set by the
 // autotuner), -1: the rule below.
 static std::atomic<int> g_fused_form[2] = {{-1}, {-1}};
@@ -1068,23 +1325,37 @@ int set_fused_form(int dtype, int form) {
 }
 int get_fused_form(int dtype) { return g_fused_form[dtype == NLS_F64 ? 1 : 0].load(); }
 
-static int fused_form(int dtype, int order, int bc, long long tiles16, long long tiles32) {
+// Tiles of a launch by their rows.
+struct TileCounts {
+    long long t16 = 0, t24 = 0, t32 = 0;
+    void add(int n, int rows) {
+        const long long nx = (n + 63) / 64;
+        t16 += nx * ((rows + 15) / 16);
+        t24 += nx * ((rows + 23) / 24);
+        t32 += nx * ((rows + 31) / 32);
+    }
+};
+static TileCounts tiles_of(int n, int rows) {
+    TileCounts t;
+    t.add(n, rows);
+    return t;
+}
+static int fused_form(int dtype, int order, int bc, const TileCounts &t) {
     const int forced = get_fused_form(dtype);
     if (forced >= 0) {
         // forms a configuration does not build run tall (launch_fused_form)
-        if (order == 7 || (forced == FORM_HALF && (dtype != NLS_F64 || bc == BC_REF))) return FORM_TALL;
+        if (forced == FORM_HALF && (order == 7 || dtype != NLS_F64 || bc == BC_REF)) return FORM_TALL;
         if (forced == FORM_TALL512 && !(dtype == NLS_F32 && order == 5 && bc == BC_PERIODIC && NLS_FUSED_PAIRS))
             return FORM_TALL;
         return forced;
     }
-    if (order == 7) return FORM_TALL;
     const int cus = device_cus();
     if (cus <= 0) return FORM_TALL;
-    if (tiles16 <= cus) return FORM_SHORT;
-    if (dtype == NLS_F64 && bc != BC_REF && tiles32 > 2LL * cus) return FORM_HALF;
+    if (t.t16 <= cus) return FORM_SHORT;
+    if (order == 7) return 5 * ((t.t24 + cus - 1) / cus) < 4 * ((t.t16 + cus - 1) / cus) ? FORM_TALL : FORM_SHORT;
+    if (dtype == NLS_F64 && bc != BC_REF && t.t32 > 2LL * cus) return FORM_HALF;
     return FORM_TALL;
 }
-static long long tiles_of(int n, int rows, int ty) { return (long long)((n + 63) / 64) * ((rows + ty - 1) / ty); }
 
 // ---- marching strips or tiles ------------------------------------------------
 // The marching kernel (nls_march.hip: order 5, periodic) runs the step of
@@ -1106,9 +1377,9 @@ constexpr int MARCH_PIECE = 16;
 static double march_us(int dtype, int percu, int rows) {
     return percu * rows * (dtype == NLS_F64 ? (percu > 1 ? 0.45 : 0.55) : (percu > 1 ? 0.23 : 0.37));
 }
-static double tiles_us(int dtype, long long tiles16, long long tiles32, int cus) {
-    if (tiles16 <= cus) return dtype == NLS_F64 ? 6.7 : 5.4;
-    return MARCH_LAUNCH + (dtype == NLS_F64 ? 7.7 * ((tiles16 + 511) / 512) : 7.4 * ((tiles32 + 511) / 512));
+static double tiles_us(int dtype, const TileCounts &t, int cus) {
+    if (t.t16 <= cus) return dtype == NLS_F64 ? 6.7 : 5.4;
+    return MARCH_LAUNCH + (dtype == NLS_F64 ? 7.7 * ((t.t16 + 511) / 512) : 7.4 * ((t.t32 + 511) / 512));
 }
 // Members the kernel takes: rows of at least one wave, and byte offsets that
 // stay below 2^32 when they run past the grid's end by up to its size.
@@ -1140,7 +1411,7 @@ static MarchGrid march_grid(const nls_problem *p) {
     MarchGrid best = {0, 0, 0, 0, 0};
     const int n = p->n, cus = device_cus();
     if (n <= 256 || !march_applies(p->dtype, p->order, p->bc) || !march_holds(n, p->dtype) || cus <= 0) return best;
-    double least = tiles_us(p->dtype, tiles_of(n, n, 16), tiles_of(n, n, 32), cus);
+    double least = tiles_us(p->dtype, tiles_of(n, n), cus);
     const StripShape sh = strip_shape(n);
     for (int per = 1; per <= march_slots(p->dtype); ++per) {
         const int pieces = std::max(1, per * cus / sh.nx);
@@ -1278,7 +1549,7 @@ static int fused_grid_run(const nls_problem *p, int iters, const T *P, cplx_t<T>
     using C = cplx_t<T>;
     const size_t N = (size_t)p->n * p->n;
     const bool dyn = p->coeffs[10] != 0.0;
-    const int form = fused_form(p->dtype, p->order, p->bc, tiles_of(p->n, p->n, 16), tiles_of(p->n, p->n, 32));
+    const int form = fused_form(p->dtype, p->order, p->bc, tiles_of(p->n, p->n));
     const int ty = fused_ty(p->order, form);
     FusedArgs<T> f;
     memset(&f, 0, sizeof f);
@@ -1340,7 +1611,7 @@ template <typename T>
 static int fused_slab_run(const nls_problem *p, int rows, const T *P, const cplx_t<T> *psi_in, const T *nres_in,
                           cplx_t<T> *psi_out, T *nres_out, hipStream_t s) {
     const int H = 2 * (p->order - 1);
-    const int form = fused_form(p->dtype, p->order, BC_SLAB, tiles_of(p->n, rows, 16), tiles_of(p->n, rows, 32));
+    const int form = fused_form(p->dtype, p->order, BC_SLAB, tiles_of(p->n, rows));
     const int ty = fused_ty(p->order, form);
     FusedArgs<T> f;
     memset(&f, 0, sizeof f);
@@ -1427,7 +1698,7 @@ static int fused_grid_run_s32(const nls_problem *p, int iters, const float *P, f
                               hipStream_t s) {
     const size_t N = (size_t)p->n * p->n;
     const bool dyn = p->coeffs[10] != 0.0;
-    const int form = fused_form(NLS_F64, p->order, p->bc, tiles_of(p->n, p->n, 16), tiles_of(p->n, p->n, 32));
+    const int form = fused_form(NLS_F64, p->order, p->bc, tiles_of(p->n, p->n));
     const int ty = fused_ty(p->order, form);
     FusedArgs<double> f;
     memset(&f, 0, sizeof f);
@@ -1921,19 +2192,18 @@ static void plan(nls_batch *b, const nls_member *members, int count, const int *
     // tiles, member by member, row-major inside a member
     int tx = 64, ty = BATCH_STAGE_TY;
     if (b->engine == NLS_ENGINE_FUSED) {
-        long long tiles16 = 0, tiles32 = 0;
+        TileCounts counts;
         for (int i = 0; i < count; ++i) {
-            tiles16 += tiles_of(members[i].n, members[i].n, 16);
-            tiles32 += tiles_of(members[i].n, members[i].n, 32);
+            counts.add(members[i].n, members[i].n);
         }
-        b->fform = fused_form(b->dtype, b->order, b->bc, tiles16, tiles32);
+        b->fform = fused_form(b->dtype, b->order, b->bc, counts);
         ty = fused_ty(b->order, b->fform);
         const int cus = device_cus();
         b->march = cus > 0 && count > 0 && march_applies(b->dtype, b->order, b->bc);
         for (int i = 0; i < count; ++i) b->march = b->march && march_holds(members[i].n, b->dtype);
         b->cuts[0] = b->cuts[1] = MarchCut();
         if (b->march) {
-            const double tiles = tiles_us(b->dtype, tiles16, tiles32, cus);
+            const double tiles = tiles_us(b->dtype, counts, cus);
             // (nothing marches faster than a few rows of every CU)
             b->march = tiles > MARCH_LAUNCH + march_us(b->dtype, 1, 12 + MARCH_PIECE);
             if (b->march)
