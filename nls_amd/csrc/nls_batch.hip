@@ -1305,12 +1305,13 @@ int device_cus() {
 //    ones are as fast or faster (a 2048 x 256 row slab: 9.7 us short, 9.5 us
 //    tall), and launches of several rounds are faster tall (a batch of
 //    512^2-class grids: 94.6 us tall, 112.4 us short);
-//  - except in double precision without reflecting boundaries when the tall
-//    tiles take more than two rounds of the CUs, FORM_HALF (alternating runs
-//    on one device): 2048^2 (8 rounds) 89 -> 82 us, the sweep512 batch
-//    196 -> 190 us; at two rounds or fewer the tall tiles are as fast or
-//    faster (1024^2: 41 us tall, 43 us half; a 2048 x 256 slab, one round:
-//    13.1 us tall, 14.9 us half);
+//  - except in double precision without reflecting boundaries, FORM_HALF where
+//    the tall tiles take more than two rounds of the CUs (2048^2, 8 rounds: 89
+//    -> 82 us, the sweep512 batch 196 -> 190 us), or more than one while a CU
+//    has fewer than three half tiles on average: 777^2 18.0 -> 16.4 us,
+//    850^2 18.7 -> 17.5, order 3 at 800^2 15.1 -> 13.1; between them the tall
+//    tiles are as fast or faster (900^2: 19.9 us tall, 20.7 us half; 1024^2
+//    22.2 and 21.9; a 2048 x 256 slab, one round: 13.1 us tall, 14.9 us half);
 //  - order 7: a CU's 64 x 24 tiles cost 1.2 to 1.3 of its 64 x 16 ones (9.0 against 6.9 us
 //    a round in double precision, 5.0 against 4.1 a tile of a CU in single), so the
 //    tall tiles are taken where a CU has fewer than 0.8 as many of them.
@@ -1353,7 +1354,7 @@ static int fused_form(int dtype, int order, int bc, const TileCounts &t) {
     if (cus <= 0) return FORM_TALL;
     if (t.t16 <= cus) return FORM_SHORT;
     if (order == 7) return 5 * ((t.t24 + cus - 1) / cus) < 4 * ((t.t16 + cus - 1) / cus) ? FORM_TALL : FORM_SHORT;
-    if (dtype == NLS_F64 && bc != BC_REF && t.t32 > 2LL * cus) return FORM_HALF;
+    if (dtype == NLS_F64 && bc != BC_REF && (t.t32 > 2LL * cus || (t.t32 > cus && t.t16 < 3LL * cus))) return FORM_HALF;
     return FORM_TALL;
 }
 
