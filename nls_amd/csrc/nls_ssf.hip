@@ -27,9 +27,9 @@
 // keeps its error far below that of single-precision transforms.
 //
 // FFTs: Stockham stages with a line's values in the registers of its threads,
-// the stage-to-stage exchanges through LDS (fft_regs).  The middle row pass of
-// 2048-point rows and the kinetic energy keep them in LDS and work in place: a
-// stage stages its butterfly inputs and twiddles in registers, synchronises,
+// the stage-to-stage exchanges through LDS (fft_regs).  The kinetic energy keeps
+// them in LDS and works in place: a stage stages its butterfly inputs and
+// twiddles in registers, synchronises,
 // then writes the outputs.  Twiddles exp(-2 pi i m / n) and the phase table are
 // generated in double precision.
 #include <cstring>
@@ -43,10 +43,12 @@ namespace nls {
 // Row kernels with their values in LDS: one 2048-point line (or several
 // shorter lines) per workgroup, 32 KB, so four workgroups share a CU.
 constexpr int ROW_PTS = 2048, ROW_LOG_PTS = 11, ROW_NTH = 256;
+
 // LDS layout of the transforms: element i at i + (i >> SHIFT), one complex of
 // padding per 2^SHIFT, so that the strided writes of the first radix-8
 // stages (stride 8, then groups of 8 at stride 64) spread over the LDS banks
-// instead of piling on a few; SHIFT = 31 is the plain layout.  Each kernel
+// instead of piling on a few; SHIFT = 31 is the plain layout, 0 a swizzle without
+// padding (each group of eight permuted by the number of its group).  Each kernel
 // takes its own shift (the padding costs index arithmetic where the
 // conflicts it removes are few).
 #ifndef NLS_SSF_ROW_PAD
@@ -61,7 +63,9 @@ constexpr int ROW_PTS = 2048, ROW_LOG_PTS = 11, ROW_NTH = 256;
 constexpr int lds_padded(int pts, int shift) { return pts + (shift < 31 ? pts >> shift : 0); }
 template <typename T, int SHIFT> struct Lds {
     cplx_t<T> *p;
-    __device__ __forceinline__ cplx_t<T> &operator[](int i) const { return p[SHIFT < 31 ? i + (i >> SHIFT) : i]; }
+    __device__ __forceinline__ cplx_t<T> &operator[](int i) const {
+        return p[SHIFT == 0 ? i ^ ((i >> 3) & 7) : SHIFT < 31 ? i + (i >> SHIFT) : i];
+    }
 };
 
 template <typename T>
@@ -249,205 +253,6 @@ __device__ __forceinline__ void fft_radix2_stage(LB buf, int logN, int logL, int
     __syncthreads();
 }
 
-// Stages whose inputs come from ld(l, e) and whose outputs go to st(l, e, v)
-// (element e of line l; q, r: the thread's butterfly and its output, known
-// at compile time once unrolled) instead of the LDS buffer: the first stage
-// of a transform can read its inputs from HBM, the last one write to HBM or
-// apply a pointwise factor on the way.  SYNC: synchronise between the reads and
-// the writes (outputs written in place over inputs other threads read); the
-// caller synchronises after the writes where they go to LDS.  TW: multiply by
-// the twiddles (the first stage's are all 1 and are skipped).  The butterfly
-// arithmetic is that of fft_radix8_stage / fft_radix4_stage.
-template <typename T, bool INV, bool LINE_FAST, int PTS, int NTH, bool SYNC, bool TW, typename LD, typename ST>
-__device__ __forceinline__ void fft_radix8_io(int logN, int logL, int logNs, const cplx_t<T> *tw, cplx_t<T> w8,
-                                              LD ld, ST st) {
-    using C = cplx_t<T>;
-    constexpr int QB = (PTS / 8 + NTH - 1) / NTH;
-    const int lognb = logN - 3;
-    const int total = 1 << (logL + lognb);
-    const int Ns = 1 << logNs;
-    const int sh = logN - logNs - 3;
-    C v[QB][8], w[QB][7];
-#pragma unroll
-    for (int q = 0; q < QB; ++q) {
-        const int b = threadIdx.x + NTH * q;
-        if (b < total) {
-            const int l = LINE_FAST ? (b & ((1 << logL) - 1)) : (b >> lognb);
-            const int j = LINE_FAST ? (b >> logL) : (b & ((1 << lognb) - 1));
-            const int k = j & (Ns - 1);
-            if (TW) {
-#pragma unroll
-                for (int r = 1; r < 8; ++r) w[q][r - 1] = tw[(r * k) << sh];
-            }
-#pragma unroll
-            for (int r = 0; r < 8; ++r) v[q][r] = ld(l, j + (r << lognb));
-        }
-    }
-    if (SYNC) __syncthreads();
-    if (INV) w8.y = -w8.y;
-#pragma unroll
-    for (int q = 0; q < QB; ++q) {
-        const int b = threadIdx.x + NTH * q;
-        if (b < total) {
-            const int l = LINE_FAST ? (b & ((1 << logL) - 1)) : (b >> lognb);
-            const int j = LINE_FAST ? (b >> logL) : (b & ((1 << lognb) - 1));
-            const int k = j & (Ns - 1);
-            if (TW) {
-#pragma unroll
-                for (int r = 1; r < 8; ++r) {
-                    C wr = w[q][r - 1];
-                    if (INV) wr.y = -wr.y;
-                    v[q][r] = cmul<T>(v[q][r], wr);
-                }
-            }
-            C e0 = v[q][0], e1 = v[q][2], e2 = v[q][4], e3 = v[q][6];
-            C o0 = v[q][1], o1 = v[q][3], o2 = v[q][5], o3 = v[q][7];
-            dft4<T, INV>(e0, e1, e2, e3);
-            dft4<T, INV>(o0, o1, o2, o3);
-            o1 = cmul<T>(o1, w8);
-            o2 = INV ? mk<T>(-o2.y, o2.x) : mk<T>(o2.y, -o2.x);
-            o3 = cmul<T>(o3, w8);
-            o3 = INV ? mk<T>(-o3.y, o3.x) : mk<T>(o3.y, -o3.x);
-            const int d = ((j >> logNs) << (logNs + 3)) + k;
-            st(l, d, mk<T>(e0.x + o0.x, e0.y + o0.y), q, 0);
-            st(l, d + Ns, mk<T>(e1.x + o1.x, e1.y + o1.y), q, 1);
-            st(l, d + 2 * Ns, mk<T>(e2.x + o2.x, e2.y + o2.y), q, 2);
-            st(l, d + 3 * Ns, mk<T>(e3.x + o3.x, e3.y + o3.y), q, 3);
-            st(l, d + 4 * Ns, mk<T>(e0.x - o0.x, e0.y - o0.y), q, 4);
-            st(l, d + 5 * Ns, mk<T>(e1.x - o1.x, e1.y - o1.y), q, 5);
-            st(l, d + 6 * Ns, mk<T>(e2.x - o2.x, e2.y - o2.y), q, 6);
-            st(l, d + 7 * Ns, mk<T>(e3.x - o3.x, e3.y - o3.y), q, 7);
-        }
-    }
-}
-
-template <typename T, bool INV, bool LINE_FAST, int PTS, int NTH, bool SYNC, typename LD, typename ST>
-__device__ __forceinline__ void fft_radix4_io(int logN, int logL, int logNs, const cplx_t<T> *tw, LD ld, ST st) {
-    using C = cplx_t<T>;
-    constexpr int QB = (PTS / 4 + NTH - 1) / NTH;
-    const int lognb = logN - 2;
-    const int total = 1 << (logL + lognb);
-    const int Ns = 1 << logNs;
-    const int sh = logN - logNs - 2;
-    C v[QB][4], w[QB][3];
-#pragma unroll
-    for (int q = 0; q < QB; ++q) {
-        const int b = threadIdx.x + NTH * q;
-        if (b < total) {
-            const int l = LINE_FAST ? (b & ((1 << logL) - 1)) : (b >> lognb);
-            const int j = LINE_FAST ? (b >> logL) : (b & ((1 << lognb) - 1));
-            const int k = j & (Ns - 1);
-#pragma unroll
-            for (int r = 1; r < 4; ++r) w[q][r - 1] = tw[(r * k) << sh];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) v[q][r] = ld(l, j + (r << lognb));
-        }
-    }
-    if (SYNC) __syncthreads();
-#pragma unroll
-    for (int q = 0; q < QB; ++q) {
-        const int b = threadIdx.x + NTH * q;
-        if (b < total) {
-            const int l = LINE_FAST ? (b & ((1 << logL) - 1)) : (b >> lognb);
-            const int j = LINE_FAST ? (b >> logL) : (b & ((1 << lognb) - 1));
-            const int k = j & (Ns - 1);
-#pragma unroll
-            for (int r = 1; r < 4; ++r) {
-                C wr = w[q][r - 1];
-                if (INV) wr.y = -wr.y;
-                v[q][r] = cmul<T>(v[q][r], wr);
-            }
-            const C t0 = mk<T>(v[q][0].x + v[q][2].x, v[q][0].y + v[q][2].y);
-            const C t1 = mk<T>(v[q][0].x - v[q][2].x, v[q][0].y - v[q][2].y);
-            const C t2 = mk<T>(v[q][1].x + v[q][3].x, v[q][1].y + v[q][3].y);
-            const C d13 = mk<T>(v[q][1].x - v[q][3].x, v[q][1].y - v[q][3].y);
-            const C t3 = INV ? mk<T>(-d13.y, d13.x) : mk<T>(d13.y, -d13.x);
-            const int d = ((j >> logNs) << (logNs + 2)) + k;
-            st(l, d, mk<T>(t0.x + t2.x, t0.y + t2.y), q, 0);
-            st(l, d + Ns, mk<T>(t1.x + t3.x, t1.y + t3.y), q, 1);
-            st(l, d + 2 * Ns, mk<T>(t0.x - t2.x, t0.y - t2.y), q, 2);
-            st(l, d + 3 * Ns, mk<T>(t1.x - t3.x, t1.y - t3.y), q, 3);
-        }
-    }
-}
-
-// The last stage of one 2048-point transform (radix 4, A) and the first of
-// the next (radix 8, B) without LDS in between.  A thread's two radix-4
-// butterflies of A produce the elements j0 + 256 s (s = 0 .. 7) of its line,
-// and those are exactly the inputs of its radix-8 butterfly of B; so the
-// outputs of A go through the pointwise map g(l, e, s, v) in registers (the
-// point's fields are the thread's slot s) straight into B, whose outputs go to
-// st(l, e, v, q, r).  One barrier between A's LDS reads and B's LDS writes
-// (B writes elements other threads read in A).  Arithmetic as in
-// fft_radix4_stage and fft_radix8_stage (B's twiddles are all 1, skipped).
-template <typename T, bool INV_A, bool INV_B, bool LINE_FAST, int PTS, int NTH, typename LD, typename G, typename ST>
-__device__ __forceinline__ void fft_2048_turn(int logL, const cplx_t<T> *tw, cplx_t<T> w8, LD ld, G g, ST st) {
-    using C = cplx_t<T>;
-    constexpr int LN = 11;
-    static_assert((PTS / 4 + NTH - 1) / NTH == 2 && (PTS / 8 + NTH - 1) / NTH == 1 && PTS == NTH * 8,
-                  "a thread holds two radix-4 and one radix-8 butterflies of its line");
-    C v[2][4], w[2][3];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        const int b = threadIdx.x + NTH * q;
-        const int l = LINE_FAST ? (b & ((1 << logL) - 1)) : (b >> (LN - 2));
-        const int j = LINE_FAST ? (b >> logL) : (b & ((1 << (LN - 2)) - 1));
-#pragma unroll
-        for (int r = 1; r < 4; ++r) w[q][r - 1] = tw[r * j];       // k = j: the last stage, Ns = 512
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[q][r] = ld(l, j + (r << (LN - 2)));
-    }
-    __syncthreads();
-    const int bb = threadIdx.x;
-    const int l = LINE_FAST ? (bb & ((1 << logL) - 1)) : (bb >> (LN - 3));
-    const int j0 = LINE_FAST ? (bb >> logL) : (bb & ((1 << (LN - 3)) - 1));
-    C x[8];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-#pragma unroll
-        for (int r = 1; r < 4; ++r) {
-            C wr = w[q][r - 1];
-            if (INV_A) wr.y = -wr.y;
-            v[q][r] = cmul<T>(v[q][r], wr);
-        }
-        const C t0 = mk<T>(v[q][0].x + v[q][2].x, v[q][0].y + v[q][2].y);
-        const C t1 = mk<T>(v[q][0].x - v[q][2].x, v[q][0].y - v[q][2].y);
-        const C t2 = mk<T>(v[q][1].x + v[q][3].x, v[q][1].y + v[q][3].y);
-        const C d13 = mk<T>(v[q][1].x - v[q][3].x, v[q][1].y - v[q][3].y);
-        const C t3 = INV_A ? mk<T>(-d13.y, d13.x) : mk<T>(d13.y, -d13.x);
-        // element j0 + 256 q + 512 r of the line: slot s = q + 2 r
-        x[q] = mk<T>(t0.x + t2.x, t0.y + t2.y);
-        x[q + 2] = mk<T>(t1.x + t3.x, t1.y + t3.y);
-        x[q + 4] = mk<T>(t0.x - t2.x, t0.y - t2.y);
-        x[q + 6] = mk<T>(t1.x - t3.x, t1.y - t3.y);
-    }
-    // the pointwise map one point at a time, after both butterflies (with
-    // the maps' temporaries interleaved, a SIMD would hold half the waves)
-#pragma unroll
-    for (int sl = 0; sl < 8; ++sl) {
-        x[sl] = g(l, j0 + 256 * sl, sl, x[sl]);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    if (INV_B) w8.y = -w8.y;
-    C e0 = x[0], e1 = x[2], e2 = x[4], e3 = x[6];
-    C o0 = x[1], o1 = x[3], o2 = x[5], o3 = x[7];
-    dft4<T, INV_B>(e0, e1, e2, e3);
-    dft4<T, INV_B>(o0, o1, o2, o3);
-    o1 = cmul<T>(o1, w8);
-    o2 = INV_B ? mk<T>(-o2.y, o2.x) : mk<T>(o2.y, -o2.x);
-    o3 = cmul<T>(o3, w8);
-    o3 = INV_B ? mk<T>(-o3.y, o3.x) : mk<T>(o3.y, -o3.x);
-    const int d = j0 << 3;                                          // Ns = 1
-    st(l, d, mk<T>(e0.x + o0.x, e0.y + o0.y), 0, 0);
-    st(l, d + 1, mk<T>(e1.x + o1.x, e1.y + o1.y), 0, 1);
-    st(l, d + 2, mk<T>(e2.x + o2.x, e2.y + o2.y), 0, 2);
-    st(l, d + 3, mk<T>(e3.x + o3.x, e3.y + o3.y), 0, 3);
-    st(l, d + 4, mk<T>(e0.x - o0.x, e0.y - o0.y), 0, 4);
-    st(l, d + 5, mk<T>(e1.x - o1.x, e1.y - o1.y), 0, 5);
-    st(l, d + 6, mk<T>(e2.x - o2.x, e2.y - o2.y), 0, 6);
-    st(l, d + 7, mk<T>(e3.x - o3.x, e3.y - o3.y), 0, 7);
-}
-
 // In-place FFT of 2^logL lines of length 2^logN (2^(logL+logN) <= PTS) in LDS.
 template <typename T, bool INV, bool LINE_FAST, int PTS, int NTH, typename LB>
 __device__ __forceinline__ void lds_fft(LB buf, int logN, int logL, int lstride, int estride,
@@ -521,62 +326,6 @@ enum { ROWS_FIRST = 0, ROWS_MIDDLE = 1, ROWS_LAST = 2 };
 // Lines of length 2^logN per workgroup of 2^logP points (at most n lines).
 __host__ __device__ constexpr int lines_per_wg(int logN, int logP) {
     return logP - logN < logN ? logP - logN : logN;
-}
-
-// Middle row pass of a grid of 2048-point rows (8 x 8 x 8 x 4), one row a
-// workgroup: the first inverse stage reads HBM; the last inverse stage, the two
-// pointwise half steps and the first forward stage run in registers
-// (fft_2048_turn: a thread's points are the elements tid + 256 s, its slots s of
-// ps and ns); the last forward stage writes HBM.  Held to 128 registers, so four
-// workgroups share a CU.  On a grid of 2048^2 points it takes 60 us (reservoir, double
-// precision; 56 us single), against 66 (60) in registers throughout
-// (k_ssf_row_regs, two workgroups a CU for its registers).  VALU issue is 26 us of it, HBM at the
-// rate of a large copy 45: the FFT stages, the pointwise part and the memory
-// phases overlap only across those four workgroups.
-template <typename S, typename T, bool DYN>
-__global__ void __launch_bounds__(ROW_NTH, 4) k_ssf_rows2048(const SsfArgs<S, T> a) {
-    using C = cplx_t<T>;
-    static_assert(sizeof(T) == 8, "double-precision transforms");
-    constexpr int PPT = ROW_PTS / ROW_NTH, LN = ROW_LOG_PTS, NN = 1 << LN;
-    static_assert(PPT == 8, "a thread holds eight points of the row");
-    __shared__ C buf_mem[lds_padded(ROW_PTS, NLS_SSF_ROW_PAD)];
-    const Lds<T, NLS_SSF_ROW_PAD> buf{buf_mem};
-    const size_t base = (size_t)blockIdx.x << LN;               // rows are contiguous
-    // the fields stay in the storage precision until used (exact
-    // conversion; single-precision storage then holds them in half the
-    // registers)
-    S ps[PPT], ns[PPT];
-#pragma unroll
-    for (int q = 0; q < PPT; ++q) {
-        const int idx = threadIdx.x + ROW_NTH * q;
-        ps[q] = a.P[base + idx];
-        ns[q] = DYN ? a.nres[base + idx] : (S)0;
-    }
-    auto lds_ld = [&](int, int e) { return buf[e]; };
-    auto lds_st = [&](int, int e, C v, int, int) { buf[e] = v; };
-    const C w8 = a.tw[NN >> 3];
-    fft_radix8_io<T, true, false, ROW_PTS, ROW_NTH, false, false>(
-        LN, 0, 0, a.tw, w8, [&](int, int e) { return widen<T, S>(a.psi[base + e]); }, lds_st);
-    __syncthreads();
-    fft_radix8_stage<T, true, false, ROW_PTS, ROW_NTH>(buf, LN, 0, NN, 1, 3, a.tw, w8);
-    fft_radix8_stage<T, true, false, ROW_PTS, ROW_NTH>(buf, LN, 0, NN, 1, 6, a.tw, w8);
-    fft_2048_turn<T, true, false, false, ROW_PTS, ROW_NTH>(
-        0, a.tw, w8, lds_ld,
-        [&](int, int e, int slot, C v) {
-            T nv = (T)ns[slot];
-            const T pv = (T)ps[slot];
-            pointwise_rk4<T, DYN>(a.c, a.inv_c11, pv, a.half_dt, v, nv);
-            pointwise_rk4<T, DYN>(a.c, a.inv_c11, pv, a.half_dt, v, nv);
-            // the reservoir is final here (the transforms act on psi only)
-            if (DYN) a.nres[base + e] = (S)nv;
-            return v;
-        },
-        lds_st);
-    __syncthreads();
-    fft_radix8_stage<T, false, false, ROW_PTS, ROW_NTH>(buf, LN, 0, NN, 1, 3, a.tw, w8);
-    fft_radix8_stage<T, false, false, ROW_PTS, ROW_NTH>(buf, LN, 0, NN, 1, 6, a.tw, w8);
-    fft_radix4_io<T, false, false, ROW_PTS, ROW_NTH, false>(
-        LN, 0, 9, a.tw, lds_ld, [&](int, int e, C v, int, int) { a.psi[base + e] = narrow<S, T>(v); });
 }
 
 // Radix-8 butterfly of Stockham stage logNs of a 2^LN-point transform on
@@ -837,6 +586,110 @@ __global__ void __launch_bounds__((line_threads<LN, PT>)) k_ssf_line(const SsfAr
         a.psi[e] = narrow<S, T>(x[r]);
         if (DYN) a.nres[e] = (S)nn[r];
     }
+}
+
+// Middle row pass of a grid of 2048-point rows (8 x 8 x 8 x 4 points), one row a
+// workgroup, in registers as k_ssf_row_regs but held to 128 registers and 40 KB of
+// LDS, so that four workgroups share a CU: the exchanges go through one buffer,
+// swizzled instead of padded, and the twiddles of the two middle stages, which
+// are 448 entries of the table, come from LDS beside it (from the table, 28 of a
+// thread's 40 loads of 16 bytes, each a miss of an L1 that the fields stream through).
+// Per pass at 2048^2, against the row in LDS with all twiddles from the table:
+// double precision 62.7 -> 57.4 us, without a reservoir 68.2 -> 65; single-precision
+// storage 55.5 -> 50.8 and 62.0 -> 57.9; k_ssf_row_regs, two workgroups a CU, 66 and
+// 60.  VALU issue is 26 us of it, HBM at the rate of a large copy 45 (23 in
+// single): the transforms, the pointwise part and the memory phases overlap
+// only across the four workgroups.
+template <typename S, typename T, bool DYN>
+__global__ void __launch_bounds__(ROW_NTH, 4) k_ssf_rows2048(const SsfArgs<S, T> a) {
+    using C = cplx_t<T>;
+    constexpr int LN = ROW_LOG_PTS, NN = 1 << LN, Q = NN / 8;
+    static_assert(Q == ROW_NTH, "a thread holds eight points of the row");
+    __shared__ C mem[NN];
+    __shared__ C twt[7][72];                                    // w^(4 (r+1) k) at [r][k + k / 8], k < 64
+    const int j = threadIdx.x;
+    const size_t row = (size_t)blockIdx.x << LN;                // rows are contiguous
+    cplx_t<S> *const psi = a.psi + row;
+    S *const nres = DYN ? a.nres + row : nullptr;
+    const S *const P = a.P + row;
+    C x[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) x[r] = widen<T, S>(psi[(unsigned)(j + Q * r)]);
+    // the fields stay in the storage precision until used (exact conversion;
+    // single-precision storage then holds them in half the registers)
+    S ps[8], ns[8];
+    auto fields = [&] {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            ps[r] = P[(unsigned)(j + Q * r)];
+            ns[r] = DYN ? nres[(unsigned)(j + Q * r)] : (S)0;
+        }
+    };
+    for (int e = j; e < 7 * 64; e += ROW_NTH) twt[e >> 6][(e & 63) + ((e & 63) >> 3)] = a.tw[(((e >> 6) + 1) * (e & 63)) << 2];
+    const C w8 = a.tw[NN >> 3];
+    const Lds<T, 0> B{mem};
+    // the thread's index, opaque: the stages' addresses, equal in both
+    // transforms, would otherwise stay in registers from one to the other
+    auto fresh = [&] {
+        int v = j;
+        asm volatile("" : "+v"(v));
+        return v;
+    };
+    auto ex = [&](int logNs) {
+        const int j = fresh(), Ns = 1 << logNs, d = ((j >> logNs) << (logNs + 3)) + (j & (Ns - 1));
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 8; ++r) B[d + r * Ns] = x[r];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 8; ++r) x[r] = B[j + Q * r];
+    };
+    auto fft = [&](auto inv) {
+        constexpr bool INV = decltype(inv)::value;
+        const int j = fresh();
+        auto turn = [&](int m) {
+            const C *w0 = &twt[0][m];
+#pragma unroll
+            for (int r = 1; r < 8; ++r) {
+                C w = w0[72 * (r - 1)];
+                if (INV) w.y = -w.y;
+                x[r] = cmul<T>(x[r], w);
+                if (r == 4) __builtin_amdgcn_sched_barrier(0);      // half the twiddles in registers at once
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        bfly8<T, INV, false>(x, j, 0, LN, a.tw, w8);
+        ex(0);
+        turn(9 * (j & 7));
+        bfly8<T, INV, false>(x, j, 3, LN, a.tw, w8);
+        ex(3);
+        if (INV) fields();               // in flight under the last two stages
+        turn((j & 63) + ((j & 63) >> 3));
+        bfly8<T, INV, false>(x, j, 6, LN, a.tw, w8);
+        ex(6);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            bfly4<T, INV, true>(x[q], x[q + 2], x[q + 4], x[q + 6], j + Q * q, LN - 2, LN, a.tw);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    fft(std::true_type());
+    const unsigned jn = (unsigned)fresh();
+    // one point at a time (with their temporaries interleaved, a SIMD would
+    // hold half the waves)
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+        T nv = (T)ns[r];
+        const T pv = (T)ps[r];
+        pointwise_rk4<T, DYN>(a.c, a.inv_c11, pv, a.half_dt, x[r], nv);
+        pointwise_rk4<T, DYN>(a.c, a.inv_c11, pv, a.half_dt, x[r], nv);
+        // the reservoir is final here (the transforms act on psi only)
+        if (DYN) nres[jn + Q * r] = (S)nv;
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    fft(std::false_type());
+#pragma unroll
+    for (int r = 0; r < 8; ++r) psi[(unsigned)(j + Q * r)] = narrow<S, T>(x[r]);
 }
 
 // Row pass: rows in registers (fft_regs), as many as fill a wave or one of
