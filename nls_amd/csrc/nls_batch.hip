@@ -1236,6 +1236,14 @@ static void launch_fused_form(int form, const FusedArgs<T> &f, hipStream_t s) {
         // zero-outside grids with a reservoir field would spill at 1024
         // threads (64 registers) and run the tall tile on 512
         constexpr int TALL = B == BC_REF && D ? FORM_TALL512 : FORM_TALL;
+        // (past two tiles a CU one point a thread at 1024 threads is the faster:
+        // 12 grids of 300^2 15.7 / 15.2 us, 2048^2 40.5 / 39.9; two a CU 11.4 / 11.9)
+        if constexpr (B == BC_REF && D)
+            if (form != FORM_SHORT && f.ntiles > 2 * device_cus()) {
+                hipLaunchKernelGGL((k_fused_step_2d<T, O, B, D, FORM_TALL, S32>), grid,
+                                   dim3(FusedTile<T, O, FORM_TALL>::NT), 0, s, f);
+                return;
+            }
         if (form == FORM_SHORT)
             hipLaunchKernelGGL((k_fused_pairs_2d<B, D, FORM_SHORT>), grid, dim3(1024), 0, s, f);
         else if (form == FORM_TALL512 && B == BC_PERIODIC)
@@ -1485,8 +1493,8 @@ static MarchCut march_cut(int dtype, const nls_member *members, int count, bool 
 }
 
 template <typename T>
-static void launch_resident(int dim, int order, int bc, bool dyn, int count, const ResidentArgs<T> &r, hipStream_t s) {
-    if (dim == 2) return launch_resident_2d<T>(order, bc, dyn, count, r, s);
+static void launch_resident(int dim, int order, int bc, bool dyn, int count, int n, const ResidentArgs<T> &r, hipStream_t s) {
+    if (dim == 2) return launch_resident_2d<T>(order, bc, dyn, count, n, r, s);
 #define NLS_CASE(O, B, D)                                                                                     \
     if (order == O && bc == B && dyn == D) {                                                                 \
         hipLaunchKernelGGL((k_resident<T, O, B, D>), dim3(count), dim3(ResShape<T>::THREADS), 0, s, r);       \
@@ -1540,7 +1548,8 @@ template <typename T> static MemberDev<T> plain_member(const nls_problem *p) {
 // a tile form is asked for (tiles step once) or the arithmetic is
 // NLS_FLAG_F64_ARITH's.
 int fused_steps_per_launch(const nls_problem *p) {
-    if (get_fused_form(p->dtype) >= 0 || (p->flags & NLS_FLAG_F64_ARITH)) return 1;
+    const bool from = p->engine == NLS_ENGINE_AUTO && p->dtype == NLS_F32 && p->n <= 64;
+    if ((!from && get_fused_form(p->dtype) >= 0) || (p->flags & NLS_FLAG_F64_ARITH)) return 1;
     return std::max(1, multi_steps(p->n, p->order, device_cus()));
 }
 
@@ -1568,7 +1577,10 @@ static int fused_grid_run(const nls_problem *p, int iters, const T *P, cplx_t<T>
     a.grid = f.grid;
     a.P = P;
     // a small grid: its own tiles, several steps a launch
-    const int many = get_fused_form(p->dtype) >= 0 ? 0 : multi_steps(p->n, p->order, device_cus());
+    // (of up to 64 points a side, in single precision: AUTO's choice instead of
+    // the resident engine, with its bits)
+    const bool from = p->engine == NLS_ENGINE_AUTO && p->dtype == NLS_F32 && p->n <= 64;
+    const int many = !from && get_fused_form(p->dtype) >= 0 ? 0 : multi_steps(p->n, p->order, device_cus());
     MultiArgs<T> b;
     memset(&b, 0, sizeof b);
     b.grid = f.grid;
@@ -1577,10 +1589,11 @@ static int fused_grid_run(const nls_problem *p, int iters, const T *P, cplx_t<T>
     T *curn = nres, *altn = dyn ? (T *)(ws + align256b(N * sizeof(C))) : nullptr;
     for (int it = 0, done; it < iters; it += done) {
         done = 1;
-        if (many && iters - it >= many) {
+        if (many && (from || iters - it >= many)) {
+            if (from) b.steps = std::min(many, iters - it);
             b.u = cur; b.un = curn; b.uo = alt; b.uno = altn;
             launch_multi<T>(p->order, p->bc, dyn, b, device_cus(), s);
-            done = many;
+            done = from ? b.steps : many;
         } else if (mg.groups) {
             a.it = it;
             a.u = cur; a.un = curn; a.uo = alt; a.uno = altn;
@@ -1679,7 +1692,7 @@ static int resident_run(const nls_problem *p, int iters, const T *P, cplx_t<T> *
     // bounded launches: each runs at most 4096 steps
     for (int done = 0; done < iters;) {
         r.iters = iters - done < 4096 ? iters - done : 4096;
-        launch_resident<T>(p->dim, p->order, p->bc, p->coeffs[10] != 0.0, 1, r, s);
+        launch_resident<T>(p->dim, p->order, p->bc, p->coeffs[10] != 0.0, 1, p->n, r, s);
         done += r.iters;
     }
     return hip_check(hipGetLastError(), "resident launch");
@@ -1776,6 +1789,7 @@ struct nls_batch {
     long long tab_total = 0;            // radial table entries (1-D reference grids)
     int min_steps = 0x7fffffff;         // smallest member step budget
     int fform = FORM_TALL;              // fused engine: tile form (fused_form)
+    int nmax = 0;                       // points per axis of the largest member
     // fused engine, marching: the pieces of the members of up to 256 points a
     // side and of the others, on the device one behind the other (strips,
     // then the workgroups' first pieces, for each)
@@ -2142,7 +2156,7 @@ static int batch_advance(nls_batch *b, int iters, const T *P, cplx_t<T> *psi, T 
         r.psi = psi;
         r.nres = nres;
         r.P = P;
-        launch_resident<T>(b->dim, b->order, b->bc, b->dyn, b->count, r, s);
+        launch_resident<T>(b->dim, b->order, b->bc, b->dyn, b->count, b->nmax, r, s);
         return hip_check(hipGetLastError(), "resident launch");
     }
     if (!batch_graphs_apply(b, iters)) return batch_steps<T>(b, 0, iters, P, psi, nres, ws, s);
@@ -2187,6 +2201,8 @@ static void plan(nls_batch *b, const nls_member *members, int count, const int *
     b->points = points;
     b->h_dx.assign(count, 0.0);
     for (int i = 0; i < count; ++i) b->h_dx[i] = members[i].dx;
+    b->nmax = 0;
+    for (int i = 0; i < count; ++i) b->nmax = std::max(b->nmax, (int)members[i].n);
     if (b->dtype == NLS_F64) fill_members<double>(b, members, ids);
     else fill_members<float>(b, members, ids);
     b->min_steps = 0x7fffffff;

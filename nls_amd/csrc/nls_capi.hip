@@ -52,16 +52,21 @@ int check_problem(const nls_problem *p) {
 // against the engines it replaced: n = 256 FP32 0.56 / 0.88 resident, n = 1000
 // radial FP32 0.59 / 3.6, n = 4096 FP64 0.67 / 6.3; longer lines took 8 to 15
 // on the per-stage kernels, 20,000 points take 0.67); in 2-D the fused engine,
-// whose small grids step several times a launch: 40^2 order 3 FP32 1.76 us per
-// step against 2.12 of one workgroup holding the grid (resident), 64^2 order 5
-// 3.0 against 5.0, 16^2 the same.  At order 7, one step a launch, the resident
-// kernel is faster up to 48^2 in single precision (4.0 against 4.7; 64^2 6.3
-// against 4.7).
+// whose small grids step several times a launch, or in single precision up to
+// small_resident points a side the resident kernel, with the same bits.  us per step,
+// launches of several steps / resident: zero-outside, order 3 32^2 1.9 / 1.3, 36^2 1.9 /
+// 2.0; order 5 32^2 2.8 / 1.6, 44^2 2.9 / 2.9; order 7 (one step a launch) 48^2 4.3 / 3.8,
+// 52^2 4.3 / 4.9; periodic, order 3 44^2 1.85 / 1.6, 48^2 1.9 / 3.1; order 5 54^2 3.15 / 3.1,
+// 56^2 3.2 / 4.9; order 7 54^2 4.9 / 4.0, 56^2 4.9 / 5.8.
+static int small_resident(int order, int bc) {
+    if (bc == NLS_BC_PERIODIC) return order == 3 ? 44 : 54;
+    return order == 3 ? 32 : order == 5 ? 44 : 48;
+}
 int plain_engine(const nls_problem *p) {
     if (p->flags & NLS_FLAG_F64_ARITH) return NLS_ENGINE_FUSED;
     if (p->engine != NLS_ENGINE_AUTO) return p->engine;
     if (p->dim == 1) return ENGINE_LINE;
-    if (p->order == 7 && p->n <= 48 && p->dtype == NLS_F32) return NLS_ENGINE_RESIDENT;
+    if (p->dtype == NLS_F32 && p->n <= small_resident(p->order, p->bc)) return NLS_ENGINE_RESIDENT;
     return fused_holds((long long)p->n * p->n, p->dtype) ? NLS_ENGINE_FUSED : NLS_ENGINE_STAGE;
 }
 

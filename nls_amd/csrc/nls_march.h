@@ -60,8 +60,9 @@ template <typename T> struct ResidentArgs {
 
 // One workgroup per member of a batch of 2-D grids of up to 64 x 64, all steps
 // of a call in one launch (nls_small.hip; not double precision of order 7).
+// n: the largest grid's side.
 template <typename T>
-void launch_resident_2d(int order, int bc, bool dyn, int count, const ResidentArgs<T> &r, hipStream_t s);
+void launch_resident_2d(int order, int bc, bool dyn, int count, int n, const ResidentArgs<T> &r, hipStream_t s);
 
 // Several steps of one small grid per launch (nls_small.hip).
 template <typename T> struct MultiArgs {
@@ -69,6 +70,8 @@ template <typename T> struct MultiArgs {
     const cplx_t<T> *u; const T *un;
     cplx_t<T> *uo; T *uno;
     const T *P;
+    int steps;                           // 0, or the steps of this launch, at most multi_steps, with
+                                         // grid_ring1_from's sums (single precision, n <= 64)
     MemberDev<T> grid;
 };
 // Steps a launch makes on an n x n grid (0: not such a grid).

@@ -45,7 +45,8 @@ template <int W, int HH, int R, int S, int WS> __device__ const StepMap<W, HH, R
 // a row) spread over the banks.
 constexpr int multi_stride(int W, int R) { return W + (R == 1 ? 2 : R == 2 ? 4 : 14); }
 
-template <typename T, int ORDER, int BC, bool DYN, int TX, int TY, int K>
+// FROM: grid_ring1_from's sums.
+template <typename T, int ORDER, int BC, bool DYN, int TX, int TY, int K, bool FROM>
 __global__ void __launch_bounds__(1024) k_multi(const MultiArgs<T> f) {
     using C = cplx_t<T>;
     constexpr int R = (ORDER - 1) / 2, NT = 1024, S = 4 * K, H = S * R;
@@ -65,6 +66,7 @@ __global__ void __launch_bounds__(1024) k_multi(const MultiArgs<T> f) {
 
     const T dt = m.dt, dt2 = dt * (T)0.5, dt6 = m.g.dt6;
     const T dtw = m.g.dtw, dtw2 = dtw * (T)0.5, dtw6 = m.g.dtw6;
+    const T dtw6lo = sixth_rest(dtw, dtw6), dt6lo = sixth_rest(dt, dt6);
     const Coeffs<T> c = m.c;
     const GridCoeffs<T> g = m.g;
 
@@ -117,7 +119,11 @@ __global__ void __launch_bounds__(1024) k_multi(const MultiArgs<T> f) {
 #pragma unroll
         for (int d = 1; d <= R; ++d) {
             const C l = rd(-d), r = rd(d), u = rd(-d * WS), b = rd(d * WS);
-            if (d == 1) {
+            if constexpr (FROM) {
+                const float q = d == 2 ? g.r2 : g.r3;
+                sr = d == 1 ? grid_ring1_from(y.x, l.x, r.x, u.x, b.x) : grid_ring_from(sr, q, y.x, l.x, r.x, u.x, b.x);
+                sm = d == 1 ? grid_ring1_from(y.y, l.y, r.y, u.y, b.y) : grid_ring_from(sm, q, y.y, l.y, r.y, u.y, b.y);
+            } else if (d == 1) {
                 sr = grid_ring1(g, l.x, r.x, u.x, b.x);
                 sm = grid_ring1(g, l.y, r.y, u.y, b.y);
             } else {
@@ -125,7 +131,7 @@ __global__ void __launch_bounds__(1024) k_multi(const MultiArgs<T> f) {
                 sm = grid_ring(sm, d == 2 ? g.r2 : g.r3, l.y, r.y, u.y, b.y);
             }
         }
-        grid_rhs<T, DYN>(g, c, cp[j], y, yn[j], mk<T>(sr, sm), k, kn);
+        grid_rhs<T, DYN, FROM>(g, c, cp[j], y, yn[j], mk<T>(sr, sm), k, kn);
     };
 
     // stage st of S: points with at least st R rings around them, a prefix of
@@ -133,6 +139,7 @@ __global__ void __launch_bounds__(1024) k_multi(const MultiArgs<T> f) {
     // its own)
 #pragma unroll
     for (int st = 1; st <= S; ++st) {
+        if (FROM && st <= 4 * (K - f.steps)) continue;      // fewer steps than K: the outer rings stay out
         const int s = (st - 1) % 4 + 1;
         const int cnt = (W - 2 * st * R) * (HH - 2 * st * R);
         int lim = cnt;
@@ -156,9 +163,15 @@ __global__ void __launch_bounds__(1024) k_multi(const MultiArgs<T> f) {
                 y = mk<T>(grid_input(uu[j].x, k.x, dtwa), grid_input(uu[j].y, k.y, dtwa));
                 if (DYN) yn[j] = grid_input(nn[j], kn, dta);
             } else {
-                y = mk<T>(grid_new(uu[j].x, acc[j].x, k.x, dtw6), grid_new(uu[j].y, acc[j].y, k.y, dtw6));
+                if constexpr (FROM) {
+                    y = mk<T>(grid_new_from(uu[j].x, acc[j].x, k.x, dtw6, dtw6lo),
+                              grid_new_from(uu[j].y, acc[j].y, k.y, dtw6, dtw6lo));
+                    if (DYN) nn[j] = yn[j] = grid_new_from(nn[j], accn[j], kn, dt6, dt6lo);
+                } else {
+                    y = mk<T>(grid_new(uu[j].x, acc[j].x, k.x, dtw6), grid_new(uu[j].y, acc[j].y, k.y, dtw6));
+                    if (DYN) nn[j] = yn[j] = grid_new(nn[j], accn[j], kn, dt6);
+                }
                 uu[j] = y;
-                if (DYN) nn[j] = yn[j] = grid_new(nn[j], accn[j], kn, dt6);
             }
             if (st < S) yout[li[j]] = y;
         }
@@ -195,13 +208,20 @@ static MultiShape multi_shape(int n, int order, int cus) {
 }
 int multi_steps(int n, int order, int cus) { return multi_shape(n, order, cus).k; }
 
-template <typename T, int O, int B, bool D, int TX, int TY, int K>
+template <typename T, int O, int B, bool D, int TX, int TY, int K, bool FROM = false>
 static void launch_multi_t(MultiArgs<T> a, hipStream_t s) {
     const int n = a.grid.n;
     a.ntx = (n + TX - 1) / TX;
-    hipLaunchKernelGGL((k_multi<T, O, B, D, TX, TY, K>), dim3(a.ntx * ((n + TY - 1) / TY)), dim3(1024), 0, s, a);
+    hipLaunchKernelGGL((k_multi<T, O, B, D, TX, TY, K, FROM>), dim3(a.ntx * ((n + TY - 1) / TY)), dim3(1024), 0, s, a);
 }
 template <typename T, int B, bool D> static void launch_multi_o(int order, const MultiArgs<T> &a, int tx, hipStream_t s) {
+    if constexpr (sizeof(T) == 4)
+        if (a.steps) {                   // up to 64 points a side: the first shapes
+            if (order == 3) launch_multi_t<T, 3, B, D, 8, 8, 4, true>(a, s);
+            else if (order == 5) launch_multi_t<T, 5, B, D, 16, 8, 2, true>(a, s);
+            else launch_multi_t<T, 7, B, D, 16, 16, 1, true>(a, s);
+            return;
+        }
     if (order == 3) {
         if (tx == 8) launch_multi_t<T, 3, B, D, 8, 8, 4>(a, s);
         else launch_multi_t<T, 3, B, D, 16, 16, 4>(a, s);
@@ -232,33 +252,37 @@ template void launch_multi<double>(int, int, bool, MultiArgs<double>, int, hipSt
 // share of 2R vertical ones, 5 a point at order 5 instead of 9, all at
 // constant offsets (rows of 64 + 2R points whatever n is, the border holding
 // zeros, or on periodic grids copies that the edge threads write).  Two
-// buffers, one barrier a stage.  The arithmetic is the fused step's.
-// Bound: vector instructions of one compute unit.  256 grids of 64^2, us per
-// step: FP32 5.96 -> 5.44 (before: one point a thread slot, 9 reads and the
-// index arithmetic a point), FP64 9.0.
+// buffers, one barrier a stage.  The arithmetic is the fused step's, in single
+// precision with grid_ring1_from's sums.
+// Bound: vector instructions of one compute unit; few grids, the latency of a
+// thread's points in turn.  256 grids of 64^2, us per step: FP32 5.96 -> 5.76, FP64
+// 9.0.  One grid, FP32, one point a thread slot with all its reads before: order 5
+// zero-outside 16^2 1.35 -> 0.93, 32^2 2.4 -> 1.6, 44^2 4.1 -> 2.9; periodic 32^2
+// 1.53 -> 1.20, 48^2 2.9 -> 2.3; with 4 points a thread whatever the size 16^2 took
+// 2.3 and 3.0.
 // ---------------------------------------------------------------------------
-template <typename T> struct SquareShape {
-    static constexpr int V = sizeof(T) == 4 ? 4 : 8, NT = 64 * (64 / V);
-};
+constexpr int square_v(int bytes) { return bytes == 4 ? 4 : 8; }      // V of 64 x 64 grids
 
-template <typename T, int ORDER, int BC, bool DYN>
-__global__ void __launch_bounds__(SquareShape<T>::NT) k_resident_2d(const ResidentArgs<T> r) {
+template <typename T, int ORDER, int BC, bool DYN, int V>
+__global__ void __launch_bounds__((V == square_v(sizeof(T)) ? 64 * 64 / V : 1024)) k_resident_2d(const ResidentArgs<T> r) {
     using C = cplx_t<T>;
-    constexpr int R = (ORDER - 1) / 2, V = SquareShape<T>::V, NT = SquareShape<T>::NT, WS = 64 + 2 * R;
+    constexpr int R = (ORDER - 1) / 2, WS = 64 + 2 * R;
     __shared__ C mem[2][WS * WS];
     const MemberDev<T> m = r.mem[blockIdx.x];
     const int n = m.n, tid = threadIdx.x;
     const int steps = min(r.iters, m.steps);
-    if (n > 64 || steps <= 0) return;    // (the host plans no larger grid)
+    // (the host plans no larger grid, nor one with more strips than threads)
+    if (n > 64 || n * ((n + V - 1) / V) > (int)blockDim.x || steps <= 0) return;
     C *psi = r.psi + m.off;
     T *nres = DYN ? r.nres + m.off : nullptr;
     const T *P = r.P + m.off;
     const T dt = m.dt, dt2 = dt * (T)0.5, dt6 = m.g.dt6;
     const T dtw = m.g.dtw, dtw2 = dtw * (T)0.5, dtw6 = m.g.dtw6;
+    const T dtw6lo = sixth_rest(dtw, dtw6), dt6lo = sixth_rest(dt, dt6);
     const Coeffs<T> c = m.c;
     const GridCoeffs<T> g = m.g;
 
-    for (int i = tid; i < WS * WS; i += NT) mem[0][i] = mem[1][i] = mk<T>(0, 0);
+    for (int i = tid; i < WS * WS; i += blockDim.x) mem[0][i] = mem[1][i] = mk<T>(0, 0);
     __syncthreads();
 
     const int strip = tid / n, col = tid - strip * n, r0 = strip * V;
@@ -272,11 +296,30 @@ __global__ void __launch_bounds__(SquareShape<T>::NT) k_resident_2d(const Reside
     // KEEP: the thread's own stage inputs stay in registers; double precision
     // has none to spare and reads its column from LDS as it goes down
     constexpr bool KEEP = sizeof(T) == 4;
+    // WRAP: few points a thread of a periodic grid read their neighbours from the
+    // places they wrap to, held in registers, and nothing is copied
+    constexpr bool WRAP = BC == BC_PERIODIC && V < square_v(sizeof(T));
+    int ry[WRAP ? V + 2 * R : 1], hx[WRAP ? V : 1][2 * R];
+    if constexpr (WRAP) {
+        auto at = [&](int y, int x) {        // (narrow grids wrap more than once)
+            return (wrap_index(y, n) + R) * WS + wrap_index(x, n) + R;
+        };
+#pragma unroll
+        for (int d = 0; d < V + 2 * R; ++d) ry[d] = at(r0 - R + d, col);
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+#pragma unroll
+            for (int d = 1; d <= R; ++d) {
+                hx[v][d - 1] = at(r0 + v, col - d);
+                hx[v][R + d - 1] = at(r0 + v, col + d);
+            }
+    }
     C u[V], y[KEEP ? V : 1], acc[V];
     T cp[V], un[V], yn[V], accn[V];
     // copies of the thread's points, just written to out, across the border
     auto copy_edges = [&](C *out) {
-        if constexpr (KEEP) {
+        if constexpr (WRAP) {
+        } else if constexpr (KEEP) {
 #pragma unroll
             for (int v = 0; v < V; ++v) {
                 if (v >= rows) continue;
@@ -320,7 +363,13 @@ __global__ void __launch_bounds__(SquareShape<T>::NT) k_resident_2d(const Reside
             unsigned a = (unsigned)(size_t)((LV *)mem[(s - 1) & 1] + (li - R * WS - R));
             asm volatile("" : "+v"(a));
             LV *in = (LV *)(size_t)a;
-            auto rd = [&](int row, int x) { const V2 z = in[(row + R) * WS + x + R]; return mk<T>(z.x, z.y); };
+            LV *const whole = (LV *)mem[(s - 1) & 1];
+            auto rd = [&](int row, int x) {
+                V2 z;
+                if constexpr (WRAP) z = whole[x == 0 ? ry[row + R] : hx[row][x < 0 ? -x - 1 : R + x - 1]];
+                else z = in[(row + R) * WS + x + R];
+                return mk<T>(z.x, z.y);
+            };
             C *const out = mem[s & 1];
             // the column from R above to R below (past the last row of a
             // short strip the rows read are the grid's next, or its border)
@@ -343,7 +392,14 @@ __global__ void __launch_bounds__(SquareShape<T>::NT) k_resident_2d(const Reside
 #pragma unroll
                 for (int d = 1; d <= R; ++d) {
                     const C l = rd(v, -d), q = rd(v, d), up = w[R + v - d], dn = w[R + v + d];
-                    if (d == 1) {
+                    if constexpr (KEEP) {
+                        const C &y0 = w[R + v];
+                        const float rt = d == 2 ? g.r2 : g.r3;
+                        sr = d == 1 ? grid_ring1_from(y0.x, l.x, q.x, up.x, dn.x)
+                                    : grid_ring_from(sr, rt, y0.x, l.x, q.x, up.x, dn.x);
+                        sm = d == 1 ? grid_ring1_from(y0.y, l.y, q.y, up.y, dn.y)
+                                    : grid_ring_from(sm, rt, y0.y, l.y, q.y, up.y, dn.y);
+                    } else if (d == 1) {
                         sr = grid_ring1(g, l.x, q.x, up.x, dn.x);
                         sm = grid_ring1(g, l.y, q.y, up.y, dn.y);
                     } else {
@@ -353,7 +409,7 @@ __global__ void __launch_bounds__(SquareShape<T>::NT) k_resident_2d(const Reside
                 }
                 C k;
                 T kn;
-                grid_rhs<T, DYN>(g, c, cp[v], w[R + v], yn[v], mk<T>(sr, sm), k, kn);
+                grid_rhs<T, DYN, KEEP>(g, c, cp[v], w[R + v], yn[v], mk<T>(sr, sm), k, kn);
                 C z;
                 if (s < 4) {
                     grid_acc(acc[v].x, k.x, s == 1);
@@ -362,9 +418,15 @@ __global__ void __launch_bounds__(SquareShape<T>::NT) k_resident_2d(const Reside
                     z = mk<T>(grid_input(u[v].x, k.x, dtwa), grid_input(u[v].y, k.y, dtwa));
                     if (DYN) yn[v] = grid_input(un[v], kn, dta);
                 } else {
-                    z = mk<T>(grid_new(u[v].x, acc[v].x, k.x, dtw6), grid_new(u[v].y, acc[v].y, k.y, dtw6));
+                    if constexpr (KEEP) {
+                        z = mk<T>(grid_new_from(u[v].x, acc[v].x, k.x, dtw6, dtw6lo),
+                                  grid_new_from(u[v].y, acc[v].y, k.y, dtw6, dtw6lo));
+                        if (DYN) un[v] = yn[v] = grid_new_from(un[v], accn[v], kn, dt6, dt6lo);
+                    } else {
+                        z = mk<T>(grid_new(u[v].x, acc[v].x, k.x, dtw6), grid_new(u[v].y, acc[v].y, k.y, dtw6));
+                        if (DYN) un[v] = yn[v] = grid_new(un[v], accn[v], kn, dt6);
+                    }
                     u[v] = z;
-                    if (DYN) un[v] = yn[v] = grid_new(un[v], accn[v], kn, dt6);
                 }
                 if (KEEP) y[KEEP ? v : 0] = z;
                 if (v < rows) out[li + v * WS] = z;
@@ -390,11 +452,22 @@ __global__ void __launch_bounds__(SquareShape<T>::NT) k_resident_2d(const Reside
         }
 }
 
+// Points a thread of grids of up to n x n: as few as 1024 threads hold, for
+// the shortest step, while every CU has at most one grid (256 of 40^2 FP32 2.4 us a
+// step); V of the largest beyond, whose shared column costs less (512 of them
+// 7.1).  Three points in double precision would spill.
 template <typename T>
-void launch_resident_2d(int order, int bc, bool dyn, int count, const ResidentArgs<T> &r, hipStream_t s) {
+void launch_resident_2d(int order, int bc, bool dyn, int count, int n, const ResidentArgs<T> &r, hipStream_t s) {
+    constexpr int VM = square_v(sizeof(T));
+    const bool few = count <= device_cus();
+    const int v = !few ? VM : n * n <= 1024 ? 1 : n * ((n + 1) / 2) <= 1024 ? 2 : VM == 4 && n * ((n + 2) / 3) <= 1024 ? 3 : VM;
+    const int nt = v == VM ? 64 * 64 / VM : (n * ((n + v - 1) / v) + 63) / 64 * 64;
 #define NLS_CASE(O, B, D)                                                                                        \
     if (order == O && bc == B && dyn == D) {                                                                     \
-        hipLaunchKernelGGL((k_resident_2d<T, O, B, D>), dim3(count), dim3(SquareShape<T>::NT), 0, s, r);          \
+        if (v == 1) hipLaunchKernelGGL((k_resident_2d<T, O, B, D, 1>), dim3(count), dim3(nt), 0, s, r);          \
+        else if (v == 2) hipLaunchKernelGGL((k_resident_2d<T, O, B, D, 2>), dim3(count), dim3(nt), 0, s, r);     \
+        else if (VM == 4 && v == 3) hipLaunchKernelGGL((k_resident_2d<T, O, B, D, VM == 4 ? 3 : VM>), dim3(count), dim3(nt), 0, s, r);     \
+        else hipLaunchKernelGGL((k_resident_2d<T, O, B, D, VM>), dim3(count), dim3(nt), 0, s, r);                \
         return;                                                                                                  \
     }
     NLS_CASE(3, 0, false) NLS_CASE(3, 0, true) NLS_CASE(3, 1, false) NLS_CASE(3, 1, true)
@@ -404,7 +477,7 @@ void launch_resident_2d(int order, int bc, bool dyn, int count, const ResidentAr
     }
 #undef NLS_CASE
 }
-template void launch_resident_2d<float>(int, int, bool, int, const ResidentArgs<float> &, hipStream_t);
-template void launch_resident_2d<double>(int, int, bool, int, const ResidentArgs<double> &, hipStream_t);
+template void launch_resident_2d<float>(int, int, bool, int, int, const ResidentArgs<float> &, hipStream_t);
+template void launch_resident_2d<double>(int, int, bool, int, int, const ResidentArgs<double> &, hipStream_t);
 
 }  // namespace nls
