@@ -574,13 +574,16 @@ def main():
         fused_points = points if engine == "fused" else sum(m.points for m in members if m.n * m.n > 4096)
         bytes_per_launch = fused_points * FUSED_BYTES_F32_DYN
         achieved = bytes_per_launch / launch_s
-        prof = ("fused_step_f32_sweep512_traffic.txt" if engine == "fused" else
-                "fused_step_f32_sweep512_hybrid_traffic.txt")
+        # its form: marching strips unless a tile form was asked for or won the tuning
+        march = native.fused_form("f32") == "auto"
+        prof = ("%s_step_f32_sweep512_traffic.txt" if engine == "fused" else
+                "%s_step_f32_sweep512_hybrid_traffic.txt") % ("march" if march else "fused")
         traffic = read_profile_value(prof, "traffic_bytes_per_launch")
         valu_per_point = read_profile_value(prof, "valu_lane_insts_per_point_step")
         roofline = {"bound": "valu", "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                     "frac": achieved / HBM_PEAK, "traffic": traffic,
-                    "kernel": "k_fused_pairs_2d<periodic,dynamic> (float, order 5)", "kernel_points": fused_points,
+                    "kernel": ("k_march<dynamic,whole rows> (float)" if march else
+                               "k_fused_pairs_2d<periodic,dynamic> (float, order 5)"), "kernel_points": fused_points,
                     "algorithmic_bytes_per_launch": bytes_per_launch, "avg_launch_us": launch_s * 1e6,
                     "note": "achieved/peak/frac: the HBM roofline of the algorithmic bytes (secondary); the "
                             "kernel's limiter is its vector ALU work (valu)"}

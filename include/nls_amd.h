@@ -58,13 +58,16 @@ extern "C" {
 /* RK4 engines (nls_problem.engine, nls_batch_create) */
 #define NLS_ENGINE_AUTO  -1   /* a plain 1-D solve: pieces of the line held in
                                  registers, many steps per launch; 2-D:
-                                 RESIDENT if the instance fits, else FUSED.
+                                 FUSED (in single precision up to 32 to 54
+                                 points a side, by order and boundary:
+                                 RESIDENT).
                                  Batches: RESIDENT if every member fits, else
                                  FUSED for 2-D and STAGE for 1-D, HYBRID if
                                  only some members fit                       */
 #define NLS_ENGINE_STAGE  0   /* one launch per RK4 stage                    */
-#define NLS_ENGINE_FUSED  1   /* one launch per RK4 step, halo recomputed on
-                                 chip (2-D only)                             */
+#define NLS_ENGINE_FUSED  1   /* one launch per RK4 step (several steps on
+                                 small grids), halo recomputed on chip (2-D
+                                 only)                                       */
 #define NLS_ENGINE_RESIDENT 2 /* a workgroup per instance holds its grid on
                                  chip and runs a block of steps per launch
                                  (1-D n <= 4096, 2-D n <= 64; not FP64 2-D
@@ -195,7 +198,7 @@ size_t nls_workspace_bytes(const nls_problem *p);
  * returns; the caller synchronises the stream.
  * Solves of at least 128 steps on the fused or per-stage engine replay a
  * captured block of 64 steps as one hipGraph launch (unless
- * NLS_FLAG_EAGER): the graph is captured on a private stream of the calling
+ * NLS_FLAG_EAGER, or where a launch makes several steps): the graph is captured on a private stream of the calling
  * thread, cached per thread by device, problem and buffer addresses (up to 8
  * entries), and launched on `stream`. */
 int nls_advance(const nls_problem *p, int iters, const void *pumping, void *psi, void *nres,
@@ -250,9 +253,9 @@ int nls_tune_stage_tile(int dtype, int rows);
 /* Tile form of the fused RK4 kernel for dtype: 0 chooses per launch (the
  * default: order-5 periodic launches that fill the device march down strips of
  * columns, others take the tile form that suits their tile counts), 1 = 64 x 32 tiles
- * of 1024 threads (64 x 16 at order 7), 2 = 64 x 16 tiles of 1024 threads,
+ * of 1024 threads (64 x 24 of 768 at order 7), 2 = 64 x 16 tiles of 1024 threads,
  * 3 = 64 x 16 tiles of 512 threads with one stage buffer (double precision
- * on periodic grids; elsewhere it runs as 1), 4 = 64 x 32 tiles of 512
+ * on periodic grids, not of order 7; elsewhere it runs as 1), 4 = 64 x 32 tiles of 512
  * threads (single precision, order 5, periodic grids; elsewhere it runs as
  * 1); form = -1 only queries.
  * Returns the setting in effect or a negative NLS_E* code.  Process-wide; a

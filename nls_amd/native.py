@@ -70,8 +70,8 @@ class ProblemDesc(C.Structure):
     def make(cls, dim, n, order, dt, dx, coeffs, bc="ref", dtype="f32", scheme="rk4", engine="auto",
              graphs=True, f64_arith=False):
         """engine: RK4 engine of a plain solve -- "auto" (1-D: pieces of the
-        line in registers, many steps per launch; 2-D: resident when the
-        instance fits on chip, else fused), "stage" (one launch per RK4 stage), "fused" (one launch per step,
+        line in registers, many steps per launch; 2-D: fused, the smallest
+        single-precision grids resident), "stage" (one launch per RK4 stage), "fused" (one launch per step,
         2-D only) or "resident" (1-D n <= 4096, 2-D n <= 64).  graphs=False
         sets NLS_FLAG_EAGER: no step-block graph replay.  f64_arith=True
         sets NLS_FLAG_F64_ARITH: a single-precision 2-D periodic problem
