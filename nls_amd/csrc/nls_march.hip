@@ -194,7 +194,11 @@ __device__ __forceinline__ void march_piece(const MarchArgs<T> &f, const StripDe
             if constexpr (AHEAD && S >= 2) h2 = beside(k, 1);
             fence();
             const T yn = nn[(k + U - 2) % U];
-            slopes(h1, u1(4), u1(3), u1(2), u1(1), u1(0), cp[(k + U - 2) % U], yn, kk, kn);
+            // the row's pumping becomes its pump term at its first use, two
+            // rows after its load
+            T &cP = cp[(k + U - 2) % U];
+            cP = pump_term<T, DYN>(c, cP);
+            slopes(h1, u1(4), u1(3), u1(2), u1(1), u1(0), cP, yn, kk, kn);
             m5(w2, 2) = mk<T>(grid_input(u1(2).x, kk.x, dtw2), grid_input(u1(2).y, kk.y, dtw2));
             C acc = a1[now];
             T bcc = b1[now], old = DYN ? grid_input(nn[(k + U - 4) % U], bcc, dt2) : (T)0;
