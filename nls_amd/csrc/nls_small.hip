@@ -255,16 +255,18 @@ template void launch_multi<double>(int, int, bool, MultiArgs<double>, int, hipSt
 // buffers, one barrier a stage.  The arithmetic is the fused step's, in single
 // precision with grid_ring1_from's sums.
 // Bound: vector instructions of one compute unit; few grids, the latency of a
-// thread's points in turn.  256 grids of 64^2, us per step: FP32 5.96 -> 5.76, FP64
-// 9.0.  One grid, FP32, one point a thread slot with all its reads before: order 5
-// zero-outside 16^2 1.35 -> 0.93, 32^2 2.4 -> 1.6, 44^2 4.1 -> 2.9; periodic 32^2
-// 1.53 -> 1.20, 48^2 2.9 -> 2.3; with 4 points a thread whatever the size 16^2 took
-// 2.3 and 3.0.
+// thread's points in turn.  us per step, order 5, one point a thread slot with all
+// its reads -> strips: FP32, one grid, zero-outside 16^2 1.46 -> 0.98, 32^2 2.2 -> 1.65,
+// 64^2 7.5 -> 5.2; periodic 32^2 1.8 -> 1.5, 48^2 3.6 -> 3.2, 56^2 4.7 -> 4.8, dynamic
+// 64^2 5.1 -> 4.9; 1000 grids of 16^2 periodic 4.5 -> 2.0.  FP64, one grid, zero-outside
+// 64^2 14.8 -> 7.9, periodic 48^2 6.6 -> 6.0, 64^2 10.9 -> 9.0; 1000 of 16^2 8.9 -> 4.2.
+// Behind are periodic algebraic grids of 33 to 36 points (33^2 order 7 2.8 -> 3.3), where
+// strips of two points fill nine waves, so that one SIMD steps three of them.
 // ---------------------------------------------------------------------------
 constexpr int square_v(int bytes) { return bytes == 4 ? 4 : 8; }      // V of 64 x 64 grids
 
 template <typename T, int ORDER, int BC, bool DYN, int V>
-__global__ void __launch_bounds__((V == square_v(sizeof(T)) ? 64 * 64 / V : 1024)) k_resident_2d(const ResidentArgs<T> r) {
+__global__ void __launch_bounds__((V > 4 ? 512 : 1024)) k_resident_2d(const ResidentArgs<T> r) {
     using C = cplx_t<T>;
     constexpr int R = (ORDER - 1) / 2, WS = 64 + 2 * R;
     __shared__ C mem[2][WS * WS];
@@ -282,9 +284,6 @@ __global__ void __launch_bounds__((V == square_v(sizeof(T)) ? 64 * 64 / V : 1024
     const Coeffs<T> c = m.c;
     const GridCoeffs<T> g = m.g;
 
-    for (int i = tid; i < WS * WS; i += blockDim.x) mem[0][i] = mem[1][i] = mk<T>(0, 0);
-    __syncthreads();
-
     const int strip = tid / n, col = tid - strip * n, r0 = strip * V;
     const int rows = min(V, n - r0);     // points of this thread; none if <= 0
     const int li = (r0 + R) * WS + col + R;
@@ -296,13 +295,16 @@ __global__ void __launch_bounds__((V == square_v(sizeof(T)) ? 64 * 64 / V : 1024
     // KEEP: the thread's own stage inputs stay in registers; double precision
     // has none to spare and reads its column from LDS as it goes down
     constexpr bool KEEP = sizeof(T) == 4;
-    // WRAP: few points a thread of a periodic grid read their neighbours from the
-    // places they wrap to, held in registers, and nothing is copied
-    constexpr bool WRAP = BC == BC_PERIODIC && V < square_v(sizeof(T));
-    int ry[WRAP ? V + 2 * R : 1], hx[WRAP ? V : 1][2 * R];
+    // WRAP: the points of a periodic grid read their neighbours from the places they
+    // wrap to, held in registers, and nothing is copied (56^2 FP32 6.2 -> 4.8 us a
+    // step); eight points in double precision with a reservoir would spill
+    constexpr bool WRAP = BC == BC_PERIODIC && (V < 8 || !DYN);
+    unsigned ry[WRAP ? V + 2 * R : 1], hx[WRAP ? V : 1][2 * R];     // LDS byte addresses in the first buffer
+    typedef T V2 __attribute__((ext_vector_type(2)));
+    using LV = __attribute__((address_space(3))) const V2;
     if constexpr (WRAP) {
-        auto at = [&](int y, int x) {        // (narrow grids wrap more than once)
-            return (wrap_index(y, n) + R) * WS + wrap_index(x, n) + R;
+        auto at = [&](int y, int x) {
+            return (unsigned)(size_t)((LV *)mem[0] + (wrap_near(y, n) + R) * WS + wrap_near(x, n) + R);
         };
 #pragma unroll
         for (int d = 0; d < V + 2 * R; ++d) ry[d] = at(r0 - R + d, col);
@@ -313,6 +315,10 @@ __global__ void __launch_bounds__((V == square_v(sizeof(T)) ? 64 * 64 / V : 1024
                 hx[v][d - 1] = at(r0 + v, col - d);
                 hx[v][R + d - 1] = at(r0 + v, col + d);
             }
+    }
+    if constexpr (!WRAP) {               // the border
+        for (int i = tid; i < WS * WS; i += blockDim.x) mem[0][i] = mem[1][i] = mk<T>(0, 0);
+        __syncthreads();
     }
     C u[V], y[KEEP ? V : 1], acc[V];
     T cp[V], un[V], yn[V], accn[V];
@@ -354,8 +360,6 @@ __global__ void __launch_bounds__((V == square_v(sizeof(T)) ? 64 * 64 / V : 1024
     if (rows > 0) copy_edges(mem[0]);
     __syncthreads();
 
-    typedef T V2 __attribute__((ext_vector_type(2)));
-    using LV = __attribute__((address_space(3))) const V2;
     auto stage = [&](auto s_) {
         constexpr int s = decltype(s_)::value;
         const T dta = s == 3 ? dt : dt2, dtwa = s == 3 ? dtw : dtw2;
@@ -363,10 +367,11 @@ __global__ void __launch_bounds__((V == square_v(sizeof(T)) ? 64 * 64 / V : 1024
             unsigned a = (unsigned)(size_t)((LV *)mem[(s - 1) & 1] + (li - R * WS - R));
             asm volatile("" : "+v"(a));
             LV *in = (LV *)(size_t)a;
-            LV *const whole = (LV *)mem[(s - 1) & 1];
             auto rd = [&](int row, int x) {
                 V2 z;
-                if constexpr (WRAP) z = whole[x == 0 ? ry[row + R] : hx[row][x < 0 ? -x - 1 : R + x - 1]];
+                if constexpr (WRAP)
+                    z = *(LV *)(size_t)((x == 0 ? ry[row + R] : hx[row][x < 0 ? -x - 1 : R + x - 1]) +
+                                        (s - 1) % 2 * (unsigned)sizeof(mem[0]));
                 else z = in[(row + R) * WS + x + R];
                 return mk<T>(z.x, z.y);
             };
@@ -452,23 +457,33 @@ __global__ void __launch_bounds__((V == square_v(sizeof(T)) ? 64 * 64 / V : 1024
         }
 }
 
-// Points a thread of grids of up to n x n: as few as 1024 threads hold, for
-// the shortest step, while every CU has at most one grid (256 of 40^2 FP32 2.4 us a
-// step); V of the largest beyond, whose shared column costs less (512 of them
-// 7.1).  Three points in double precision would spill.
+// Points a thread of grids of up to n x n: as few as 1024 threads hold in single
+// precision, in double 512 (256 registers; three and four points of 1024 threads
+// would spill, and with 8 whatever the size 48^2 took 9.8 us a step instead of 6.0).
+// A step's length is the points a thread times the waves of a SIMD, and small
+// grids keep it short for each of many as for one: with V of the largest for more
+// grids than CUs, 1000 grids of 16^2 FP32 took 12.3 us a step instead of 2.0.  Only
+// zero-outside FP32 grids of more than 48 points do better so: two workgroups of V = 4
+// share a CU's registers, those of 3 do not (300 of 52^2 8.2 -> 7.3, 300 of 48^2 6.7
+// against 5.0).
 template <typename T>
 void launch_resident_2d(int order, int bc, bool dyn, int count, int n, const ResidentArgs<T> &r, hipStream_t s) {
     constexpr int VM = square_v(sizeof(T));
-    const bool few = count <= device_cus();
-    const int v = !few ? VM : n * n <= 1024 ? 1 : n * ((n + 1) / 2) <= 1024 ? 2 : VM == 4 && n * ((n + 2) / 3) <= 1024 ? 3 : VM;
-    const int nt = v == VM ? 64 * 64 / VM : (n * ((n + v - 1) / v) + 63) / 64 * 64;
-#define NLS_CASE(O, B, D)                                                                                        \
-    if (order == O && bc == B && dyn == D) {                                                                     \
-        if (v == 1) hipLaunchKernelGGL((k_resident_2d<T, O, B, D, 1>), dim3(count), dim3(nt), 0, s, r);          \
-        else if (v == 2) hipLaunchKernelGGL((k_resident_2d<T, O, B, D, 2>), dim3(count), dim3(nt), 0, s, r);     \
-        else if (VM == 4 && v == 3) hipLaunchKernelGGL((k_resident_2d<T, O, B, D, VM == 4 ? 3 : VM>), dim3(count), dim3(nt), 0, s, r);     \
-        else hipLaunchKernelGGL((k_resident_2d<T, O, B, D, VM>), dim3(count), dim3(nt), 0, s, r);                \
-        return;                                                                                                  \
+    auto strips = [&](int v) { return n * ((n + v - 1) / v); };
+    int v = strips(1) <= 1024 ? 1 : strips(2) <= 1024 ? 2 : VM;
+    if (sizeof(T) == 8 && v == VM) v = strips(5) <= 512 ? 5 : strips(6) <= 512 ? 6 : VM;
+    if (sizeof(T) == 4 && v == VM && strips(3) <= 1024) v = 3;
+    if (sizeof(T) == 4 && bc == NLS_BC_REF && n > 48 && count > device_cus()) v = VM;
+    const int nt = v == VM ? 64 * 64 / VM : (strips(v) + 63) / 64 * 64;
+#define NLS_V(O, B, D, V) \
+    if (v == V) hipLaunchKernelGGL((k_resident_2d<T, O, B, D, V>), dim3(count), dim3(nt), 0, s, r);
+#define NLS_CASE(O, B, D)                                  \
+    if (order == O && bc == B && dyn == D) {               \
+        NLS_V(O, B, D, 1) NLS_V(O, B, D, 2)                \
+        NLS_V(O, B, D, VM)                                 \
+        if constexpr (sizeof(T) == 4) { NLS_V(O, B, D, 3) } \
+        else { NLS_V(O, B, D, 5) NLS_V(O, B, D, 6) }       \
+        return;                                            \
     }
     NLS_CASE(3, 0, false) NLS_CASE(3, 0, true) NLS_CASE(3, 1, false) NLS_CASE(3, 1, true)
     NLS_CASE(5, 0, false) NLS_CASE(5, 0, true) NLS_CASE(5, 1, false) NLS_CASE(5, 1, true)
@@ -476,6 +491,7 @@ void launch_resident_2d(int order, int bc, bool dyn, int count, int n, const Res
         NLS_CASE(7, 0, false) NLS_CASE(7, 0, true) NLS_CASE(7, 1, false) NLS_CASE(7, 1, true)
     }
 #undef NLS_CASE
+#undef NLS_V
 }
 template void launch_resident_2d<float>(int, int, bool, int, int, const ResidentArgs<float> &, hipStream_t);
 template void launch_resident_2d<double>(int, int, bool, int, int, const ResidentArgs<double> &, hipStream_t);
