@@ -1608,12 +1608,7 @@ static int fused_grid_run(const nls_problem *p, int iters, const T *P, cplx_t<T>
     }
     int rc = hip_check(hipGetLastError(), "fused step launch");
     if (rc) return rc;
-    if (cur != psi) {
-        rc = hip_check(hipMemcpyAsync(psi, cur, N * sizeof(C), hipMemcpyDeviceToDevice, s), "copy state");
-        if (rc) return rc;
-        if (dyn) rc = hip_check(hipMemcpyAsync(nres, curn, N * sizeof(T), hipMemcpyDeviceToDevice, s), "copy reservoir");
-    }
-    return rc;
+    return cur == psi ? rc : copy_state<T>(N, cur, psi, dyn ? curn : nullptr, dyn ? nres : nullptr, s);
 }
 
 // One RK4 step of one row slab of a grid periodic along its rows (BC_SLAB):

@@ -216,7 +216,8 @@ static int wave_points(int order, int q) { return 64 * q - 4 * (order - 1); }
 
 // The plan with the least estimated time for `iters` steps, from what the
 // kernel measured (MI355X, us; FP32 and FP64, algebraic and dynamic alike
-// within 15%): a launch costs 2.0 beside its steps, a step 0.16 for the LDS
+// within 15%): a launch costs 2.0 beside its steps, a copy back from the workspace
+// (chunks whose launches cannot be even) as much, a step 0.16 for the LDS
 // round trip, the barrier and the latency of its four stages and 0.26 for
 // each point a SIMD's lane steps (points a lane x waves on the SIMD).  So few
 // points a lane and a wave on every SIMD are worth more than little overlap:
@@ -233,14 +234,15 @@ static LinePlan line_plan(const nls_problem *p, int iters, int cus) {
     auto consider = [&](int q, int nw, int k, int B) {
         const double blocks = B ? (p->n + B - 1) / B : 1, launches = (iters + k - 1) / k;
         const double waves = (nw + 3) / 4 * ceil(blocks / cus);
-        const double t = launches * LAUNCH + iters * (STEP + POINT * q * waves);
+        const bool copy = B && (int)launches % 2 && iters <= launches;
+        const double t = (launches + copy) * LAUNCH + iters * (STEP + POINT * q * waves);
         if (least < 0 || t < least) { least = t; best = LinePlan{q, nw, k, B}; }
     };
     for (int q = 1; q <= 4; q *= 2) {
         const int S = wave_points(p->order, q);
         const int nw = (p->n + S - 1) / S;
         if (nw <= LINE_WAVES) consider(q, nw, 4096, 0);
-        for (int k = 1; k <= 64; ++k)
+        for (int k = 1; k <= std::min(iters, 64); ++k)
             for (int w = 4; w <= LINE_WAVES; w += 4) {
                 const int B = w * S - 2 * H * (k - 1);
                 if (B >= 16) consider(q, w, k, B);
@@ -289,12 +291,7 @@ static int line_run(const nls_problem *p, const LinePlan &pl, int iters, const T
     }
     int rc = hip_check(hipGetLastError(), "line launch");
     if (rc) return rc;
-    if (cur != psi) {
-        rc = hip_check(hipMemcpyAsync(psi, cur, n * sizeof(C), hipMemcpyDeviceToDevice, s), "copy state");
-        if (rc) return rc;
-        if (dyn) rc = hip_check(hipMemcpyAsync(nres, curn, n * sizeof(T), hipMemcpyDeviceToDevice, s), "copy reservoir");
-    }
-    return rc;
+    return cur == psi ? rc : copy_state<T>(n, cur, psi, dyn ? curn : nullptr, dyn ? nres : nullptr, s);
 }
 
 size_t line_workspace_bytes(const nls_problem *p) {

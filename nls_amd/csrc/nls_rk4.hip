@@ -5,6 +5,7 @@
 // reservoir.  2-D: one 64 x 16 tile per workgroup; 1-D: 256 points.
 #include <atomic>
 
+#include "nls_internal.h"
 #include "nls_rk4.h"
 
 namespace nls {
@@ -106,5 +107,27 @@ template void launch_rk4_stage<float>(int, int, int, bool, const StageArgs<float
 template void launch_rk4_stage<double>(int, int, int, bool, const StageArgs<double> &, hipStream_t);
 template void launch_radial_table<float>(int, int, double, float *, hipStream_t);
 template void launch_radial_table<double>(int, int, double, double *, hipStream_t);
+
+template <typename T>
+__global__ void __launch_bounds__(256) k_copy_state(int N, const cplx_t<T> *src, cplx_t<T> *dst, const T *srcn, T *dstn) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= N) return;
+    dst[i] = src[i];
+    if (dstn) dstn[i] = srcn[i];
+}
+
+template <typename T>
+int copy_state(size_t N, const cplx_t<T> *src, cplx_t<T> *dst, const T *srcn, T *dstn, hipStream_t s) {
+    if (N <= COPY_POINTS) {
+        hipLaunchKernelGGL((k_copy_state<T>), dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, (int)N, src, dst, srcn,
+                           dstn);
+        return hip_check(hipGetLastError(), "copy launch");
+    }
+    int rc = hip_check(hipMemcpyAsync(dst, src, N * sizeof(cplx_t<T>), hipMemcpyDeviceToDevice, s), "copy state");
+    if (!rc && dstn) rc = hip_check(hipMemcpyAsync(dstn, srcn, N * sizeof(T), hipMemcpyDeviceToDevice, s), "copy reservoir");
+    return rc;
+}
+template int copy_state<float>(size_t, const float2 *, float2 *, const float *, float *, hipStream_t);
+template int copy_state<double>(size_t, const double2 *, double2 *, const double *, double *, hipStream_t);
 
 }  // namespace nls
