@@ -215,25 +215,38 @@ __device__ __forceinline__ void stage_tile_1d(const StageArgs<T> &a, int x0, cpl
     constexpr int R = (ORDER - 1) / 2;
     constexpr int LW = TILE1 + 2 * R;
     const int n = a.n, st = a.stage;
-    const LineStep<T> h = line_step(a.dt);
-    // stage input u + k_prev (dt/2, dt/2, dt)
-    auto input = [&](T u, T k) {
-        T unused = 0;
-        return st == 1 ? u : st == 4 ? line_combine<T, 3>(unused, k, u, h)
-                                     : line_combine<T, 1>(unused, k, u, h);
-    };
+    // stage input u + k_prev (dt/2, dt/2, dt), both factors exact
+    const T step = a.dt * a.scale;
+    auto input = [&](T u, T k) { return st == 1 ? u : fma(k, step, u); };
+    // the own point's fields, in flight while the tile is filled; base: the
+    // accumulator before this stage
+    const int gx = x0 + threadIdx.x;
+    const size_t gi = (size_t)min(gx, n - 1);
+    const cplx_t<T> *const base = st == 2 ? a.kin : a.acc;
+    const T *const base_n = st == 2 ? a.kin_n : a.acc_n;
+    const cplx_t<T> u = a.u[gi];
+    const T P = a.P[gi];
+    cplx_t<T> acc = mk<T>(0, 0);
+    T un = 0, kin_n = 0, accn = 0;
+    if (DYN) un = a.un[gi];
+    if (st != 1) {
+        acc = base[gi];
+        if (DYN) { kin_n = a.kin_n[gi]; accn = base_n[gi]; }
+    }
     for (int idx = threadIdx.x; idx < LW; idx += TILE1) {
-        int gx = x0 + idx - R;
-        if (BC == BC_PERIODIC) gx = wrap_index(gx, n);
+        int g = x0 + idx - R;
+        if (BC == BC_PERIODIC) g = wrap_index(g, n);
         cplx_t<T> y = mk<T>(0, 0);
-        if (gx >= 0 && gx < n) {
-            const cplx_t<T> u = a.u[gx], k = st == 1 ? mk<T>(0, 0) : a.kin[gx];
-            y = mk<T>(input(u.x, k.x), input(u.y, k.y));
+        if (BC == BC_PERIODIC || (g >= 0 && g < n)) {
+            y = a.u[g];
+            if (st != 1) {
+                const cplx_t<T> k = a.kin[g];
+                y = mk<T>(input(y.x, k.x), input(y.y, k.y));
+            }
         }
         tile[idx] = y;
     }
     __syncthreads();
-    const int gx = x0 + threadIdx.x;
     if (gx >= n) return;
     const int l = threadIdx.x + R;
     T ex[2 * R + 1], ey[2 * R + 1];
@@ -255,22 +268,15 @@ __device__ __forceinline__ void stage_tile_1d(const StageArgs<T> &a, int x0, cpl
         lr = line_lap_row<T, R>(w, ex + R);
         li = line_lap_row<T, R>(w, ey + R);
     }
-    const size_t gi = (size_t)gx;
-    const cplx_t<T> u = a.u[gi];
-    cplx_t<T> acc = st == 1 ? mk<T>(0, 0) : st == 2 ? a.kin[gi] : a.acc[gi];
-    T un = 0, kin_n = 0, accn = 0;
-    if (DYN) {
-        un = a.un[gi];
-        kin_n = st == 1 ? (T)0 : a.kin_n[gi];
-        accn = st == 1 ? (T)0 : st == 2 ? kin_n : a.acc_n[gi];
-    }
     cplx_t<T> k;
     T kn = 0;
-    line_rhs<T, DYN>(a.c, pump_term<T, DYN>(a.c, a.P[gi]), mk<T>(ex[R], ey[R]), input(un, kin_n), lr, li, k, kn);
+    line_rhs<T, DYN>(a.c, pump_term<T, DYN>(a.c, P), mk<T>(ex[R], ey[R]), input(un, kin_n), lr, li, k, kn);
     // the accumulator after stages 2 and 3, the new state after stage 4
     cplx_t<T> av;
     T avn = 0;
+    LineStep<T> h = {};
     if (st == 4) {
+        h = line_step(a.dt);             // (two divisions, this stage's alone)
         av.x = line_combine<T, 4>(acc.x, k.x, u.x, h);
         av.y = line_combine<T, 4>(acc.y, k.y, u.y, h);
         avn = line_combine<T, 4>(accn, kn, un, h);
