@@ -1048,27 +1048,33 @@ template <typename T> struct ResShape;
 template <> struct ResShape<float> { static constexpr int THREADS = 1024; };
 template <> struct ResShape<double> { static constexpr int THREADS = 512; };
 
-template <typename T, int ORDER, int BC, int DIM>
-__device__ __forceinline__ cplx_t<T> resident_lap(const cplx_t<T> *Y, int idx, int n, const T *w,
-                                                  const T *wrow) {
+// Laplacian of point idx of a line (wrow: its row of the radial table; outside
+// the reference's grid the line is zero) and of a 2-D grid.
+template <typename T, int ORDER, int BC>
+__device__ __forceinline__ cplx_t<T> lap_line(const cplx_t<T> *Y, int idx, int n, const T *w, const T *wrow) {
     constexpr int R = (ORDER - 1) / 2;
-    if constexpr (DIM == 1) {
-        // the points around it; outside the reference's grid zero
-        T ex[2 * R + 1], ey[2 * R + 1];
+    T ex[2 * R + 1], ey[2 * R + 1];
 #pragma unroll
-        for (int d = -R; d <= R; ++d) {
+    for (int d = -R; d <= R; ++d) {
+        cplx_t<T> v;
+        if constexpr (BC == BC_PERIODIC) {
             int j = idx + d;
-            if (BC == BC_PERIODIC) {
-                if (j < 0) j += n;
-                if (j >= n) j -= n;
-            }
-            const cplx_t<T> v = j >= 0 && j < n ? Y[j] : mk<T>(0, 0);
-            ex[R + d] = v.x;
-            ey[R + d] = v.y;
+            if (d < 0 && j < 0) j += n;
+            if (d > 0 && j >= n) j -= n;
+            v = Y[j];
+        } else {
+            v = idx + d >= 0 && idx + d < n ? Y[idx + d] : mk<T>(0, 0);
         }
-        if (BC == BC_PERIODIC) return mk<T>(line_lap<T, R>(w, ex + R), line_lap<T, R>(w, ey + R));
-        return mk<T>(line_lap_row<T, R>(wrow, ex + R), line_lap_row<T, R>(wrow, ey + R));
-    } else {
+        ex[R + d] = v.x;
+        ey[R + d] = v.y;
+    }
+    if (BC == BC_PERIODIC) return mk<T>(line_lap<T, R>(w, ex + R), line_lap<T, R>(w, ey + R));
+    return mk<T>(line_lap_row<T, R>(wrow, ex + R), line_lap_row<T, R>(wrow, ey + R));
+}
+
+template <typename T, int ORDER, int BC>
+__device__ __forceinline__ cplx_t<T> lap_grid(const cplx_t<T> *Y, int idx, int n, const T *w) {
+    constexpr int R = (ORDER - 1) / 2;
     const cplx_t<T> c = Y[idx];
     const int row = idx / n, col = idx - row * n;
     T lr = lap_centre<T>((T)2 * w[0], c.x), li = lap_centre<T>((T)2 * w[0], c.y);
@@ -1092,11 +1098,15 @@ __device__ __forceinline__ cplx_t<T> resident_lap(const cplx_t<T> *Y, int idx, i
         li += lap_quad<T>(w[d], c.y, a0.y, a1.y, b0.y, b1.y, d);
     }
     return mk<T>(lr, li);
-    }
 }
 
+// Waves a SIMD: in single precision two workgroups share a CU's LDS, and its
+// registers where a thread needs no more than 64, which zero-outside order 5
+// without a reservoir does by two (64; order 3 with one by seven, and would spill).
 template <typename T, int ORDER, int BC, bool DYN>
-__global__ void __launch_bounds__(ResShape<T>::THREADS) k_resident(const ResidentArgs<T> r) {
+constexpr int res_waves = sizeof(T) == 8 ? 2 : ORDER == 5 && BC == BC_REF && !DYN ? 8 : 4;
+template <typename T, int ORDER, int BC, bool DYN>
+__global__ void __launch_bounds__(ResShape<T>::THREADS, (res_waves<T, ORDER, BC, DYN>)) k_resident(const ResidentArgs<T> r) {
     using C = cplx_t<T>;
     constexpr int RES_THREADS = ResShape<T>::THREADS, RES_PPT = RES_MAXP / RES_THREADS;
     // Y[b] is the psi stage input, double-buffered -- stage s reads Y[b] and
@@ -1153,7 +1163,7 @@ __global__ void __launch_bounds__(ResShape<T>::THREADS) k_resident(const Residen
             return s == 4 ? v : u;
         };
         auto slopes = [&](const C *Yin, int q, int idx, C &kk, T &kn) {
-            const C lap = resident_lap<T, ORDER, BC, 1>(Yin, idx, n, w, wtab ? wtab + (size_t)idx * ORDER : nullptr);
+            const C lap = lap_line<T, ORDER, BC>(Yin, idx, n, w, wtab ? wtab + (size_t)idx * ORDER : nullptr);
             line_rhs<T, DYN>(m.c, pump_term<T, DYN>(m.c, pp[q]), Yin[idx], yn[q], lap.x, lap.y, kk, kn);
         };
         if constexpr (PINGPONG) {
@@ -2050,7 +2060,9 @@ __global__ void __launch_bounds__(256) k_batch_energy(const MemberDev<T> *mem, c
     double v[3] = {0, 0, 0};
     for (long long i = threadIdx.x; i < N; i += 256) {
         const double wi = (DIM == 1 && BC == BC_REF) ? (double)i : 1.0;
-        const cplx_t<T> lap = resident_lap<T, ORDER, BC, DIM>(u, (int)i, n, w, wt ? wt + (size_t)i * ORDER : nullptr);
+        cplx_t<T> lap;
+        if constexpr (DIM == 1) lap = lap_line<T, ORDER, BC>(u, (int)i, n, w, wt ? wt + (size_t)i * ORDER : nullptr);
+        else lap = lap_grid<T, ORDER, BC>(u, (int)i, n, w);
         const double pr = u[i].x, pi = u[i].y;
         const double sq = pr * pr + pi * pi;
         const double r = nn ? (double)nn[i] : c12 * (double)pp[i] / (c13 + c14 * sq);

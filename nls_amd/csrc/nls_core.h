@@ -85,18 +85,12 @@ __device__ __forceinline__ void rhs_point(const Coeffs<T> &c, T P, cplx_t<T> y, 
 //     (the weights of a stencil sum to zero).  For d = 1 the differences to c
 //     are formed first -- exact when the values are close, as on a smooth
 //     field on a fine grid -- so the largest weights (w_1 ~ 1/h^2) no longer
-//     amplify the rounding of c; for d >= 2 the neighbour sum less 2c (1-D) or
-//     4c (2-D).  This keeps the single-precision Laplacian accurate where the
+//     amplify the rounding of c; for d >= 2 the neighbour sum less 2c (1-D,
+//     line_lap) or 4c (2-D, lap_quad).  This keeps the single-precision Laplacian accurate where the
 //     stencil sum cancels to a small result.
 // The two forms are equal up to rounding.
 template <typename T> __device__ __forceinline__ T lap_centre(T wc, T c) {
     return sizeof(T) == 8 ? wc * c : (T)0;
-}
-
-template <typename T> __device__ __forceinline__ T lap_pair(T w, T c, T a0, T a1, int d) {
-    if (sizeof(T) == 8) return w * (a0 + a1);
-    if (d == 1) return w * ((a0 - c) + (a1 - c));
-    return w * ((a0 + a1) - (T)2 * c);
 }
 
 template <typename T> __device__ __forceinline__ T lap_quad(T w, T c, T a0, T a1, T b0, T b1, int d) {
@@ -218,8 +212,8 @@ template <typename T> __device__ __forceinline__ T grid_new_from(T u, T acc, T k
 // kernels, with every fused multiply-add written out and contraction off:
 // both kernels round each operation alike, so a line solved alone and in a
 // batch gives the same bits whichever of them runs it.
-// Periodic Laplacian from the neighbours e[-R..R] (e[0] the point): the
-// forms of lap_centre / lap_pair.
+// Periodic Laplacian from the neighbours e[-R..R] (e[0] the point), in the
+// forms above.
 template <typename T, int R> __device__ __forceinline__ T line_lap(const T *w, const T *e) {
 #pragma clang fp contract(off)
     T l;
