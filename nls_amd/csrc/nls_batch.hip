@@ -24,6 +24,7 @@
 //                       (2-D) or per-stage (1-D) engine.
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <type_traits>
 #include <cstring>
 #include <vector>
@@ -1379,26 +1380,34 @@ static int fused_form(int dtype, int order, int bc, const TileCounts &t) {
 // ---- marching strips or tiles ------------------------------------------------
 // The marching kernel (nls_march.hip: order 5, periodic) runs the step of
 // launches that fill the device; its strips are cut for that.  Times in us on
-// MI355X, as measured:
+// MI355X, from 380 grids and batches of 64 to 4096 points a side timed both ways:
 //  - a piece costs its rows and MARCH_PIECE more (its halo's stages and first
 //    loads), and a CU's workgroups add up: 0.37 a row for one on the CU (one
-//    wave a SIMD does not hide its latency), 0.23 for each of several; double
-//    precision 0.55 and 0.45;
+//    wave a SIMD does not hide its latency), 0.21 for each of several, 0.28
+//    without a reservoir (each stage divides); double precision 0.55 and 0.43;
 //  - a round of tiles (512 of the pair kernel's 64 x 32, 512 of double
-//    precision's 64 x 16) costs 7.4 and 7.7; short tiles that fit one per CU
-//    5.4 and 6.7 in all.
+//    precision's 64 x 16) costs 7.4 and 7.7, short tiles that fit one per CU
+//    5.4 and 6.7 in all; past the first round the next one's tiles start as CUs
+//    come free, and the time grows with the tiles.
+// With these the slower of the two is taken by 3% at most; with whole rounds and
+// one rate a row for both reservoirs, grids without one marched up to 1.3 times
+// slower than on tiles (12 of 300^2 FP32 16.9 against 13.0, 30 of 512^2 64 against 53).
 // us per step, tiles -> strips: 2048^2 FP32 32.5 -> 26.5, FP64 58.6 -> 49; 154
 // grids of 128^2 and 102 of 256^2 FP32 73 -> 52, FP64 175 -> 117; 64 of 200^2
 // FP32 28.1 -> 21.9, FP64 52.4 -> 40.8; one 1024^2 grid stays on tiles (11.7; FP64
 // 19.8 as strips and tiles).
 constexpr double MARCH_LAUNCH = 3.0;
 constexpr int MARCH_PIECE = 16;
-static double march_us(int dtype, int percu, int rows) {
-    return percu * rows * (dtype == NLS_F64 ? (percu > 1 ? 0.45 : 0.55) : (percu > 1 ? 0.23 : 0.37));
+static double march_us(int dtype, bool dyn, int percu, int rows) {
+    if (dtype == NLS_F64) return percu * rows * (percu > 1 ? 0.43 : 0.55);
+    return percu * rows * (percu == 1 ? 0.37 : dyn ? 0.21 : 0.28);
 }
-static double tiles_us(int dtype, const TileCounts &t, int cus) {
-    if (t.t16 <= cus) return dtype == NLS_F64 ? 6.7 : 5.4;
-    return MARCH_LAUNCH + (dtype == NLS_F64 ? 7.7 * ((t.t16 + 511) / 512) : 7.4 * ((t.t32 + 511) / 512));
+static double tiles_us(int dtype, bool dyn, const TileCounts &t, int cus) {
+    const bool f64 = dtype == NLS_F64;
+    if (t.t16 <= cus) return f64 ? 6.7 : 5.4;
+    const double r = (f64 ? t.t16 : t.t32) / 512.0, round = f64 ? 7.7 : 7.4, whole = MARCH_LAUNCH + round * ceil(r);
+    if (r <= 1) return whole;
+    return std::min(whole, f64 ? (dyn ? 5.5 + 7.7 * r : 5.0 + 7.2 * r) : (dyn ? 6.5 + 7.4 * r : 6.0 + 6.4 * r));
 }
 // Members the kernel takes: rows of at least one wave, and byte offsets that
 // stay below 2^32 when they run past the grid's end by up to its size.
@@ -1430,12 +1439,13 @@ static MarchGrid march_grid(const nls_problem *p) {
     MarchGrid best = {0, 0, 0, 0, 0};
     const int n = p->n, cus = device_cus();
     if (n <= 256 || !march_applies(p->dtype, p->order, p->bc) || !march_holds(n, p->dtype) || cus <= 0) return best;
-    double least = tiles_us(p->dtype, tiles_of(n, n), cus);
+    const bool dyn = p->coeffs[10] != 0.0;
+    double least = tiles_us(p->dtype, dyn, tiles_of(n, n), cus);
     const StripShape sh = strip_shape(n);
     for (int per = 1; per <= march_slots(p->dtype); ++per) {
         const int pieces = std::max(1, per * cus / sh.nx);
         const int L = (n + pieces - 1) / pieces, groups = sh.nx * ((n + L - 1) / L);
-        const double t = MARCH_LAUNCH + march_us(p->dtype, per, L + MARCH_PIECE) * ((groups + per * cus - 1) / (per * cus));
+        const double t = MARCH_LAUNCH + march_us(p->dtype, dyn, per, L + MARCH_PIECE) * ((groups + per * cus - 1) / (per * cus));
         if (t < least) { least = t; best = MarchGrid{groups, per, sh.nx, sh.wd, L}; }
     }
     return best;
@@ -1450,7 +1460,7 @@ struct MarchCut {
     int percu = 0;
     double us = 0;
 };
-static MarchCut march_cut(int dtype, const nls_member *members, int count, bool full, int cus) {
+static MarchCut march_cut(int dtype, bool dyn, const nls_member *members, int count, bool full, int cus) {
     MarchCut best;
     // cuts for workgroups of at most `cost` rows, MARCH_PIECE of them a piece's;
     // returns the number of workgroups
@@ -1493,7 +1503,7 @@ static MarchCut march_cut(int dtype, const nls_member *members, int count, bool 
             if (cut(mid, nullptr) > groups) lo = mid;
             else hi = mid;
         }
-        const double us = MARCH_LAUNCH + march_us(dtype, per, hi);
+        const double us = MARCH_LAUNCH + march_us(dtype, dyn, per, hi);
         if (best.percu && us >= best.us) continue;
         cut(hi, &best);
         best.percu = per;
@@ -2232,11 +2242,11 @@ static void plan(nls_batch *b, const nls_member *members, int count, const int *
         for (int i = 0; i < count; ++i) b->march = b->march && march_holds(members[i].n, b->dtype);
         b->cuts[0] = b->cuts[1] = MarchCut();
         if (b->march) {
-            const double tiles = tiles_us(b->dtype, counts, cus);
+            const double tiles = tiles_us(b->dtype, b->dyn, counts, cus);
             // (nothing marches faster than a few rows of every CU)
-            b->march = tiles > MARCH_LAUNCH + march_us(b->dtype, 1, 12 + MARCH_PIECE);
+            b->march = tiles > MARCH_LAUNCH + march_us(b->dtype, b->dyn, 1, 12 + MARCH_PIECE);
             if (b->march)
-                for (int w = 0; w < 2; ++w) b->cuts[w] = march_cut(b->dtype, members, count, w == 0, cus);
+                for (int w = 0; w < 2; ++w) b->cuts[w] = march_cut(b->dtype, b->dyn, members, count, w == 0, cus);
             b->march = b->march && b->cuts[0].us + b->cuts[1].us < tiles;
         }
     }
