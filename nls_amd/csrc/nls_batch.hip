@@ -256,6 +256,14 @@ static_assert(RingMap<80, 48, 2, 84>().v[2048] == (6 * 84 + 6 | 6 << 16 | 6 << 2
 static_assert(RingMap<80, 32, 2, 84>().v[1024] == (6 * 84 + 6 | 6 << 16 | 6 << 24), "stage-3 ring follows the 64 x 16 tile");
 template <int W, int HH, int R, int WS> __device__ const RingMap<W, HH, R, WS> ring_map{};
 
+// A tile whose waves hold few columns of the grid: double-precision arithmetic of a
+// wave with eight active lanes or fewer takes longer than of one with all (8 grids of
+// order 3 zero-outside: 73^2 4.4 us a step, 72^2, whose last tile is eight columns
+// wide, 5.4, as all lanes 4.6), so there every lane runs and the stores are masked.
+template <typename T> __device__ __forceinline__ bool few_columns(int n, int x0) {
+    return sizeof(T) == 8 && n - x0 <= 8;
+}
+
 // S32 (double precision only): the fields sit in HBM in single precision --
 // state, reservoir and pumping are widened on load and the new state rounded
 // once on store -- and everything else is the double-precision step: FP64
@@ -326,6 +334,7 @@ k_fused_step_2d(const FusedArgs<T> f) {
         return;
     }
 
+    const bool few = few_columns<T>(n, td.x0);
     const T dt = m.dt, dt2 = dt * (T)0.5, dt6 = m.g.dt6;                   // of the reservoir
     const T dtw = m.g.dtw, dtw2 = dtw * (T)0.5, dtw6 = m.g.dtw6;           // of psi
     Coeffs<T> c = m.c;
@@ -496,7 +505,8 @@ k_fused_step_2d(const FusedArgs<T> f) {
         for (int j = 0; j < J; ++j) {
             if (NT * j >= cnt) break;
             if (tid + NT * j >= lim) continue;
-            if (BC == BC_REF && !((inside >> j) & 1u)) continue;
+            const bool in = BC != BC_REF || ((inside >> j) & 1u);
+            if (BC == BC_REF && !in && !few) continue;
             C k;
             T kn;
             stage_rhs(yin, j, k, kn);
@@ -504,8 +514,8 @@ k_fused_step_2d(const FusedArgs<T> f) {
             grid_acc(acc[j].y, k.y, s == 1);
             if (DYN) grid_acc(accn[j], kn, s == 1);
             const C yv = mk<T>(grid_input(uu[j].x, k.x, dtwa), grid_input(uu[j].y, k.y, dtwa));
-            if (DB) yout[li[j]] = yv;
-            else ynext[j] = yv;
+            if (!DB) ynext[j] = yv;
+            else if (in) yout[li[j]] = yv;
             if (DYN) yn[j] = grid_input(nn[j], kn, dta);
         }
         __syncthreads();
@@ -527,10 +537,12 @@ k_fused_step_2d(const FusedArgs<T> f) {
     for (int j = 0; j < JOUT; ++j) {
         const int k0 = tid + NT * j;
         const int gx = td.x0 + (k0 & (TX - 1)), gy = td.y0 + k0 / TX;
-        if (gx >= n || gy >= ylim) continue;
+        const bool in = gx < n && gy < ylim;
+        if (!in && !few) continue;
         C k;
         T kn;
         stage_rhs(yb, j, k, kn);
+        if (!in) continue;
         const size_t gi = (size_t)gy * n + gx;
         uo[gi] = SC{(SR)grid_new(uu[j].x, acc[j].x, k.x, dtw6), (SR)grid_new(uu[j].y, acc[j].y, k.y, dtw6)};
         if (DYN) uno[gi] = (SR)grid_new(nn[j], accn[j], kn, dt6);
@@ -876,6 +888,7 @@ k_fused_groups_2d(const FusedArgs<T> f) {
         return;
     }
 
+    const bool few = few_columns<T>(n, td.x0);
     const T dt = m.dt, dt2 = dt * (T)0.5, dt6 = m.g.dt6;
     const T dtw = m.g.dtw, dtw2 = dtw * (T)0.5, dtw6 = m.g.dtw6;
     Coeffs<T> c = m.c;
@@ -1022,9 +1035,9 @@ k_fused_groups_2d(const FusedArgs<T> f) {
         const int k0 = tid + NT * j;
         if (k0 >= NOUT) break;
         const int gx = td.x0 + (k0 & (TX - 1)), gy = td.y0 + R * (k0 / TX);
-        if (gx >= n || gy >= ylim) continue;
+        if (!few && (gx >= n || gy >= ylim)) continue;
         group_rhs(yb, j, [&](int q, const C &k, T kn) {
-            if (gy + q < ylim) {
+            if (gx < n && gy + q < ylim) {
                 const size_t gi = (size_t)(gy + q) * n + gx;
                 uo[gi] = SC{(SR)grid_new(uu[j][q].x, acc[j][q].x, k.x, dtw6),
                             (SR)grid_new(uu[j][q].y, acc[j][q].y, k.y, dtw6)};
