@@ -475,8 +475,15 @@ void launch_resident_2d(int order, int bc, bool dyn, int count, int n, const Res
     if (sizeof(T) == 4 && v == VM && strips(3) <= 1024) v = 3;
     if (sizeof(T) == 4 && bc == NLS_BC_REF && n > 48 && count > device_cus()) v = VM;
     const int nt = v == VM ? 64 * 64 / VM : (strips(v) + 63) / 64 * 64;
+    // Grids of a hybrid batch on up to half the CUs keep them to themselves, by unused
+    // LDS: a tile of the other members on the same CU steps at half the rate, and the
+    // batch's step waits for it (20 of 64^2 beside 20 of 128^2 FP32 zero-outside 9.9
+    // us a step sharing, 6.7 apart; 256 of 64^2, on every CU, 10.3 and 12.1)
+    constexpr int ALONE = 120 * 1024;    // leaves less than the smallest tile takes
+    const int row = 64 + order - 1, own = 2 * row * row * (int)sizeof(cplx_t<T>);
+    const int pad = 2 * count <= device_cus() && own < ALONE ? ALONE - own : 0;
 #define NLS_V(O, B, D, V) \
-    if (v == V) hipLaunchKernelGGL((k_resident_2d<T, O, B, D, V>), dim3(count), dim3(nt), 0, s, r);
+    if (v == V) hipLaunchKernelGGL((k_resident_2d<T, O, B, D, V>), dim3(count), dim3(nt), pad, s, r);
 #define NLS_CASE(O, B, D)                                  \
     if (order == O && bc == B && dyn == D) {               \
         NLS_V(O, B, D, 1) NLS_V(O, B, D, 2)                \
