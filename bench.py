@@ -529,14 +529,7 @@ def main():
         log("tuned batch engine: %s (%s us/step)" % (engine, ", ".join("%s %.1f" % kv for kv in tuning.items())))
         if engine in ("fused", "hybrid"):
             form = tuner.fused_form(members, dim=2, order=5, bc="periodic", dtype="f32", engine=engine)
-            times = {k: v * 1e6 for k, v in tuner.last.items()}
-            # the library's own choice (marching strips where they pay) beside the tile forms
-            native.fused_form("f32", "auto")
-            times["auto"] = min(tuner._time_batch(members, 2, 5, "periodic", "f32", engine) for _ in range(2)) * 1e6
-            if times[form] < times["auto"]:
-                native.fused_form("f32", form)
-            else:
-                form = "auto"
+            times = {k: v * 1e6 for k, v in dict(tuner.last, auto=tuner.auto_seconds).items()}
             tuning = {"engine": tuning, "fused_form": times}
             log("tuned fused tile form: %s (%s us/step)" % (form, ", ".join(
                 "%s %.1f" % kv for kv in tuning["fused_form"].items())))

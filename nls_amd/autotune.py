@@ -9,7 +9,9 @@ problem class, so each choice is measured once per machine and reused after.
 What is tuned:
   * ``plain_engine(desc)``   -- engine of a plain solve (nls_advance): resident
     (instances that fit on chip), fused (2-D) or per-stage, each with its
-    step-block graphs;
+    step-block graphs, or in 1-D the library's own choice ("auto": pieces of the
+    line in registers, which no engine name reaches; in 2-D it is one of the
+    named engines);
   * ``stage_tile(dtype)``    -- tile height (4, 8, 16, 32 rows) of the 2-D
     per-stage kernels (nls_tune_stage_tile), applied to the library;
   * ``batch_engine(members, ...)`` -- engine of a batch (nls_batch_create):
@@ -18,9 +20,12 @@ What is tuned:
     of the fused kernel (nls_tune_fused_form), applied to the library:
     64 x 32 tiles of 1024 threads ("tall"), 64 x 16 tiles of 1024 threads
     ("short"), or, in double precision on periodic grids, 64 x 16 tiles of 512
-    threads with one stage buffer ("half").  The halo is not a free
-    parameter: one launch per RK4 step needs the 4R rings its four stages
-    consume (R the stencil radius).
+    threads with one stage buffer ("half"); order 7: 64 x 24 ("tall") or
+    64 x 16 ("short").  A form asked for turns marching strips and launches of
+    several steps off for its dtype in the whole process, so the library's own
+    choice is timed too, and kept ("auto") where it is the faster.  The halo is
+    not a free parameter: one launch per RK4 step needs the 4R rings its four
+    stages consume (R the stencil radius).
 
 The cache file is ``$NLS_AMD_TUNE_CACHE`` or ``~/.cache/nls_amd/tune.json``;
 ``Tuner(path=None)`` keeps the results in memory only.
@@ -51,7 +56,8 @@ def _device_name():
 
 class Tuner(object):
     """``timer(candidate, setup) -> seconds`` may be injected (tests); by
-    default candidates run on the GPU and are timed with HIP events."""
+    default candidates run on the GPU and are timed with HIP events.  One that
+    raises LookupError for the form "auto" leaves it out."""
 
     def __init__(self, path="default", steps=64, reps=3, timer=None, device_name=None):
         self.path = default_cache_path() if path == "default" else path
@@ -60,6 +66,7 @@ class Tuner(object):
         self._device = device_name
         self.table = {}
         self.last = {}            # timings of the last measured choice, by candidate
+        self.auto_seconds = None  # of the library's own choice beside the last tile form
         if self.path and os.path.exists(self.path):
             try:
                 with open(self.path) as f:
@@ -104,6 +111,7 @@ class Tuner(object):
 
     # ---- plain solves ------------------------------------------------------
     def plain_candidates(self, desc):
+        """The named engines that can run desc."""
         cands = []
         for e in (ENGINES_2D if desc.dim == 2 else ENGINES_1D):
             if e == "resident" and not _resident_fits(desc):
@@ -115,9 +123,12 @@ class Tuner(object):
         """Fastest RK4 engine for a plain solve of desc's problem class."""
         if desc.scheme != native.SCHEME["rk4"]:
             return "auto"
-        key = self._key("plain", dim=desc.dim, n=desc.n, dtype=desc.dtype, order=desc.order, bc=desc.bc,
-                        dyn=int(desc.dynamic))
-        return self._choose(key, self.plain_candidates(desc), lambda e: self._time_plain(desc, e))
+        fields = dict(dim=desc.dim, n=desc.n, dtype=desc.dtype, order=desc.order, bc=desc.bc, dyn=int(desc.dynamic))
+        cands = self.plain_candidates(desc)
+        if desc.dim == 1:
+            cands.append("auto")
+            fields["auto"] = 1                 # choices stored without it are measured again
+        return self._choose(self._key("plain", **fields), cands, lambda e: self._time_plain(desc, e))
 
     def tuned(self, desc):
         """A copy of desc with the tuned engine."""
@@ -168,13 +179,16 @@ class Tuner(object):
     # ---- fused kernel tile form ---------------------------------------------
     @staticmethod
     def form_candidates(dtype, bc, order):
+        """Tile forms by name; order 7 takes "short" beside these (_form_choice)."""
         if order == 7:
-            return ["tall"]                        # one form at order 7
+            return ["tall"]
         periodic = bc in ("periodic", 1)
         return (["tall", "short"] + (["half"] if dtype in ("f64", 1) and periodic else []) +
                 (["tall512"] if dtype in ("f32", 0) and periodic and order == 5 else []))
 
-    def _form_choice(self, key, dtype, cands, run, apply):
+    def _form_choice(self, kind, dtype, bc, order, run, apply, **fields):
+        cands = self.form_candidates(dtype, bc, order) + (["short"] if order == 7 else [])
+        key = self._key(kind, dtype=dtype, bc=bc, order=order, auto=1, **fields)
         prev = native.fused_form(dtype) if self._timer is None else None
 
         def timed(form):
@@ -182,41 +196,53 @@ class Tuner(object):
                 native.fused_form(dtype, form)
             return run(form)
 
-        best = self._choose(key, cands, timed)
+        hit = self.table.get(key)
+        if hit is not None and hit.get("best") in cands + ["auto"]:
+            best, self.last, self.auto_seconds = hit["best"], dict(hit["seconds_per_step"]), hit.get("auto")
+        else:
+            best = self._choose(key, cands, timed)
+            # the library's own choice, in turn with the best form: a form is
+            # asked for unless that is faster by more than such timings differ
+            try:
+                turns = [(timed("auto"), timed(best)) for _ in range(max(3, self.reps))]
+                self.auto_seconds, form_seconds = (min(t) for t in zip(*turns))
+                if self.auto_seconds < 0.9 * form_seconds:
+                    best = "auto"
+            except LookupError:
+                self.auto_seconds = None
+            self.table[key] = {"best": best, "seconds_per_step": self.last, "auto": self.auto_seconds}
+            self._save()
         if self._timer is None:
             native.fused_form(dtype, best if apply else prev)
         return best
 
     def fused_form(self, members, dim=2, order=5, bc="periodic", dtype="f32", engine="fused", apply=True):
         """Fastest tile form of the fused kernel for a batch of this member
-        mix on `engine` ("fused" or "hybrid"); applied to the library."""
+        mix on `engine` ("fused" or "hybrid"), or "auto" where the library's own
+        choice is faster than any; applied to the library."""
         sizes = {}
         for m in members:
             sizes[int(m.n)] = sizes.get(int(m.n), 0) + 1
         mix = ",".join("%dx%d" % (n, c) for n, c in sorted(sizes.items()))
         dyn = int(np.asarray(members[0].coeffs)[10] != 0.0)
-        key = self._key("fused_form", dim=dim, order=order, bc=bc, dtype=dtype, dyn=dyn, mix=mix, engine=engine)
-
         def run(form):
             if self._timer is not None:
                 return self._timer(("fused_form", form), members)
             return self._time_batch(members, dim, order, bc, dtype, engine)
 
-        return self._form_choice(key, dtype, self.form_candidates(dtype, bc, order), run, apply)
+        return self._form_choice("fused_form", dtype, bc, order, run, apply, dim=dim, dyn=dyn, mix=mix, engine=engine)
 
     def plain_fused_form(self, desc, apply=True):
         """Fastest tile form of the fused kernel for a plain 2-D solve of
-        desc's problem class; applied to the library."""
+        desc's problem class, or "auto" as fused_form; applied to the library."""
         dtype = "f64" if desc.dtype == 1 else "f32"
         bc = "periodic" if desc.bc == 1 else "ref"
-        key = self._key("plain_fused_form", n=desc.n, dtype=dtype, order=desc.order, bc=bc, dyn=int(desc.dynamic))
-
         def run(form):
             if self._timer is not None:
                 return self._timer(("plain_fused_form", form), desc)
             return self._time_plain(desc, "fused")
 
-        return self._form_choice(key, dtype, self.form_candidates(dtype, bc, desc.order), run, apply)
+        return self._form_choice("plain_fused_form", dtype, bc, desc.order, run, apply, n=desc.n, dyn=int(desc.dynamic))
 
     # ---- batches -----------------------------------------------------------
     def batch_engine(self, members, dim=2, order=5, bc="periodic", dtype="f32"):
