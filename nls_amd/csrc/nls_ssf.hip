@@ -302,7 +302,6 @@ __device__ __forceinline__ void pointwise_rk4(const Coeffs<T> &c, T inv_c11, T P
 // FP32), so a single-precision state only halves the HBM bytes and is
 // rounded once per pass, not at every FFT stage.
 template <typename S, typename T> struct SsfArgs {
-    int logN;
     T half_dt, inv_c11;
     Coeffs<T> c;
     cplx_t<S> *psi;
@@ -833,7 +832,6 @@ static int ssf_run(const nls_problem *p, int iters, const S *P, cplx_t<S> *psi, 
     hipLaunchKernelGGL(k_ssf_tables<T>, dim3((N + 255) / 256), dim3(256), 0, s, N, p->dx, p->dt, 1.0 / N, tw, ph);
     SsfArgs<S, T> a;
     memset(&a, 0, sizeof a);
-    a.logN = logN;
     a.half_dt = (T)(0.5 * p->dt);
     a.c = make_coeffs<T>(p->coeffs);
     a.inv_c11 = DYN ? (T)(1.0 / p->coeffs[10]) : (T)0;
