@@ -1116,11 +1116,16 @@ __device__ __forceinline__ cplx_t<T> lap_grid(const cplx_t<T> *Y, int idx, int n
 
 // Waves a SIMD: in single precision two workgroups share a CU's LDS, and its
 // registers where a thread needs no more than 64, which zero-outside order 5
-// without a reservoir does by two (64; order 3 with one by seven, and would spill).
+// without a reservoir does by two.  Order 3 with one needs 71, of which twelve are
+// the weights of a thread's points; for more lines than CUs (MANY) those are loaded
+// every stage, so that two workgroups share one (us per step, 256 points each: 512 lines
+// 1.64 -> 1.08; 64 lines, one a CU either way, 0.82 -> 1.05).
 template <typename T, int ORDER, int BC, bool DYN>
-constexpr int res_waves = sizeof(T) == 8 ? 2 : ORDER == 5 && BC == BC_REF && !DYN ? 8 : 4;
-template <typename T, int ORDER, int BC, bool DYN>
-__global__ void __launch_bounds__(ResShape<T>::THREADS, (res_waves<T, ORDER, BC, DYN>)) k_resident(const ResidentArgs<T> r) {
+constexpr bool res_many = sizeof(T) == 4 && ORDER == 3 && BC == BC_REF && DYN;
+template <typename T, int ORDER, int BC, bool DYN, bool MANY>
+constexpr int res_waves = sizeof(T) == 8 ? 2 : MANY || (ORDER == 5 && BC == BC_REF && !DYN) ? 8 : 4;
+template <typename T, int ORDER, int BC, bool DYN, bool MANY>
+__global__ void __launch_bounds__(ResShape<T>::THREADS, (res_waves<T, ORDER, BC, DYN, MANY>)) k_resident(const ResidentArgs<T> r) {
     using C = cplx_t<T>;
     constexpr int RES_THREADS = ResShape<T>::THREADS, RES_PPT = RES_MAXP / RES_THREADS;
     // Y[b] is the psi stage input, double-buffered -- stage s reads Y[b] and
@@ -1165,7 +1170,11 @@ __global__ void __launch_bounds__(ResShape<T>::THREADS, (res_waves<T, ORDER, BC,
     }
     __syncthreads();
     int b = 0;
-    const LineStep<T> h = line_step(m.dt);
+    LineStep<T> h = line_step(m.dt);
+    if constexpr (MANY) {                // into scalar registers: the same for all lanes
+        auto uniform = [](T v) { return __builtin_bit_cast(T, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v))); };
+        h = LineStep<T>{uniform(h.dt), uniform(h.dt2), uniform(h.dt6), uniform(h.dt6lo)};
+    }
     auto run_stage = [&](auto s_) {
         constexpr int s = decltype(s_)::value;
         // the next stage input, or at stage 4 the new state; returns the state
@@ -1177,7 +1186,9 @@ __global__ void __launch_bounds__(ResShape<T>::THREADS, (res_waves<T, ORDER, BC,
             return s == 4 ? v : u;
         };
         auto slopes = [&](const C *Yin, int q, int idx, C &kk, T &kn) {
-            const C lap = lap_line<T, ORDER, BC>(Yin, idx, n, w, wtab ? wtab + (size_t)idx * ORDER : nullptr);
+            unsigned row = idx * ORDER;
+            if (MANY) asm volatile("" : "+v"(row));  // (loop-invariant loads otherwise)
+            const C lap = lap_line<T, ORDER, BC>(Yin, idx, n, w, BC == BC_REF ? wtab + row : nullptr);
             line_rhs<T, DYN>(m.c, pump_term<T, DYN>(m.c, pp[q]), Yin[idx], yn[q], lap.x, lap.y, kk, kn);
         };
         if constexpr (PINGPONG) {
@@ -1530,7 +1541,12 @@ static void launch_resident(int dim, int order, int bc, bool dyn, int count, int
     if (dim == 2) return launch_resident_2d<T>(order, bc, dyn, count, n, r, s);
 #define NLS_CASE(O, B, D)                                                                                     \
     if (order == O && bc == B && dyn == D) {                                                                 \
-        hipLaunchKernelGGL((k_resident<T, O, B, D>), dim3(count), dim3(ResShape<T>::THREADS), 0, s, r);       \
+        if constexpr (res_many<T, O, B, D>)                                                                   \
+            if (count > device_cus()) {                                                                       \
+                hipLaunchKernelGGL((k_resident<T, O, B, D, true>), dim3(count), dim3(ResShape<T>::THREADS), 0, s, r); \
+                return;                                                                                       \
+            }                                                                                                 \
+        hipLaunchKernelGGL((k_resident<T, O, B, D, false>), dim3(count), dim3(ResShape<T>::THREADS), 0, s, r); \
         return;                                                                                               \
     }
     NLS_CASE(3, 0, false) NLS_CASE(3, 0, true) NLS_CASE(3, 1, false) NLS_CASE(3, 1, true)
