@@ -259,7 +259,7 @@ template <int W, int HH, int R, int WS> __device__ const RingMap<W, HH, R, WS> r
 // A tile whose waves hold few columns of the grid: double-precision arithmetic of a
 // wave with eight active lanes or fewer takes longer than of one with all (8 grids of
 // order 3 zero-outside: 73^2 4.4 us a step, 72^2, whose last tile is eight columns
-// wide, 5.4, as all lanes 4.6), so there every lane runs and the stores are masked.
+// wide, 5.4, as all lanes 5.0), so there every lane runs and the stores are masked.
 template <typename T> __device__ __forceinline__ bool few_columns(int n, int x0) {
     return sizeof(T) == 8 && n - x0 <= 8;
 }

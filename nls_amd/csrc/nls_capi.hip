@@ -50,14 +50,16 @@ int check_problem(const nls_problem *p) {
 
 // RK4 engine of a plain solve.  AUTO: the line kernel for 1-D (us per step
 // against the engines it replaced: n = 256 FP32 0.56 / 0.88 resident, n = 1000
-// radial FP32 0.59 / 3.6, n = 4096 FP64 0.67 / 6.3; longer lines took 8 to 15
-// on the per-stage kernels, 20,000 points take 0.67); in 2-D the fused engine,
+// radial FP32 0.61 / 3.6, n = 4096 FP64 0.65 / 6.3; longer lines took 8 to 15
+// on the per-stage kernels, 20,000 points take 0.69); in 2-D the fused engine,
 // whose small grids step several times a launch, or in single precision up to
 // small_resident points a side the resident kernel, with the same bits.  us per step,
-// launches of several steps / resident: zero-outside, order 3 32^2 1.9 / 1.3, 36^2 1.9 /
-// 2.0; order 5 32^2 2.8 / 1.6, 44^2 2.9 / 2.9; order 7 (one step a launch) 48^2 4.3 / 3.8,
-// 52^2 4.3 / 4.9; periodic, order 3 44^2 1.85 / 1.6, 48^2 1.9 / 3.1; order 5 54^2 3.15 / 3.1,
-// 56^2 3.2 / 4.9; order 7 54^2 4.9 / 4.0, 56^2 4.9 / 5.8.
+// launches of several steps / resident, without a reservoir (with one): zero-outside,
+// order 3 32^2 1.75 / 1.3 (1.7 / 1.1), 36^2 1.75 / 2.05 (1.65 / 1.3); order 5 32^2 2.7 /
+// 1.6 (1.5), 44^2 2.7 / 2.85 (2.6), 48^2 2.7 / 3.5 (2.5); order 7 (one step a launch) 48^2
+// 4.1 / 3.8 (3.35), 52^2 4.1 / 4.8 (4.55); periodic, order 3 44^2 1.8 / 2.1 (1.6), 48^2 1.8
+// / 2.8 (1.8); order 5 54^2 2.9 / 3.7 (3.1), 56^2 2.9 / 4.65 (3.6); order 7 54^2 4.5 / 4.5
+// (4.7 / 4.0), 56^2 4.45 / 5.45 (4.65 / 4.45).
 static int small_resident(int order, int bc) {
     if (bc == NLS_BC_PERIODIC) return order == 3 ? 44 : 54;
     return order == 3 ? 32 : order == 5 ? 44 : 48;

@@ -22,7 +22,7 @@
 // of a point at order 5, at four cycles each) and the LDS round trip; memory
 // is read once in K steps.  Measured, us per step (the resident kernel, or
 // beyond 4096 points the per-stage kernels, before): n = 256 FP32 dynamic
-// 0.56 (0.88), n = 1000 radial FP32 0.59 (3.6), n = 4096 FP64 0.65 (6.3).
+// 0.56 (0.88), n = 1000 radial FP32 0.61 (3.6), n = 4096 FP64 0.65 (6.3).
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -221,7 +221,7 @@ static int wave_points(int order, int q) { return 64 * q - 4 * (order - 1); }
 // round trip, the barrier and the latency of its four stages and 0.26 for
 // each point a SIMD's lane steps (points a lane x waves on the SIMD).  So few
 // points a lane and a wave on every SIMD are worth more than little overlap:
-// n = 4096 runs 0.58 us a step as 256 workgroups of 16 points over 12 steps
+// n = 4096 runs 0.65 us a step as 256 workgroups of 16 points over 12 steps
 // and 1.25 as 11 workgroups of 400; 16 is the least a chunk writes.  Wide
 // lanes (Q = 4: 6 to 12% overlap instead of 25%) come in when the waves fill
 // the device, beyond about 60,000 points.

@@ -15,12 +15,13 @@
 // piece and 16 columns a strip (none where a strip is a whole row of up to
 // 256 points), and loads and stores run along with the arithmetic.
 //
-// Bound: VALU issue -- 133 vector instructions a row and wave (single
-// precision) at 86% of the issue rate on a 2048^2 grid, where the strips and
-// pieces add 1.31 of redundancy -- and for batches beyond the 256 MB cache HBM
-// (256^2 and 128^2 grids, 283 MB a step, at 5.4 TB/s).  Per step, against the
-// tile kernels on the same box: 2048^2 FP32 32.5 -> 26.5 us, FP64 58.6 -> 49;
-// 4096^2 172 -> 113 and 296 -> 211; 154 x 128^2 + 102 x 256^2 FP32 73 -> 52.
+// Bound: on a 2048^2 grid in single precision VALU issue (134 vector instructions
+// a row and wave, 77% of a launch's issue slots, where the strips and pieces add
+// 1.31 of redundancy) and traffic together, in double precision the traffic behind
+// the L2s (284 MiB for 224 of fields, 6.3 TB/s); for batches beyond the 256 MB cache
+// HBM (131 grids of 128^2 and 109 of 256^2, 300 MB a step, at 5.1 TB/s).  Per step,
+// against the tile kernels on the same box: 2048^2 FP32 31.8 -> 25.1 us, FP64 58.8 ->
+// 45.6; 4096^2 162 -> 115 and 286 -> 213; those 240 grids FP32 88 -> 67.
 // Measured and left: deeper prefetch (three rows, ten rows at the start) and
 // stages guarded at run time instead of an unrolled start (10% slower).
 #include <algorithm>
