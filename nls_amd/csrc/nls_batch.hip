@@ -475,8 +475,8 @@ k_fused_step_2d(const FusedArgs<T> f) {
             const C a0 = rd(idx - d), a1 = rd(idx + d);
             const C b0 = rd(idx - d * WS), b1 = rd(idx + d * WS);
             if (d == 1) {
-                sr = grid_ring1(g, a0.x, a1.x, b0.x, b1.x);
-                sm = grid_ring1(g, a0.y, a1.y, b0.y, b1.y);
+                sr = grid_ring1<R>(g, a0.x, a1.x, b0.x, b1.x);
+                sm = grid_ring1<R>(g, a0.y, a1.y, b0.y, b1.y);
             } else {
                 sr = grid_ring(sr, d == 2 ? g.r2 : g.r3, a0.x, a1.x, b0.x, b1.x);
                 sm = grid_ring(sm, d == 2 ? g.r2 : g.r3, a0.y, a1.y, b0.y, b1.y);
@@ -732,7 +732,7 @@ k_fused_pairs_2d(const FusedArgs<float> f) {
         auto rd = [&](int i) { const V2 v = ys[i]; return mk<T>(v.x, v.y); };
         const C c0 = rd(0), c1 = rd(WS), yA = rd(2 * WS), yB = rd(3 * WS), c4 = rd(4 * WS), c5 = rd(5 * WS);
         const C a1m = rd(2 * WS - 1), a1p = rd(2 * WS + 1), a2m = rd(2 * WS - 2), a2p = rd(2 * WS + 2);
-        T sr = grid_ring1(g, a1m.x, a1p.x, c1.x, yB.x), sm = grid_ring1(g, a1m.y, a1p.y, c1.y, yB.y);
+        T sr = grid_ring1<R>(g, a1m.x, a1p.x, c1.x, yB.x), sm = grid_ring1<R>(g, a1m.y, a1p.y, c1.y, yB.y);
         sr = grid_ring(sr, g.r2, a2m.x, a2p.x, c0.x, c4.x);
         sm = grid_ring(sm, g.r2, a2m.y, a2p.y, c0.y, c4.y);
         grid_rhs<T, DYN>(g, c, cp[j][0], yA, yn[j][0], mk<T>(sr, sm), k[0], kn[0]);
@@ -740,8 +740,8 @@ k_fused_pairs_2d(const FusedArgs<float> f) {
         // reads do not all live in registers at once
         __builtin_amdgcn_sched_barrier(0);
         const C b1m = rd(3 * WS - 1), b1p = rd(3 * WS + 1), b2m = rd(3 * WS - 2), b2p = rd(3 * WS + 2);
-        sr = grid_ring1(g, b1m.x, b1p.x, yA.x, c4.x);
-        sm = grid_ring1(g, b1m.y, b1p.y, yA.y, c4.y);
+        sr = grid_ring1<R>(g, b1m.x, b1p.x, yA.x, c4.x);
+        sm = grid_ring1<R>(g, b1m.y, b1p.y, yA.y, c4.y);
         sr = grid_ring(sr, g.r2, b2m.x, b2p.x, c1.x, c5.x);
         sm = grid_ring(sm, g.r2, b2m.y, b2p.y, c1.y, c5.y);
         grid_rhs<T, DYN>(g, c, cp[j][1], yB, yn[j][1], mk<T>(sr, sm), k[1], kn[1]);
@@ -988,8 +988,8 @@ k_fused_groups_2d(const FusedArgs<T> f) {
             for (int d = 1; d <= R; ++d) {
                 const C l = rd((R + q) * WS - d), r = rd((R + q) * WS + d), &up = col[R + q - d], &dn = col[R + q + d];
                 if (d == 1) {
-                    sr = grid_ring1(g, l.x, r.x, up.x, dn.x);
-                    sm = grid_ring1(g, l.y, r.y, up.y, dn.y);
+                    sr = grid_ring1<R>(g, l.x, r.x, up.x, dn.x);
+                    sm = grid_ring1<R>(g, l.y, r.y, up.y, dn.y);
                 } else {
                     sr = grid_ring(sr, d == 2 ? g.r2 : g.r3, l.x, r.x, up.x, dn.x);
                     sm = grid_ring(sm, d == 2 ? g.r2 : g.r3, l.y, r.y, up.y, dn.y);

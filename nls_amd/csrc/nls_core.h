@@ -99,20 +99,27 @@ template <typename T> __device__ __forceinline__ T lap_quad(T w, T c, T a0, T a1
     return w * (((a0 + a1) + (b0 + b1)) - (T)4 * c);
 }
 
-// Coefficients of the fused 2-D step.  Single precision keeps the slopes of
-// psi in units of the first neighbour weight w_1: with K = k / w_1 the
-// neighbour sum enters with weights 1, w_2/w_1, w_3/w_1 (order 5: -1/16,
-// exact), the centre weight becomes 2 w_0/w_1 (-3.75, exact) and joins the
-// point's own factor, and the step sizes take the factor w_1 back (dt w_1).
-// Two products a point and stage fewer; and what is large in the Laplacian,
-// its weights, is no longer rounded: against 64 bits the 2048^2 grid ends 300
-// steps 5.8e-7 off instead of 3.3e-6, the 512-grid sweep 500 steps 5.9e-7
-// instead of 2.1e-6.  Double precision takes the weights as they are (the
-// unit of its slopes is 1).  The reservoir's slope keeps its own units.
+// Coefficients of the fused 2-D step: the slopes of psi are kept in a unit, the
+// step sizes take it back (dt unit), the centre weight joins the point's own
+// factor.  A coefficient, a weight or a step that is rounded is rounded alike at
+// every point and step: a drift, beside which the points' own roundings average out.
+//   Order 5, single precision: the unit is the first neighbour weight w_1, and the
+// weights 1, -1/16 and -3.75 are exact; rounded they cost the 2048^2 grid 3.3e-6
+// against 64 bits after 300 steps instead of 5.8e-7, the 512-grid sweep 2.1e-6 after
+// 500 instead of 5.9e-7.  It is moved by what dt w_1 / 6 is rounded by, so that the
+// step of the new state is exact and the weights take its rounding.
+//   Orders 3 and 7: a power of two, so that the coefficients and dt are exact in it;
+// the weights cannot all be, but sum to zero (order 3 as they are, order 7 by the
+// third).  In units of w_1 a product a point and stage less is needed, 2% of a step
+// at order 3 and 1% at 7, but grids of 65 to 1200 points ended up to 3.5 times further
+// from 64 bits than with the coefficients as they are, 1.16 times at nine in ten;
+// now no further.
+//   Double precision takes everything as it is (unit 1).  The reservoir's slope
+// keeps its own units.
 template <typename T> struct GridCoeffs {
     T c3, c4, c5, c6, wc;    // c_k / unit, 2 w_0 / unit
-    T r1, r2, r3;            // w_d / unit
-    T dtw, dtw6, dt6;        // dt unit, dt unit / 6, dt / 6, each rounded once
+    T r1, r2, r3;            // w_d / unit (order 5, single precision: r1 = 1)
+    T dtw, dtw6, dt6;        // dt unit, dt unit / 6, dt / 6
 };
 template <typename T> inline GridCoeffs<T> make_grid_coeffs(const double *c, int order, double dt, double dx) {
     // where the Laplacian's weights vanish beside the coefficients (a spacing
@@ -122,18 +129,27 @@ template <typename T> inline GridCoeffs<T> make_grid_coeffs(const double *c, int
     double cmax = 0.0;
     for (int k = 2; k < 6; ++k) cmax = c[k] > cmax ? c[k] : -c[k] > cmax ? -c[k] : cmax;
     const double w = stencil_s2(order, 1, dx), least = cmax * 0x1p-100;
-    const double unit = sizeof(T) == 8 ? 1.0 : w > least ? w : least;
+    double unit = sizeof(T) == 8 ? 1.0 : w > least ? w : least;
     // in units of w_1 the ratios do not depend on the spacing
-    const double h = sizeof(T) == 8 ? dx : 1.0, per = sizeof(T) == 8 ? 1.0 : stencil_s2(order, 1, 1.0);
+    double h = dx, per = 1.0;
+    if (sizeof(T) == 4 && order == 5) {
+        h = 1.0;
+        per = stencil_s2(order, 1, h);
+        const float step = (float)(dt * unit / 6.0);
+        if (std::isnormal(step)) unit = 6.0 * step / dt;
+    } else if (sizeof(T) == 4) {
+        per = unit = std::ldexp(1.0, std::ilogb(unit));
+    }
     GridCoeffs<T> g;
     g.c3 = (T)(c[2] / unit); g.c4 = (T)(c[3] / unit); g.c5 = (T)(c[4] / unit); g.c6 = (T)(c[5] / unit);
     g.wc = (T)(2.0 * stencil_s2(order, 0, h) / per);
     g.r1 = (T)(stencil_s2(order, 1, h) / per);
     g.r2 = order > 3 ? (T)(stencil_s2(order, 2, h) / per) : (T)0;
     g.r3 = order > 5 ? (T)(stencil_s2(order, 3, h) / per) : (T)0;
-    g.dtw = (T)(dt * unit);
-    g.dtw6 = (T)(dt * unit / 6.0);
-    g.dt6 = (T)(dt / 6.0);
+    if (sizeof(T) == 4 && order > 5) g.r3 = (T)(-0.25 * (double)g.wc - (double)g.r1 - (double)g.r2);
+    g.dt6 = (T)dt / (T)6;
+    g.dtw = (T)(sizeof(T) == 4 && order == 5 ? dt * unit : (T)dt * unit);
+    g.dtw6 = (T)(sizeof(T) == 4 && order == 5 ? dt * unit / 6.0 : g.dt6 * unit);
     return g;
 }
 
@@ -141,11 +157,11 @@ template <typename T> inline GridCoeffs<T> make_grid_coeffs(const double *c, int
 // every fused multiply-add written out and contraction off: a grid's result
 // has the same bits in every form, tile shape and row slab.
 // The neighbour sum, ring by ring: sum of r_d ((left + right) + (up + down)),
-// r_1 = 1 in single precision.
-template <typename T> __device__ __forceinline__ T grid_ring1(const GridCoeffs<T> &g, T l, T r, T u, T d) {
+// r_1 = 1 in single precision of order 5.
+template <int R, typename T> __device__ __forceinline__ T grid_ring1(const GridCoeffs<T> &g, T l, T r, T u, T d) {
 #pragma clang fp contract(off)
     const T s = (l + r) + (u + d);
-    return sizeof(T) == 4 ? s : g.r1 * s;
+    return sizeof(T) == 4 && R == 2 ? s : g.r1 * s;
 }
 template <typename T> __device__ __forceinline__ T grid_ring(T S, T ratio, T l, T r, T u, T d) {
 #pragma clang fp contract(off)
@@ -156,11 +172,13 @@ template <typename T> __device__ __forceinline__ T grid_ring(T S, T ratio, T l, 
 // from it exactly, and neither the sum nor the point's factor is rounded at
 // the size of the centre weight.  Eight operations a point and stage more than
 // with the centre weight in the factor; those kernels wait for latency.
-// Error against 64 bits, 447 steps: 40^2 order 3 8.1e-7 -> 5.9e-7, 40^2 order 7
-// 9.4e-7 -> 5.3e-7.
-__device__ __forceinline__ float grid_ring1_from(float c, float l, float r, float u, float d) {
+// Coefficients, weights and dt are the problem's own, and dt/6 carries what its
+// rounding leaves (grid_new_from): against 64 bits grids of 20 to 64 points end 200 to
+// 1500 steps as far off as with divisions by 6, 1.03 times at nine in ten; in units of
+// w_1 1.3 times at nine in ten and 2.3 at worst, for 3% of a step.
+__device__ __forceinline__ float grid_ring1_from(float w, float c, float l, float r, float u, float d) {
 #pragma clang fp contract(off)
-    return ((l - c) + (r - c)) + ((u - c) + (d - c));
+    return w * (((l - c) + (r - c)) + ((u - c) + (d - c)));
 }
 __device__ __forceinline__ float grid_ring_from(float S, float ratio, float c, float l, float r, float u, float d) {
 #pragma clang fp contract(off)
@@ -198,14 +216,15 @@ template <typename T> __device__ __forceinline__ T grid_new(T u, T acc, T k, T s
     return fma(acc + k, step6, u);
 }
 // The same with the sixth of the step in two terms (beside grid_ring1_from), and
-// the second of them: what the first, rounded, leaves of it.
+// the second of them: what the first, rounded, leaves of it.  It is added to the
+// increment; to u it would be lost.
 template <typename T> __device__ __forceinline__ T sixth_rest(T step, T step6) {
     return fma((T)-6, step6, step) * (T)(1.0 / 6.0);
 }
 template <typename T> __device__ __forceinline__ T grid_new_from(T u, T acc, T k, T step6, T lo) {
 #pragma clang fp contract(off)
     const T s = acc + k;
-    return fma(s, step6, fma(s, lo, u));
+    return u + fma(s, step6, s * lo);
 }
 
 // Arithmetic of one point of a 1-D line, shared by the resident and the line

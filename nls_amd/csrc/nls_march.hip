@@ -169,7 +169,7 @@ __device__ __forceinline__ void march_piece(const MarchArgs<T> &f, const StripDe
     // Slopes at a point from the five rows of its column and those.
     auto slopes = [&](const Row4 &h, const C &ym2, const C &ym1, const C &y, const C &yp1, const C &yp2, T cP, T yn,
                       C &kk, T &kn) {
-        T sr = grid_ring1(g, h.l1.x, h.q1.x, ym1.x, yp1.x), sm = grid_ring1(g, h.l1.y, h.q1.y, ym1.y, yp1.y);
+        T sr = grid_ring1<R>(g, h.l1.x, h.q1.x, ym1.x, yp1.x), sm = grid_ring1<R>(g, h.l1.y, h.q1.y, ym1.y, yp1.y);
         sr = grid_ring(sr, g.r2, h.l2.x, h.q2.x, ym2.x, yp2.x);
         sm = grid_ring(sm, g.r2, h.l2.y, h.q2.y, ym2.y, yp2.y);
         grid_rhs<T, DYN>(g, c, cP, y, yn, mk<T>(sr, sm), kk, kn);
