@@ -55,11 +55,11 @@ int check_problem(const nls_problem *p) {
 // whose small grids step several times a launch, or in single precision up to
 // small_resident points a side the resident kernel, with the same bits.  us per step,
 // launches of several steps / resident, without a reservoir (with one): zero-outside,
-// order 3 32^2 1.75 / 1.3 (1.7 / 1.1), 36^2 1.75 / 2.05 (1.65 / 1.3); order 5 32^2 2.7 /
-// 1.6 (1.5), 44^2 2.7 / 2.85 (2.6), 48^2 2.7 / 3.5 (2.5); order 7 (one step a launch) 48^2
-// 4.1 / 3.8 (3.35), 52^2 4.1 / 4.8 (4.55); periodic, order 3 44^2 1.8 / 2.1 (1.6), 48^2 1.8
-// / 2.8 (1.8); order 5 54^2 2.9 / 3.7 (3.1), 56^2 2.9 / 4.65 (3.6); order 7 54^2 4.5 / 4.5
-// (4.7 / 4.0), 56^2 4.45 / 5.45 (4.65 / 4.45).
+// order 3 32^2 1.75 / 1.4 (1.7 / 1.1), 36^2 1.75 / 2.1 (1.7 / 1.35); order 5 32^2 2.7 /
+// 1.6 (1.5), 44^2 2.9 / 2.9 (2.8 / 2.7), 48^2 2.85 / 3.7 (2.5); order 7 (one step a launch)
+// 48^2 4.05 / 3.9 (3.4), 52^2 4.2 / 4.9 (4.6); periodic, order 3 44^2 1.85 / 2.2 (1.7), 48^2
+// 1.85 / 3.0 (1.9); order 5 54^2 2.9 / 3.8 (3.1), 56^2 2.9 / 4.8 (3.8); order 7 54^2 4.5 /
+// 4.6 (4.7 / 4.0), 56^2 4.5 / 5.7 (4.7 / 4.5).
 static int small_resident(int order, int bc) {
     if (bc == NLS_BC_PERIODIC) return order == 3 ? 44 : 54;
     return order == 3 ? 32 : order == 5 ? 44 : 48;
