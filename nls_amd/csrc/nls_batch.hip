@@ -482,7 +482,7 @@ k_fused_step_2d(const FusedArgs<T> f) {
                 sm = grid_ring(sm, d == 2 ? g.r2 : g.r3, a0.y, a1.y, b0.y, b1.y);
             }
         }
-        grid_rhs<T, DYN>(g, c, cp[j], y, yn[j], mk<T>(sr, sm), k, kn);
+        grid_rhs<T, DYN>(g, c, cp[j], y, yn[j], grid_sum<R, T>(g, y, sr, sm), k, kn);
     };
 
     // stages 1..3 on the shrinking rectangles.  Stage s computes the points
@@ -997,7 +997,7 @@ k_fused_groups_2d(const FusedArgs<T> f) {
             }
             C k;
             T kn;
-            grid_rhs<T, DYN>(g, c, cp[j][q], col[R + q], yn[j][q], mk<T>(sr, sm), k, kn);
+            grid_rhs<T, DYN>(g, c, cp[j][q], col[R + q], yn[j][q], grid_sum<R, T>(g, col[R + q], sr, sm), k, kn);
             done(q, k, kn);
             // the next row's reads after this point is done, so that they do
             // not all live in registers at once
@@ -1577,8 +1577,20 @@ size_t fused_grid_workspace_bytes(const nls_problem *p) {
     return align256b(N * 2 * rs) + (p->coeffs[10] != 0.0 ? align256b(N * rs) : 0);
 }
 
+// Coefficients of a 2-D grid's step; from: for the kernels of grid_ring1_from's sums.
+template <typename T>
+static void set_grid_coeffs(MemberDev<T> &d, const double *c, int order, double dt, double dx, bool from) {
+    if constexpr (sizeof(T) == 4) {
+        if (from) {
+            d.g = make_grid_coeffs<T>(c, order, dt, dx, d.lo);
+            return;
+        }
+    }
+    d.g = make_grid_coeffs<T>(c, order, dt, dx);
+}
+
 // Member descriptor of a plain (single-instance) solve.
-template <typename T> static MemberDev<T> plain_member(const nls_problem *p) {
+template <typename T> static MemberDev<T> plain_member(const nls_problem *p, bool from = false) {
     MemberDev<T> d;
     memset(&d, 0, sizeof d);
     d.n = p->n;
@@ -1586,7 +1598,7 @@ template <typename T> static MemberDev<T> plain_member(const nls_problem *p) {
     d.tab = -1;
     d.dt = (T)p->dt;
     d.c = make_coeffs<T>(p->coeffs);
-    d.g = make_grid_coeffs<T>(p->coeffs, p->order, p->dt, p->dx);
+    if (p->dim == 2) set_grid_coeffs(d, p->coeffs, p->order, p->dt, p->dx, from);
     T w[4] = {0, 0, 0, 0};
     for (int q = 0; q <= (p->order - 1) / 2; ++q) w[q] = (T)stencil_s2(p->order, q, p->dx);
     d.w0 = w[0]; d.w1 = w[1]; d.w2 = w[2]; d.w3 = w[3];
@@ -1615,7 +1627,13 @@ static int fused_grid_run(const nls_problem *p, int iters, const T *P, cplx_t<T>
     f.grid_ntx = (p->n + 63) / 64;
     f.ntiles = f.grid_ntx * ((p->n + ty - 1) / ty);
     f.chunk = (f.ntiles + 7) / 8;
-    f.grid = plain_member<T>(p);
+    // a small grid: its own tiles, several steps a launch
+    // (of up to 64 points a side, in single precision: AUTO's choice instead of
+    // the resident engine, with its bits)
+    const int steps = multi_steps(p->n, p->order, device_cus());
+    const bool from = steps > 0 && p->engine == NLS_ENGINE_AUTO && p->dtype == NLS_F32 && p->n <= 64;
+    const int many = !from && get_fused_form(p->dtype) >= 0 ? 0 : steps;
+    f.grid = plain_member<T>(p, from);
     f.P = P;
     const MarchGrid mg = march_grid(p);
     MarchArgs<T> a;
@@ -1625,11 +1643,6 @@ static int fused_grid_run(const nls_problem *p, int iters, const T *P, cplx_t<T>
     a.grid_nx = mg.nx; a.grid_wd = mg.wd; a.grid_L = mg.rows;
     a.grid = f.grid;
     a.P = P;
-    // a small grid: its own tiles, several steps a launch
-    // (of up to 64 points a side, in single precision: AUTO's choice instead of
-    // the resident engine, with its bits)
-    const bool from = p->engine == NLS_ENGINE_AUTO && p->dtype == NLS_F32 && p->n <= 64;
-    const int many = !from && get_fused_form(p->dtype) >= 0 ? 0 : multi_steps(p->n, p->order, device_cus());
     MultiArgs<T> b;
     memset(&b, 0, sizeof b);
     b.grid = f.grid;
@@ -1720,7 +1733,7 @@ template <typename T>
 static int resident_run(const nls_problem *p, int iters, const T *P, cplx_t<T> *psi, T *nres, char *ws,
                         hipStream_t s) {
     static_assert(sizeof(MemberDev<T>) <= 256, "member descriptor fits its workspace slot");
-    MemberDev<T> one = plain_member<T>(p);
+    MemberDev<T> one = plain_member<T>(p, true);
     ResidentArgs<T> r;
     memset(&r, 0, sizeof r);
     r.psi = psi;
@@ -1891,7 +1904,7 @@ static void fill_members(nls_batch *b, const nls_member *ms, const int *ids) {
         d.dV = radial ? 2.0 * M_PI * m.dx * m.dx : (b->dim == 1 ? m.dx : m.dx * m.dx);
         d.dt = (T)m.dt;
         d.c = make_coeffs<T>(m.coeffs);
-        d.g = make_grid_coeffs<T>(m.coeffs, b->order, m.dt, m.dx);
+        if (b->dim == 2) set_grid_coeffs(d, m.coeffs, b->order, m.dt, m.dx, b->engine == NLS_ENGINE_RESIDENT);
         const int R = (b->order - 1) / 2;
         T w[4] = {0, 0, 0, 0};
         for (int q = 0; q <= R; ++q) w[q] = (T)stencil_s2(b->order, q, m.dx);

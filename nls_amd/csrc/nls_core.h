@@ -108,20 +108,25 @@ template <typename T> __device__ __forceinline__ T lap_quad(T w, T c, T a0, T a1
 // against 64 bits after 300 steps instead of 5.8e-7, the 512-grid sweep 2.1e-6 after
 // 500 instead of 5.9e-7.  It is moved by what dt w_1 / 6 is rounded by, so that the
 // step of the new state is exact and the weights take its rounding.
-//   Orders 3 and 7: a power of two, so that the coefficients and dt are exact in it;
-// the weights cannot all be, but sum to zero (order 3 as they are, order 7 by the
-// third).  In units of w_1 a product a point and stage less is needed, 2% of a step
-// at order 3 and 1% at 7, but grids of 65 to 1200 points ended up to 3.5 times further
-// from 64 bits than with the coefficients as they are, 1.16 times at nine in ten;
-// now no further.
+//   Orders 3 and 7, and grid_ring1_from's sums at every order: the one of 32 units
+// whose coefficients, weights and step round least together.  The weights still sum to
+// zero: of order 3 as they are, of order 7 in units of w_1, with a product of the sum
+// (grid_sum).  A product or two a point and stage, 1 to 3% of a step (2 to 5% up to
+// 64^2), against units of w_1, in which long solves ended up to 3.5 times further from
+// 64 bits than with coefficients, weights and dt as they are, and against those as they
+// are, up to 5 times further than in units of w_1.  Of 3000 random problems of 20^2 to
+// 1200^2 nine in ten are now at most 1.03 times as far as with either, one is more than
+// 1.5 times as far as with the coefficients as they are and four as in units of w_1.
 //   Double precision takes everything as it is (unit 1).  The reservoir's slope
 // keeps its own units.
+constexpr float GRID_CENTRE_7 = (float)(-98.0 / 27.0);    // 2 w_0 / w_1 at order 7
 template <typename T> struct GridCoeffs {
-    T c3, c4, c5, c6, wc;    // c_k / unit, 2 w_0 / unit
-    T r1, r2, r3;            // w_d / unit (order 5, single precision: r1 = 1)
+    T c3, c4, c5, c6, wc;    // c_k / unit, 2 w_0 / unit (order 7, single precision: 0)
+    T r1, r2, r3;            // w_d / unit (single precision, order 5: r1 = 1, order 7: r2, r3 of w_1)
     T dtw, dtw6, dt6;        // dt unit, dt unit / 6, dt / 6
 };
-template <typename T> inline GridCoeffs<T> make_grid_coeffs(const double *c, int order, double dt, double dx) {
+template <typename T>
+inline GridCoeffs<T> make_grid_coeffs(const double *c, int order, double dt, double dx, T *lo = nullptr) {
     // where the Laplacian's weights vanish beside the coefficients (a spacing
     // beyond 1e14 or so), the unit is held at 2^-100 of the largest
     // coefficient, so that the quotients stay in range; the Laplacian then
@@ -129,27 +134,61 @@ template <typename T> inline GridCoeffs<T> make_grid_coeffs(const double *c, int
     double cmax = 0.0;
     for (int k = 2; k < 6; ++k) cmax = c[k] > cmax ? c[k] : -c[k] > cmax ? -c[k] : cmax;
     const double w = stencil_s2(order, 1, dx), least = cmax * 0x1p-100;
-    double unit = sizeof(T) == 8 ? 1.0 : w > least ? w : least;
-    // in units of w_1 the ratios do not depend on the spacing
-    double h = dx, per = 1.0;
-    if (sizeof(T) == 4 && order == 5) {
+    double unit = sizeof(T) == 8 ? 1.0 : w > least ? w : least, h = dx, per = 1.0;
+    GridCoeffs<T> g;
+    auto weights = [&] {
+        if (sizeof(T) == 4 && order == 7 && !lo) {
+            g.wc = (T)0;
+            g.r1 = (T)(stencil_s2(order, 1, dx) / per);
+            g.r2 = (T)-0.1;
+            g.r3 = (T)(-0.25 * (double)GRID_CENTRE_7 - 1.0 - (double)g.r2);
+            return;
+        }
+        g.wc = (T)(2.0 * stencil_s2(order, 0, h) / per);
+        g.r1 = (T)(stencil_s2(order, 1, h) / per);
+        g.r2 = order > 3 ? (T)(stencil_s2(order, 2, h) / per) : (T)0;
+        g.r3 = order > 5 ? (T)(stencil_s2(order, 3, h) / per) : (T)0;
+    };
+    if (sizeof(T) == 4 && order == 5 && !lo) {
+        // in units of w_1 the ratios do not depend on the spacing
         h = 1.0;
         per = stencil_s2(order, 1, h);
         const float step = (float)(dt * unit / 6.0);
         if (std::isnormal(step)) unit = 6.0 * step / dt;
     } else if (sizeof(T) == 4) {
-        per = unit = std::ldexp(1.0, std::ilogb(unit));
+        // the unit's place between two powers of two: where the roundings of the
+        // coefficients and the Laplacian (its second moment), each with the step's, are
+        // least together
+        const double base = std::ldexp(1.0, std::ilogb(unit));
+        const double moment = w + 4.0 * (order > 3 ? stencil_s2(order, 2, dx) : 0.0) +
+                              9.0 * (order > 5 ? stencil_s2(order, 3, dx) : 0.0);
+        double best = HUGE_VAL;
+        unit = per = base;
+        for (int j = 0; j < 32; ++j) {
+            const double u = base * (1.0 + j / 32.0), step = dt * u / 6.0, es = lo ? 0.0 : (float)step / step - 1.0;
+            per = u;
+            weights();
+            double e = order == 7 && !lo ? g.r1 * u / w : (g.r1 + 4.0 * g.r2 + 9.0 * g.r3) * u / moment, sum;
+            e += es - 1.0;
+            sum = e * e;
+            for (int k = 2; k < 6; ++k) {
+                const double x = c[k] / u;
+                e = x != 0.0 ? (float)x / x - 1.0 + es : 0.0;
+                sum += e * e;
+            }
+            if (sum < best) { best = sum; unit = u; }
+        }
+        per = unit;
     }
-    GridCoeffs<T> g;
+    weights();
     g.c3 = (T)(c[2] / unit); g.c4 = (T)(c[3] / unit); g.c5 = (T)(c[4] / unit); g.c6 = (T)(c[5] / unit);
-    g.wc = (T)(2.0 * stencil_s2(order, 0, h) / per);
-    g.r1 = (T)(stencil_s2(order, 1, h) / per);
-    g.r2 = order > 3 ? (T)(stencil_s2(order, 2, h) / per) : (T)0;
-    g.r3 = order > 5 ? (T)(stencil_s2(order, 3, h) / per) : (T)0;
-    if (sizeof(T) == 4 && order > 5) g.r3 = (T)(-0.25 * (double)g.wc - (double)g.r1 - (double)g.r2);
-    g.dt6 = (T)dt / (T)6;
-    g.dtw = (T)(sizeof(T) == 4 && order == 5 ? dt * unit : (T)dt * unit);
-    g.dtw6 = (T)(sizeof(T) == 4 && order == 5 ? dt * unit / 6.0 : g.dt6 * unit);
+    g.dtw = (T)(dt * unit);
+    g.dtw6 = (T)(dt * unit / 6.0);
+    g.dt6 = (T)(dt / 6.0);
+    if (lo) {
+        lo[0] = (T)(dt * unit / 6.0 - g.dtw6);
+        lo[1] = (T)(dt / 6.0 - g.dt6);
+    }
     return g;
 }
 
@@ -161,21 +200,27 @@ template <typename T> inline GridCoeffs<T> make_grid_coeffs(const double *c, int
 template <int R, typename T> __device__ __forceinline__ T grid_ring1(const GridCoeffs<T> &g, T l, T r, T u, T d) {
 #pragma clang fp contract(off)
     const T s = (l + r) + (u + d);
-    return sizeof(T) == 4 && R == 2 ? s : g.r1 * s;
+    return sizeof(T) == 4 && R > 1 ? s : g.r1 * s;
 }
 template <typename T> __device__ __forceinline__ T grid_ring(T S, T ratio, T l, T r, T u, T d) {
 #pragma clang fp contract(off)
     return fma(ratio, (l + r) + (u + d), S);
+}
+// Order 7 in single precision: the centre's share joins the sum, in units of w_1.
+template <int R, typename T>
+__device__ __forceinline__ cplx_t<T> grid_sum(const GridCoeffs<T> &g, cplx_t<T> y, T sr, T sm) {
+#pragma clang fp contract(off)
+    if constexpr (sizeof(T) == 4 && R == 3)
+        return mk<T>(g.r1 * fma(GRID_CENTRE_7, y.x, sr), g.r1 * fma(GRID_CENTRE_7, y.y, sm));
+    return mk<T>(sr, sm);
 }
 // The same sums less the centre's share, for the kernels of grids of up to 64
 // points a side in single precision: neighbours close to the centre c differ
 // from it exactly, and neither the sum nor the point's factor is rounded at
 // the size of the centre weight.  Eight operations a point and stage more than
 // with the centre weight in the factor; those kernels wait for latency.
-// Coefficients, weights and dt are the problem's own, and dt/6 carries what its
-// rounding leaves (grid_new_from): against 64 bits grids of 20 to 64 points end 200 to
-// 1500 steps as far off as with divisions by 6, 1.03 times at nine in ten; in units of
-// w_1 1.3 times at nine in ten and 2.3 at worst, for 3% of a step.
+// The sixth of the step carries what its rounding leaves (grid_new_from), so that the
+// unit need not suit it.
 __device__ __forceinline__ float grid_ring1_from(float w, float c, float l, float r, float u, float d) {
 #pragma clang fp contract(off)
     return w * (((l - c) + (r - c)) + ((u - c) + (d - c)));
@@ -215,12 +260,8 @@ template <typename T> __device__ __forceinline__ T grid_input(T u, T k, T step) 
 template <typename T> __device__ __forceinline__ T grid_new(T u, T acc, T k, T step6) {
     return fma(acc + k, step6, u);
 }
-// The same with the sixth of the step in two terms (beside grid_ring1_from), and
-// the second of them: what the first, rounded, leaves of it.  It is added to the
-// increment; to u it would be lost.
-template <typename T> __device__ __forceinline__ T sixth_rest(T step, T step6) {
-    return fma((T)-6, step6, step) * (T)(1.0 / 6.0);
-}
+// The same with the sixth of the step in two terms (beside grid_ring1_from).  The
+// second, lo, is added to the increment; to u it would be lost.
 template <typename T> __device__ __forceinline__ T grid_new_from(T u, T acc, T k, T step6, T lo) {
 #pragma clang fp contract(off)
     const T s = acc + k;

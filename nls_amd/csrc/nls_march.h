@@ -6,7 +6,12 @@
 
 namespace nls {
 
-template <typename T> struct MemberDev {
+// What rounding leaves of GridCoeffs' dtw6 and dt6 (beside grid_ring1_from).
+template <typename T> struct StepRest {};
+template <> struct StepRest<float> {
+    float lo[2];
+};
+template <typename T> struct MemberDev : StepRest<T> {
     int n, steps;
     long long off;          // first point of the member in the packed arrays
     long long tab;          // first entry of its radial table (1-D ref), else -1

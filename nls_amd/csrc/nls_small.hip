@@ -45,15 +45,6 @@ template <int W, int HH, int R, int S, int WS> __device__ const StepMap<W, HH, R
 // a row) spread over the banks.
 constexpr int multi_stride(int W, int R) { return W + (R == 1 ? 2 : R == 2 ? 4 : 14); }
 
-// Coefficients for grid_ring1_from's sums: in the problem's own units.
-template <typename T> __device__ __forceinline__ GridCoeffs<T> from_coeffs(const MemberDev<T> &m) {
-    GridCoeffs<T> g = m.g;
-    g.c3 = m.c.c3; g.c4 = m.c.c4; g.c5 = m.c.c5; g.c6 = m.c.c6;
-    g.r1 = m.w1; g.r2 = m.w2; g.r3 = m.w3;
-    g.dtw = m.dt; g.dtw6 = m.g.dt6;
-    return g;
-}
-
 // FROM: grid_ring1_from's sums.
 template <typename T, int ORDER, int BC, bool DYN, int TX, int TY, int K, bool FROM>
 __global__ void __launch_bounds__(1024) k_multi(const MultiArgs<T> f) {
@@ -73,11 +64,12 @@ __global__ void __launch_bounds__(1024) k_multi(const MultiArgs<T> f) {
 #pragma unroll
     for (int j = 0; j < J; ++j) ent[j] = (NP % NT == 0 || j < J - 1 || tid + NT * j < NP) ? map[tid + NT * j] : 0u;
 
-    const T dt = m.dt, dt2 = dt * (T)0.5, dt6 = m.g.dt6;
+    const T dt = m.dt, dt2 = dt * (T)0.5;
     const Coeffs<T> c = m.c;
-    const GridCoeffs<T> g = FROM ? from_coeffs(m) : m.g;
+    const GridCoeffs<T> g = m.g;
+    T dtw6lo = 0, dt6lo = 0;
+    if constexpr (FROM) { dtw6lo = m.lo[0]; dt6lo = m.lo[1]; }
     const T dtw = g.dtw, dtw2 = dtw * (T)0.5, dtw6 = g.dtw6;
-    const T dt6lo = sixth_rest(dt, dt6);
 
     C uu[J], acc[J];
     T cp[J], nn[J], yn[J], accn[J];
@@ -140,7 +132,7 @@ __global__ void __launch_bounds__(1024) k_multi(const MultiArgs<T> f) {
                 sm = grid_ring(sm, d == 2 ? g.r2 : g.r3, l.y, r.y, u.y, b.y);
             }
         }
-        grid_rhs<T, DYN, FROM>(g, c, cp[j], y, yn[j], mk<T>(sr, sm), k, kn);
+        grid_rhs<T, DYN, FROM>(g, c, cp[j], y, yn[j], FROM ? mk<T>(sr, sm) : grid_sum<R, T>(g, y, sr, sm), k, kn);
     };
 
     // stage st of S: points with at least st R rings around them, a prefix of
@@ -173,12 +165,12 @@ __global__ void __launch_bounds__(1024) k_multi(const MultiArgs<T> f) {
                 if (DYN) yn[j] = grid_input(nn[j], kn, dta);
             } else {
                 if constexpr (FROM) {
-                    y = mk<T>(grid_new_from(uu[j].x, acc[j].x, k.x, dtw6, dt6lo),
-                              grid_new_from(uu[j].y, acc[j].y, k.y, dtw6, dt6lo));
-                    if (DYN) nn[j] = yn[j] = grid_new_from(nn[j], accn[j], kn, dt6, dt6lo);
+                    y = mk<T>(grid_new_from(uu[j].x, acc[j].x, k.x, dtw6, dtw6lo),
+                              grid_new_from(uu[j].y, acc[j].y, k.y, dtw6, dtw6lo));
+                    if (DYN) nn[j] = yn[j] = grid_new_from(nn[j], accn[j], kn, g.dt6, dt6lo);
                 } else {
                     y = mk<T>(grid_new(uu[j].x, acc[j].x, k.x, dtw6), grid_new(uu[j].y, acc[j].y, k.y, dtw6));
-                    if (DYN) nn[j] = yn[j] = grid_new(nn[j], accn[j], kn, dt6);
+                    if (DYN) nn[j] = yn[j] = grid_new(nn[j], accn[j], kn, g.dt6);
                 }
                 uu[j] = y;
             }
@@ -287,11 +279,12 @@ __global__ void __launch_bounds__((V > 4 ? 512 : 1024)) k_resident_2d(const Resi
     C *psi = r.psi + m.off;
     T *nres = DYN ? r.nres + m.off : nullptr;
     const T *P = r.P + m.off;
-    const T dt = m.dt, dt2 = dt * (T)0.5, dt6 = m.g.dt6;
+    const T dt = m.dt, dt2 = dt * (T)0.5;
     const Coeffs<T> c = m.c;
-    const GridCoeffs<T> g = sizeof(T) == 4 ? from_coeffs(m) : m.g;
+    const GridCoeffs<T> g = m.g;
+    T dtw6lo = 0, dt6lo = 0;
+    if constexpr (sizeof(T) == 4) { dtw6lo = m.lo[0]; dt6lo = m.lo[1]; }
     const T dtw = g.dtw, dtw2 = dtw * (T)0.5, dtw6 = g.dtw6;
-    const T dt6lo = sixth_rest(dt, dt6);
 
     const int strip = tid / n, col = tid - strip * n, r0 = strip * V;
     const int rows = min(V, n - r0);     // points of this thread; none if <= 0
@@ -433,12 +426,12 @@ __global__ void __launch_bounds__((V > 4 ? 512 : 1024)) k_resident_2d(const Resi
                     if (DYN) yn[v] = grid_input(un[v], kn, dta);
                 } else {
                     if constexpr (KEEP) {
-                        z = mk<T>(grid_new_from(u[v].x, acc[v].x, k.x, dtw6, dt6lo),
-                                  grid_new_from(u[v].y, acc[v].y, k.y, dtw6, dt6lo));
-                        if (DYN) un[v] = yn[v] = grid_new_from(un[v], accn[v], kn, dt6, dt6lo);
+                        z = mk<T>(grid_new_from(u[v].x, acc[v].x, k.x, dtw6, dtw6lo),
+                                  grid_new_from(u[v].y, acc[v].y, k.y, dtw6, dtw6lo));
+                        if (DYN) un[v] = yn[v] = grid_new_from(un[v], accn[v], kn, g.dt6, dt6lo);
                     } else {
                         z = mk<T>(grid_new(u[v].x, acc[v].x, k.x, dtw6), grid_new(u[v].y, acc[v].y, k.y, dtw6));
-                        if (DYN) un[v] = yn[v] = grid_new(un[v], accn[v], kn, dt6);
+                        if (DYN) un[v] = yn[v] = grid_new(un[v], accn[v], kn, g.dt6);
                     }
                     u[v] = z;
                 }
