@@ -1274,10 +1274,11 @@ static void launch_fused_form(int form, const FusedArgs<T> &f, hipStream_t s) {
         // zero-outside grids with a reservoir field would spill at 1024
         // threads (64 registers) and run the tall tile on 512
         constexpr int TALL = B == BC_REF && D ? FORM_TALL512 : FORM_TALL;
-        // (past two tiles a CU one point a thread at 1024 threads is the faster:
-        // 12 grids of 300^2 15.7 / 15.2 us, 2048^2 40.5 / 39.9; two a CU 11.4 / 11.9)
+        // (up to one tile a CU, and past two, one point a thread at 1024 threads is the
+        // faster: us per step, pairs / points, 30 grids of 70^2 7.5 / 7.0, 700^2 8.4 / 8.2,
+        // 12 of 300^2 15.7 / 15.2; between 8 of 296^2 10.8 / 11.0, 1000^2 12.1 / 12.3)
         if constexpr (B == BC_REF && D)
-            if (form != FORM_SHORT && f.ntiles > 2 * device_cus()) {
+            if (form != FORM_SHORT && (f.ntiles > 2 * device_cus() || f.ntiles <= device_cus())) {
                 hipLaunchKernelGGL((k_fused_step_2d<T, O, B, D, FORM_TALL, S32>), grid,
                                    dim3(FusedTile<T, O, FORM_TALL>::NT), 0, s, f);
                 return;
